@@ -166,14 +166,15 @@ namespace {
 // Workspace of one attention call: the larger of the tuned kernels' layout
 // (either cache kind) and the general kernels' (the shapes outside the tuned
 // ones); Prod keys add a projected-query region to the latter.
-int64_t attention_workspace_bytes(int B, int Hq, int Hkv, int L, int dim, int64_t max_tokens, bool prod) {
+int64_t attention_workspace_bytes(int B, int Hq, int Hkv, int L, int dim, int64_t max_tokens, bool prod,
+                                  bool without_wide = false) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || dim <= 0 || max_tokens < 0 || Hq % Hkv)
     return 0;
   const int64_t T = std::max<int64_t>(max_tokens, 1);
   const int64_t tuned =
       std::max(workspace_bytes(plan_splits(B, Hq, Hkv, L, T, dim, true), B, Hq, Hkv, L, dim),
                workspace_bytes(plan_splits(B, Hq, Hkv, L, T, dim, false), B, Hq, Hkv, L, dim));
-  return std::max(tuned, general_workspace_bytes(B, Hq, Hkv, L, dim, dim, T, prod));
+  return std::max(tuned, general_workspace_bytes(B, Hq, Hkv, L, dim, dim, T, prod, without_wide));
 }
 
 }  // namespace
@@ -214,7 +215,8 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
   const bool tuned_dim = dim == 64 || dim == 128 || dim == 256;
   const bool prod_small = prod && dim <= 128 && static_cast<int64_t>(Hq / Hkv) * L <= 4 && k_bits >= 1;
   const bool tile = !prod && tile_rows_path(kv_kind, dim, dim, (Hq / Hkv) * L);
-  if (!tuned_dim || (prod && !prod_small) || tile) {
+  const bool wide = !prod && wide_rows_path(kv_kind, dim, dim, (Hq / Hkv) * L);
+  if (!tuned_dim || (prod && !prod_small) || tile || wide) {
     GenCall c{};
     c.q = q;
     c.q_dtype = q_dtype;
@@ -256,7 +258,8 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
     c.workspace = workspace;
     c.workspace_bytes = workspace_bytes_given;
     c.stream = stream;
-    return general_attention(c);
+    // a wide call whose types or workspace do not suit runs the tuned kernels
+    if (!tuned_dim || (prod && !prod_small) || tile || wide_call(c)) return general_attention(c);
   }
   if (q_dtype != TQ_DTYPE_F32 && q_dtype != TQ_DTYPE_F16 && q_dtype != TQ_DTYPE_BF16)
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: q_dtype %d", q_dtype);
@@ -526,7 +529,8 @@ extern "C" int tq_attention_noalloc(const void* q, int q_dtype, int B, int Hq, i
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention (no-alloc): bad shape (B %d, Hq %d, Hkv %d, L %d, dim %d)",
                 B, Hq, Hkv, L, dim);
   if (B == 0) return TQ_OK;
-  const int64_t need = tq_attention_workspace_size(B, Hq, Hkv, L, dim, max_tokens);
+  // the wide kernel runs where its own need fits too; no problem is refused for it
+  const int64_t need = attention_workspace_bytes(B, Hq, Hkv, L, dim, max_tokens, false, true);
   if (need > kScratchBytes)
     return fail(TQ_ERR_WORKSPACE, "attention (no-alloc): the problem needs %lld bytes of scratch, "
                 "above the static %lld; use tq_attention with a caller workspace",

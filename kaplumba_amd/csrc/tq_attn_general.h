@@ -60,6 +60,7 @@ struct GenParams {
   const void* ksg;   // Prod QJL sign rows [B, Hkv, cap, Dk / 32] u32
   const void* krn;   // Prod residual norms [B, Hkv, cap]
   int kpw;           // packed MSE key row width in words (0 for 1-bit Prod)
+  int kbits, vbits;  // packed MSE widths (0 for plain)
   const float* kcb;  // key (MSE part) codebook
   int k_rot_kind;
   const float* krot;  // Hadamard signs (Dk) or dense R_K (Dk x Dk)
@@ -82,6 +83,8 @@ struct GenParams {
   const void* mask;
   int mask_kind;  // TQ_MASK_*
   int64_t m_sb, m_sg, m_sr, m_sl, m_st;
+  int2* mrange;                        // wide kernel: kept keys (first, last + 1) per mask row, or null
+  int mr_sb, mr_sg, mr_sr, mr_sl;      // its strides (0 along axes the mask does not vary along)
   // split-K
   int n_splits, chunk, n_rg;
   // workspace
@@ -104,9 +107,17 @@ struct GenParams {
 constexpr int kTileMinRows = 64;
 bool tile_rows_path(int kv_kind, int Dk, int Dv, int rows);
 
-// Workspace bytes of the general path for this problem.
+// Query rows per kv head from which the shapes of wide_dims() run the wide
+// kernel (tq_attn_wide.h), and the shapes.
+constexpr int kWideMinRows = 64;
+bool wide_rows_path(int kv_kind, int Dk, int Dv, int rows);
+
+// Workspace bytes of the general path for this problem, whichever of its
+// kernels runs; without_wide: of the kernels before the wide one, which takes
+// a call only where its own need fits (callers with fixed scratch keep every
+// problem they had).
 int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T,
-                                bool prod);
+                                bool prod, bool without_wide = false);
 
 // Arguments of one general attention call (validated by general_attention).
 struct GenCall {
@@ -145,5 +156,12 @@ struct GenCall {
 };
 
 int general_attention(const GenCall& c);
+
+// Whether general_attention would run the wide kernel for this call (shape,
+// types, alignment, workspace).
+bool wide_call(const GenCall& c);
+int launch_wide_packed(const GenParams& p, bool f32_weights, hipStream_t st);
+int launch_wide_f16(const GenParams& p, bool f32_weights, hipStream_t st);
+int launch_wide_bf16(const GenParams& p, bool f32_weights, hipStream_t st);
 
 }  // namespace tq

@@ -6,6 +6,7 @@
 #include "tq_attn_general.h"
 #include "tq_attn_merge.h"
 #include "tq_attn_tile.h"
+#include "tq_attn_wide_prep.h"
 
 namespace tq {
 namespace {
@@ -616,11 +617,11 @@ __global__ __launch_bounds__(kGenThreads) void gen_merge_kernel(GenParams p) {
 }
 
 // Element-wise merge: partials in the natural basis (plain values), or the
-// tile kernel's Hadamard-rotated ones (merge_had, Dv = 128).  Thread = (row,
-// 4 output columns): the splits' (m, l) and o by log-sum-exp, / max(l,
-// 1e-6); for merge_had then R_V^-1 on the merged row (the 32 threads of a
-// row are 32 consecutive lanes: butterflies over the 4 columns in registers,
-// over column bits 2-6 across lanes, then the signs and 1/sqrt(Dv), the
+// tile and wide kernels' Hadamard-rotated ones (merge_had, Dv = 64, 128 or
+// 256).  Thread = (row, 4 output columns): the splits' (m, l) and o by
+// log-sum-exp, / max(l, 1e-6); for merge_had then R_V^-1 on the merged row (the
+// Dv / 4 threads of a row are consecutive lanes of one wave: butterflies over
+// the 4 columns in registers, over the higher column bits across lanes, then the signs and 1/sqrt(Dv), the
 // order of _rht_inverse, turboquant_cache.py:3564-3575); output in the
 // query dtype.  A split without tokens (m = -inf) has no o written; it is
 // selected away, never multiplied.  Index type I: int when the item count
@@ -710,8 +711,20 @@ __global__ __launch_bounds__(256) void gen_merge_flat_kernel(GenParams p, I n_it
     TQ_MERGE_STAGE(2)
     TQ_MERGE_STAGE(4)
     TQ_MERGE_STAGE(8)
-    TQ_MERGE_STAGE(16)
+    if (p.Dv >= 128) {
+      TQ_MERGE_STAGE(16)
+    }
 #undef TQ_MERGE_STAGE
+    if (p.Dv == 256) {  // column bit 7: the wave's halves (lanes < 32: (v, v[l + 32]); others (v[l - 32], v))
+      float2 h = halves(v0);
+      v0 = (c4 & 32) ? h.x - h.y : h.x + h.y;
+      h = halves(v1);
+      v1 = (c4 & 32) ? h.x - h.y : h.x + h.y;
+      h = halves(v2);
+      v2 = (c4 & 32) ? h.x - h.y : h.x + h.y;
+      h = halves(v3);
+      v3 = (c4 & 32) ? h.x - h.y : h.x + h.y;
+    }
     const float4 sg = reinterpret_cast<const float4*>(p.vrot)[c4];
     v0 *= sg.x * p.rscale_v;
     v1 *= sg.y * p.rscale_v;
@@ -731,6 +744,16 @@ __global__ __launch_bounds__(256) void gen_merge_flat_kernel(GenParams p, I n_it
 }
 
 // --------------------------------------------------------------- launch ---
+int64_t a256(int64_t x) { return (x + 255) / 256 * 256; }
+int round32(int d) { return (d + 31) / 32 * 32; }
+int pow2_at_least(int d) {
+  int r = 32;
+  while (r < d) r <<= 1;
+  return r;
+}
+
+void launch_qprep_mode(const GenParams& p, int64_t rows, int mode, const float* mat, float* dst, hipStream_t st);
+
 struct GenPlan {
   int n_splits, chunk, n_rg;
 };
@@ -774,12 +797,102 @@ GenPlan tile_plan(int B, int Hq, int Hkv, int L, int64_t T) {
   return gp;
 }
 
-int64_t a256(int64_t x) { return (x + 255) / 256 * 256; }
-int round32(int d) { return (d + 31) / 32 * 32; }
-int pow2_at_least(int d) {
-  int r = 32;
-  while (r < d) r <<= 1;
-  return r;
+// The wide kernel's plan: blocks of its row count, and the number of splits
+// with the least estimated time: rounds of one workgroup per CU, each its
+// tokens plus a fixed part (set-up, first loads, epilogue: about 8 us), plus
+// the partials' way through memory (written, then read by the merge, at about
+// 4 TB/s).  Microseconds per token measured on the prefill shapes.
+constexpr int kWideMaxSplits = 32;
+
+GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
+  GenPlan gp{};
+  int ks = 0, ct = 0;
+  wide_dims(Dk, Dv, ks, ct);
+  const int64_t rows = static_cast<int64_t>(Hq / Hkv) * L;
+  const int64_t per = wide_block_rows(ks);
+  gp.n_rg = static_cast<int>((rows + kGenNQ - 1) / kGenNQ);
+  const int64_t blocks = static_cast<int64_t>(B) * Hkv * ((rows + per - 1) / per);
+  const int64_t cus = device_cu_count();
+  const double token_us = (32 * ks + 16 * ct) * (wide_rt(ks) == 2 ? 0.00045 : 0.00023);
+  const double merge_us = static_cast<double>(B) * Hq * L * Dv * 8 / 4e6;  // per split
+  int64_t best = 1;
+  double best_cost = 0;
+  for (int64_t ns = 1; ns <= kWideMaxSplits && (ns == 1 || (T + ns - 1) / ns >= 32); ++ns) {
+    const double cost =
+        static_cast<double>((blocks * ns + cus - 1) / cus) * (static_cast<double>((T + ns - 1) / ns) * token_us + 8) +
+        static_cast<double>(ns) * merge_us;
+    if (ns == 1 || cost < best_cost) {
+      best = ns;
+      best_cost = cost;
+    }
+  }
+  gp.n_splits = static_cast<int>(best);
+  gp.chunk = 0;  // each block splits the tokens its rows see (in the kernel)
+  return gp;
+}
+
+// Workspace: [q_rot rows DkP f32 (packed)][po][pml][query words][sq rows][mask ranges]
+struct WideLayout {
+  int64_t po, pml, qhl, qsq, mrange, bytes;
+};
+
+WideLayout wide_layout(int B, int Hq, int Hkv, int L, int Dk, int Dv, const GenPlan& gp, bool packed, bool mask) {
+  int ks = 0, ct = 0;
+  wide_dims(Dk, Dv, ks, ct);
+  const int64_t rows = static_cast<int64_t>(B) * Hq * L;
+  const int64_t parts = static_cast<int64_t>(B) * Hkv * gp.n_rg * gp.n_splits * kGenNQ;
+  WideLayout w{};
+  w.po = packed ? a256(rows * round32(Dk) * 4) : 0;
+  w.pml = w.po + a256(parts * Dv * 4);
+  w.qhl = w.pml + a256(parts * 2 * 4);
+  w.qsq = w.qhl + a256(rows * ks * 64 * (packed ? 2 : 1));
+  w.mrange = w.qsq + (packed ? a256(rows * 4) : 0);
+  w.bytes = w.mrange + (mask ? a256(rows * 8) : 0);
+  return w;
+}
+
+// Hadamard queries that wide_qprep_kernel rotates itself (its lanes hold whole padded rows)
+bool wide_had_queries(int Dk, int rot_kind) {
+  return rot_kind == TQ_ROT_HADAMARD && (Dk == 64 || Dk == 128 || Dk == 256);
+}
+
+// Prepares the queries (and mask ranges) and runs the wide kernel over p,
+// whose workspace pointers follow wide_layout; general: the weights were f32
+// in the vector kernel.
+int run_wide(GenParams& p, int64_t rows, bool plain, hipStream_t st) {
+  int ks = 0, ct = 0;
+  wide_dims(p.Dk, p.Dv, ks, ct);
+  const dim3 qgrid(static_cast<unsigned>((rows + kWideQpThreads / 16 - 1) / (kWideQpThreads / 16)));
+  const int nr = static_cast<int>(rows);
+  if (plain)
+    hipLaunchKernelGGL(wide_qprep_kernel<kWideQPlain>, qgrid, dim3(kWideQpThreads), 0, st, p, nr, 4 * ks);
+  else if (wide_had_queries(p.Dk, p.k_rot_kind))
+    hipLaunchKernelGGL(wide_qprep_kernel<kWideQHad>, qgrid, dim3(kWideQpThreads), 0, st, p, nr, 4 * ks);
+  else
+    hipLaunchKernelGGL(wide_qprep_kernel<kWideQRows>, qgrid, dim3(kWideQpThreads), 0, st, p, nr, 4 * ks);
+  int rc = check_launch("wide_qprep_kernel");
+  if (rc) return rc;
+  if (p.mask_kind != TQ_MASK_NONE && !p.causal) {
+    // one range per distinct mask row: axes the mask is broadcast along share
+    // theirs (per-sequence windows keep the batch axis)
+    const bool bb = p.B > 1 && (p.m_sb != 0 || p.seq_lens || p.seq_starts);
+    const int nb = bb ? p.B : 1, ng = p.m_sg != 0 ? p.Hkv : 1, nrep = p.m_sr != 0 ? p.R : 1, nl = p.m_sl != 0 ? p.L : 1;
+    p.mr_sl = nl > 1 ? 1 : 0;
+    p.mr_sr = nrep > 1 ? nl : 0;
+    p.mr_sg = ng > 1 ? nl * nrep : 0;
+    p.mr_sb = nb > 1 ? nl * nrep * ng : 0;
+    hipLaunchKernelGGL(gen_mask_range_kernel, dim3(static_cast<unsigned>(nb * ng * nrep * nl)), dim3(256), 0, st, p,
+                       ng, nrep, nl);
+    rc = check_launch("gen_mask_range_kernel");
+    if (rc) return rc;
+  } else {
+    p.mrange = nullptr;
+  }
+  // the vector kernel's f32 weights: array masks and the dims it alone served
+  const bool pow2dim = p.Dk == p.Dv && (p.Dk == 64 || p.Dk == 128 || p.Dk == 256);
+  const bool f32_weights = p.mask_kind != TQ_MASK_NONE || !pow2dim || (!plain && p.k_rot_kind != p.v_rot_kind);
+  if (!plain) return launch_wide_packed(p, f32_weights, st);
+  return p.key_kind == kGenPlainBf16 ? launch_wide_bf16(p, f32_weights, st) : launch_wide_f16(p, f32_weights, st);
 }
 
 template <int KB, int VB>
@@ -874,9 +987,53 @@ bool tile_rows_path(int kv_kind, int Dk, int Dv, int rows) {
   return kv_kind == TQ_KV_PACKED && Dk == 128 && Dv == 128 && rows >= kTileMinRows;
 }
 
-int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod) {
+bool wide_rows_path(int kv_kind, int Dk, int Dv, int rows) {
+  int ks = 0, ct = 0;
+  return (kv_kind == TQ_KV_PACKED || kv_kind == TQ_KV_PLAIN) && rows >= kWideMinRows && wide_dims(Dk, Dv, ks, ct);
+}
+
+// Work from which the wide kernel is the faster one, in query row x token x
+// (Dk + Dv) products of 2^28 (its set-up, and the partials of the splits that
+// fill the chip, cost 10-15 us).  Measured crossovers against the kernel that
+// would run instead, 2 and 8 kv heads, 64-1024 rows each, 256-4352 tokens:
+// tuned kernels at d = 64: 0.85-1.0x up to 5, 1.15x at 17; plain d = 128:
+// 0.65-1.15x at 2, 1.15x from 4; d = 256: 0.76-1.0x at 0.3-1, 1.3x from 1.25;
+// vector kernel with dense queries 0.8x at 0.4, 1.0x at 0.75, 1.1x from 1.5;
+// its other calls (masks, plain caches of other dims) 1.05x and more from the
+// smallest on.
+bool wide_pays(const GenCall& c) {
+  const double work = static_cast<double>(c.B) * c.Hq * c.L * static_cast<double>(c.max_tokens) * (c.Dk + c.Dv) / (1 << 28);
+  const bool plain = c.kv_kind == TQ_KV_PLAIN;
+  const bool tuned = c.mask_kind == TQ_MASK_NONE && c.Dk == c.Dv && (plain || c.k_rot_kind == c.v_rot_kind);
+  if (tuned && c.Dk == 64) return work >= 6;
+  if (tuned && c.Dk == 128) return work >= 4;
+  if (tuned && c.Dk == 256) return work >= 1.25;
+  return plain || c.k_rot_kind == TQ_ROT_HADAMARD || work >= 1;
+}
+
+bool wide_call(const GenCall& c) {
+  const int rows = (c.Hq / c.Hkv) * c.L;
+  if (!wide_rows_path(c.kv_kind, c.Dk, c.Dv, rows) || !wide_pays(c)) return false;
+  if (c.mask_kind == TQ_MASK_NONE && tile_rows_path(c.kv_kind, c.Dk, c.Dv, rows)) return false;
+  if (c.capacity > INT32_MAX || static_cast<int64_t>(c.B) * c.Hq * c.L >= (int64_t(1) << 30)) return false;
+  if (c.kv_kind == TQ_KV_PLAIN &&
+      (c.q_dtype != c.kv_dtype || c.Dk % 8 || c.Dv % 8 ||
+       ((reinterpret_cast<uintptr_t>(c.k) | reinterpret_cast<uintptr_t>(c.v)) & 15u)))
+    return false;
+  const int64_t T = std::max<int64_t>(c.max_tokens, 1);
+  const GenPlan gp = wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T);
+  return static_cast<int64_t>(c.Hkv) * gp.n_rg <= 65535 && c.B <= 65535 &&
+         c.workspace_bytes >= wide_layout(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, gp, c.kv_kind == TQ_KV_PACKED,
+                                          c.mask_kind != TQ_MASK_NONE).bytes;
+}
+
+int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod,
+                                bool without_wide) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || Dk <= 0 || Dv <= 0 || Hq % Hkv) return 0;
   T = std::max<int64_t>(T, 1);
+  int64_t wide = 0;
+  if (!without_wide && wide_rows_path(TQ_KV_PACKED, Dk, Dv, (Hq / Hkv) * L))
+    wide = wide_layout(B, Hq, Hkv, L, Dk, Dv, wide_plan(B, Hq, Hkv, L, Dk, Dv, T), true, true).bytes;
   GenPlan gp = gen_plan(B, Hq, Hkv, L, T);
   const int64_t rows = static_cast<int64_t>(B) * Hq * L;
   int64_t tile_q = 0;  // the tile kernel's prepared query rows
@@ -886,9 +1043,9 @@ int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, i
     tile_q = a256(rows * Dk * 4) + a256(rows * 4);
   }
   const int64_t groups = static_cast<int64_t>(B) * Hkv * gp.n_rg;
-  return a256(rows * round32(Dk) * 4) * (prod ? 2 : 1) +
-         a256(groups * gp.n_splits * kGenNQ * static_cast<int64_t>(Dv) * 4) +
-         a256(groups * gp.n_splits * kGenNQ * 2 * 4) + tile_q;
+  return std::max(wide, a256(rows * round32(Dk) * 4) * (prod ? 2 : 1) +
+                            a256(groups * gp.n_splits * kGenNQ * static_cast<int64_t>(Dv) * 4) +
+                            a256(groups * gp.n_splits * kGenNQ * 2 * 4) + tile_q);
 }
 
 int general_attention(const GenCall& c) {
@@ -949,11 +1106,17 @@ int general_attention(const GenCall& c) {
   const bool tile = c.kv_kind == TQ_KV_PACKED && c.mask_kind == TQ_MASK_NONE &&
                     tile_rows_path(c.kv_kind, c.Dk, c.Dv, (c.Hq / c.Hkv) * c.L) &&
                     static_cast<int64_t>(c.B) * c.Hq * c.L < (int64_t(1) << 30);
-  const GenPlan gp = tile ? tile_plan(c.B, c.Hq, c.Hkv, c.L, T) : gen_plan(c.B, c.Hq, c.Hkv, c.L, T);
+  const bool wide = wide_call(c);
+  const GenPlan gp = wide   ? wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T)
+                     : tile ? tile_plan(c.B, c.Hq, c.Hkv, c.L, T)
+                            : gen_plan(c.B, c.Hq, c.Hkv, c.L, T);
   if (static_cast<int64_t>(c.Hkv) * gp.n_rg > 65535 || c.B > 65535)
     return fail(TQ_ERR_UNSUPPORTED, "attention: %lld kv head row groups / %d sequences exceed one launch",
                 (long long)c.Hkv * gp.n_rg, c.B);
-  const int64_t need = general_workspace_bytes(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T, prod);
+  const WideLayout wl =
+      wide ? wide_layout(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, gp, !plain, c.mask_kind != TQ_MASK_NONE) : WideLayout{};
+  const int64_t need =
+      wide ? wl.bytes : general_workspace_bytes(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T, prod, true);
   if (c.workspace_bytes < need)
     return fail(TQ_ERR_WORKSPACE, "attention: workspace %lld < %lld bytes", (long long)c.workspace_bytes,
                 (long long)need);
@@ -982,6 +1145,8 @@ int general_attention(const GenCall& c) {
   p.ksg = c.k_signs;
   p.krn = c.k_rnorms;
   p.kpw = plain ? 0 : tq_packed_width(c.Dk, kb);
+  p.kbits = plain ? 0 : kb;
+  p.vbits = plain ? 0 : c.v_bits;
   p.kcb = c.k_codebook;
   p.k_rot_kind = c.k_rot_kind;
   p.krot = c.k_rot;
@@ -1013,7 +1178,7 @@ int general_attention(const GenCall& c) {
   const int64_t rows = static_cast<int64_t>(c.B) * c.Hq * c.L;
   char* ws = static_cast<char*>(c.workspace);
   p.qrot = reinterpret_cast<float*>(ws);
-  ws += a256(rows * p.DkP * 4);
+  if (!wide) ws += a256(rows * p.DkP * 4);
   if (prod) {
     p.qproj = reinterpret_cast<float*>(ws);
     ws += a256(rows * p.DkP * 4);
@@ -1028,6 +1193,14 @@ int general_attention(const GenCall& c) {
     ws += a256(rows * c.Dk * 4);
     p.qsq = reinterpret_cast<float*>(ws);
   }
+  if (wide) {
+    ws = static_cast<char*>(c.workspace);
+    p.po = reinterpret_cast<float*>(ws + wl.po);
+    p.pml = reinterpret_cast<float*>(ws + wl.pml);
+    p.qhl = reinterpret_cast<uint32_t*>(ws + wl.qhl);
+    p.qsq = reinterpret_cast<float*>(ws + wl.qsq);
+    p.mrange = reinterpret_cast<int2*>(ws + wl.mrange);
+  }
   p.rscale_k = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(c.Dk)));
   p.rscale_v = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(c.Dv)));
   p.qjl_scale = static_cast<float>(__builtin_sqrt(3.14159265358979323846 / 2.0) / c.Dk);
@@ -1038,10 +1211,15 @@ int general_attention(const GenCall& c) {
   // which rotates Hadamard queries itself); its Hadamard-rotated partials go
   // to the element-wise merge, which applies R_V^-1 once per row
   p.po_natural = plain ? 1 : 0;
-  p.merge_had = (tile && c.v_rot_kind == TQ_ROT_HADAMARD) ? 1 : 0;
-  if (plain)
+  p.merge_had = ((tile || (wide && !plain && (c.Dv == 64 || c.Dv == 128 || c.Dv == 256))) &&
+                 c.v_rot_kind == TQ_ROT_HADAMARD)
+                    ? 1
+                    : 0;
+  if (wide && (plain || wide_had_queries(c.Dk, c.k_rot_kind)))
+    ;
+  else if (plain)
     launch_qprep_mode(p, rows, 0, nullptr, p.qrot, st);
-  else if (tile && c.k_rot_kind == TQ_ROT_HADAMARD)
+  else if (tile && !wide && c.k_rot_kind == TQ_ROT_HADAMARD)
     ;
   else if (c.k_rot_kind == TQ_ROT_HADAMARD && kb > 0)
     launch_qprep_mode(p, rows, 1, c.k_rot, p.qrot, st);
@@ -1050,14 +1228,16 @@ int general_attention(const GenCall& c) {
   if (prod) launch_qprep_mode(p, rows, 2, c.projection, p.qproj, st);
   int rc = check_launch("gen_qprep_kernel");
   if (rc) return rc;
-  if (tile) {
+  if (tile && !wide) {
     const int64_t wgs = (rows + kTileQpRows * (kTileQpThreads / 64) - 1) / (kTileQpRows * (kTileQpThreads / 64));
     hipLaunchKernelGGL(gen_tile_qprep_kernel, dim3(static_cast<unsigned>(wgs)), dim3(kTileQpThreads), 0, st, p,
                        static_cast<int>(rows));
     rc = check_launch("gen_tile_qprep_kernel");
     if (rc) return rc;
   }
-  rc = tile ? launch_tile_partial(p, kb, c.v_bits, st) : launch_gen_partial(p, kb, plain ? 0 : c.v_bits, st);
+  rc = wide   ? run_wide(p, rows, plain, st)
+       : tile ? launch_tile_partial(p, kb, c.v_bits, st)
+              : launch_gen_partial(p, kb, plain ? 0 : c.v_bits, st);
   if (rc) return rc;
   // the flat merge takes 4 value columns per thread: plain values need Dv % 4 == 0
   if ((plain && c.Dv % 4 == 0) || p.merge_had) {
@@ -1065,7 +1245,7 @@ int general_attention(const GenCall& c) {
     const int64_t pair_items = static_cast<int64_t>(c.Hq / c.Hkv) * c.L * (c.Dv / 4);
     // after the tile kernel, each pair's merge blocks run on the XCD whose
     // L2 took that pair's partials
-    p.merge_bpp = (tile && (static_cast<int64_t>(c.B) * c.Hkv) % 8 == 0 && pair_items % 256 == 0)
+    p.merge_bpp = ((tile || wide) && (static_cast<int64_t>(c.B) * c.Hkv) % 8 == 0 && pair_items % 256 == 0)
                       ? static_cast<int>(pair_items / 256)
                       : 0;
     const dim3 fgrid(static_cast<unsigned>((items + 255) / 256));

@@ -43,6 +43,7 @@
 
 #include "tq_attn_general.h"
 #include "tq_attn_mfma.h"
+#include "tq_attn_slots.h"
 #include "tq_attn_small.h"
 
 namespace tq {
@@ -91,16 +92,6 @@ struct TileShape {
   static_assert(KROW % 16 == 0 && STG_BYTES % 16 == 0 && DEC_BYTES % 16 == 0, "16-byte aligned LDS rows");
   static_assert(STG_V == SUB * PWK * 4 && STG_KN == STG_V + SUB * PWV * 4, "staging in load-slot order");
 };
-
-// Slot of token t's decoded key row: row m = 4 (t / 8) + t % 4 of tile
-// h = (t / 4) % 2, so that score lane group g collects tokens 8 g .. 8 g + 7.
-__device__ __forceinline__ int tile_kslot(int t) { return 16 * ((t >> 2) & 1) + 4 * (t >> 3) + (t & 3); }
-
-// Slot of token t's 32-byte row in a 16-column value block: bit 3 of t
-// folded into bit 2, so the eight rows a half-wave's transposed read touches
-// (8 g + 4 h + 0..3 for g = 2 k, 2 k + 1) sit in eight distinct 32-byte bank
-// groups.  An involution, hence a permutation of 0..31.
-__device__ __forceinline__ int tile_vslot(int t) { return t ^ ((t >> 1) & 4); }
 
 template <int KB, int VB>
 __global__ __launch_bounds__(kTileThreads) void gen_tile_kernel(GenParams p, int n_blocks) {

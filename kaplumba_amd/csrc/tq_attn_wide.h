@@ -1,0 +1,764 @@
+// Many query rows per kv head (prefill chunks, wide verify) outside the
+// packed d = 128 causal case of tq_attn_tile.h: a partial kernel of the
+// general path (tq_attn_general.h) on the matrix cores.  One body serves
+//   packed MSE caches of any bit widths, plain f16 and plain bf16 caches,
+//   head dims padded to 32 KS (keys) and 16 CT (values),
+//   causal rows, ragged windows and array masks.
+// A workgroup is 8 waves of 16 RT query rows of one kv head over one slab of
+// its tokens.  Each SUB-token step decodes (or copies) K and V into LDS once,
+// as MFMA operands, and every wave reads them from there.
+//
+// LDS holds one K and one V slot; a step has two phases, each closed by a
+// barrier:
+//   A  scores and softmax of step i from the K slot; V of step i into the V slot
+//   B  O += P V of step i from the V slot; K of step i + 1 into the K slot
+// so decode work always runs beside matrix products of the other slot.  The
+// four lead waves decode first, the four trailing ones (their SIMD partners)
+// last, so that one wave's decode meets the other's products.  Every thread
+// loads the packed words (or 16-byte pieces) of its own units one whole step
+// ahead, into registers; nothing is staged in between.
+//
+// What bounds it: matrix products, LDS reads (an operand is read once per
+// 16 RT rows) and softmax add up at two waves per SIMD.  SUB is 64 where the
+// slots fit, 32 at the widest packed heads; RT is the largest that keeps
+// queries and outputs (2 x 16 RT (KS + CT/2) registers) within half of 256.
+//
+// Measured, append and attention of one layer, against the kernel that took
+// the call before: 512 queries x 8192 tokens under a 4096-key boolean window,
+// d = 128, 3 bits: 2815 -> 170 us (vector kernel); 2 x 500 queries x 4097
+// tokens, d = 64, K3/V4: 243 -> 129 us, and 512 queries x 4096 tokens, d = 256,
+// K4/V2, dense: 540 -> 372 us (attn_mfma_kernel: decodes per 16 or 4 rows);
+// 512 queries x 8192 plain bf16 tokens, d = 128: 345 -> 170 us
+// (attn_plain_kernel: reads K/V per 16 rows).  Partial kernels alone: 156, 119,
+// 119 and 172 us.
+//
+// Weight pieces WP.  1: f16 weights, as the other packed kernels.  More where
+// the general vector kernel held weights in f32: f16 hi + lo (2; weights
+// carry 2^8 so the lo parts stay normal), bf16 hi + mid + lo (3); plain bf16
+// layers always take hi + lo (2), as attn_plain_kernel.  Scores: packed keys
+// K_hi Q_hi + K_hi Q_lo + K_lo Q_hi (f32-class); plain keys are exact in
+// their type and so are the queries, which share it: one product.
+//
+// Masked tokens keep the other kernels' rules (-FLT_MAX scores, uniform rows
+// where everything is masked); a block only walks the tokens that some row of
+// it sees: up to the last causal limit, and between the first and last key
+// that gen_mask_range_kernel found kept, its splits sharing that range evenly.
+#pragma once
+
+#include "tq_attn_general.h"
+#include "tq_attn_mfma.h"
+#include "tq_attn_slots.h"
+#include "tq_attn_small.h"
+
+namespace tq {
+
+enum WideSrc { kWidePacked = 0, kWideF16 = 1, kWideBf16 = 2 };
+
+constexpr int kWideNW = 8;
+constexpr int kWideThreads = 64 * kWideNW;
+
+// The smallest built (key steps of 32, value blocks of 16) that holds the
+// dims; false where none does.
+inline bool wide_dims(int Dk, int Dv, int& ks, int& ct) {
+  const int sizes[5][2] = {{2, 4}, {3, 6}, {4, 8}, {6, 8}, {8, 16}};
+  for (const auto& z : sizes)
+    if (Dk <= 32 * z[0] && Dv <= 16 * z[1]) {
+      ks = z[0];
+      ct = z[1];
+      return true;
+    }
+  return false;
+}
+
+// 16-row tiles per wave and query rows per workgroup at ks key steps
+constexpr int wide_rt(int ks) { return ks <= 4 ? 2 : 1; }
+constexpr int wide_block_rows(int ks) { return 16 * wide_rt(ks) * kWideNW; }
+
+template <int KS, int CT, int RT, int SRC, int WP>
+struct WideShape {
+  static constexpr bool PACKED = SRC == kWidePacked;
+  static constexpr int DKP = 32 * KS;
+  static constexpr int DVP = 16 * CT;
+  static constexpr int SUB = PACKED && DKP + DVP > 256 ? 32 : 64;  // tokens per step
+  static constexpr int H = SUB / 32;                               // 32-token halves per step
+  static constexpr int PARTS = PACKED ? 2 : 1;                     // hi / lo operand parts
+  static constexpr int ROWS = 16 * RT * kWideNW;                   // query rows per workgroup
+  static constexpr int KROW = 2 * DKP + 16;   // bytes per key row (f16, padded)
+  static constexpr int VCT = H * 1024 + 32;   // bytes per 16-column value block; + 32: blocks of one
+                                              // token's row start in different banks
+  static constexpr int KTAB = 0;
+  static constexpr int VTAB = KTAB + (PACKED ? 16384 : 0);  // pair tables: up to 256 keys x 8 or 64 x 32 entries
+  static constexpr int KHI = VTAB + (PACKED ? 16384 : 0);
+  static constexpr int KLO = KHI + SUB * KROW;
+  static constexpr int VHI = KHI + PARTS * SUB * KROW;
+  static constexpr int VLO = VHI + CT * VCT;
+  static constexpr int NRM = VHI + PARTS * CT * VCT;  // SUB key norms, SUB value norms
+  static constexpr int RNG = NRM + (PACKED ? SUB * 8 : 0);
+  static constexpr int BYTES = RNG + kWideNW * 8;
+  static constexpr int KU = SUB * DKP / 8 / kWideThreads + (SUB * DKP / 8 % kWideThreads != 0);  // units of 8 coordinates per thread
+  static constexpr int VU = SUB * DVP / 8 / kWideThreads + (SUB * DVP / 8 % kWideThreads != 0);
+  static constexpr int RW = PACKED ? 2 : 4;  // registers per loaded unit
+  static_assert(BYTES <= 160 * 1024, "wide kernel LDS");
+  static_assert(KHI % 16 == 0 && VHI % 16 == 0 && VCT % 16 == 0 && NRM % 16 == 0, "16-byte LDS pieces");
+  static_assert(SUB * DKP / 8 % 64 == 0 && SUB * DVP / 8 % 64 == 0, "whole waves of units");
+};
+
+// The general path kept f32 weights: more pieces, and array masks.
+template <int SRC, int WP>
+constexpr bool wide_general() {
+  return WP == (SRC == kWideBf16 ? 3 : 2);
+}
+
+template <int SRC>
+__device__ __forceinline__ f32x4_t mfma_wide(u32x4_t a, u32x4_t b, f32x4_t c) {
+  typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+  if constexpr (SRC == kWideBf16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, a), __builtin_bit_cast(bf8_t, b), c, 0, 0, 0);
+  else
+    return mfma_f16(a, b, c);
+}
+
+// Eight mask bytes (nonzero = keep) of keys tok .. tok + 7 of one mask row:
+// one 8-byte load where keys are adjacent, else one load per key; keys at or
+// past n (the window's end) are not read and count as kept.
+__device__ __forceinline__ uint2 wide_mask_bytes(const uint8_t* row, int64_t st, int tok, int n) {
+  if (st == 1 && tok + 8 <= n) {
+    uint2 v;
+    __builtin_memcpy(&v, row + tok, 8);
+    return v;
+  }
+  uint32_t w[2] = {0u, 0u};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t k = tok + j < n ? (row[(tok + j) * st] != 0 ? 1u : 0u) : 1u;
+    w[j >> 2] |= k << (8 * (j & 3));
+  }
+  return make_uint2(w[0], w[1]);
+}
+
+// An additive mask entry in log2 units; finite entries stay finite.
+__device__ __forceinline__ float wide_mask_add(const GenParams& p, int64_t off) {
+  float m;
+  if (p.mask_kind == TQ_MASK_ADD_F32)
+    m = static_cast<const float*>(p.mask)[off];
+  else if (p.mask_kind == TQ_MASK_ADD_F16)
+    m = f16_bits_to_f32(static_cast<const uint16_t*>(p.mask)[off]);
+  else
+    m = bf16_bits_to_f32(static_cast<const uint16_t*>(p.mask)[off]);
+  const float t = m * 1.4426950408889634f;
+  return (t == -INFINITY && m != -INFINITY) ? -FLT_MAX : t;
+}
+
+template <int KS, int CT, int RT, int SRC, int WP>
+__global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int n_blocks) {
+  using S = WideShape<KS, CT, RT, SRC, WP>;
+  constexpr bool PACKED = S::PACKED;
+  constexpr bool GEN = wide_general<SRC, WP>();
+  constexpr int SUB = S::SUB, H = S::H;
+  constexpr float kLazy = 7.f;
+  constexpr int kWExp = (SRC != kWideBf16 && WP > 1) ? 8 : 0;  // weights carry 2^kWExp
+  __shared__ __align__(16) unsigned char lds[S::BYTES];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15;
+  const int g = lane >> 4;
+  // workgroup ids go to the 8 XCDs in turn: with a multiple of 8 (sequence,
+  // kv head) pairs, pair h runs on XCD h % 8 (its K/V enter one L2 once)
+  int pair, wi;
+  {
+    const int id = blockIdx.x;
+    const int per = n_blocks * p.n_splits;
+    if ((p.B * p.Hkv) % 8 == 0) {
+      const int k = id >> 3;
+      pair = (k / per) * 8 + (id & 7);
+      wi = k % per;
+    } else {
+      pair = id / per;
+      wi = id % per;
+    }
+  }
+  const int split = wi % p.n_splits;
+  const int rb = wi / p.n_splits;
+  const int gk = pair % p.Hkv;
+  const int b = pair / p.Hkv;
+  const int RL = p.R * p.L;
+  const int row_w0 = rb * S::ROWS + 16 * RT * wave;  // first kv-head row of this wave
+  const bool wave_live = row_w0 < RL;
+  const int64_t grp0 = (static_cast<int64_t>(b) * p.Hkv + gk) * p.n_rg;  // 8-row groups of this head
+
+  int64_t start;
+  int len;
+  {
+    int64_t end = p.seq_lens ? static_cast<int64_t>(p.seq_lens[b]) : p.T;
+    end = end > p.T ? p.T : (end < 0 ? 0 : end);
+    int64_t s0 = p.seq_starts ? static_cast<int64_t>(p.seq_starts[b]) : 0;
+    s0 = s0 < 0 ? 0 : (s0 > end ? end : s0);
+    start = s0;
+    len = static_cast<int>(end - s0);
+  }
+
+  // ---- rows of this wave: causal limits, mask rows, the keys they see
+  bool row_ok[RT];
+  int lim[RT];        // causal: tokens t <= lim (relative to the window) are visible
+  int64_t mrow[GEN ? RT : 1];
+  int wlo = INT32_MAX, whi = 0, lim_min = INT32_MAX;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int rr_lane = row_w0 + 16 * rt + n;
+    row_ok[rt] = rr_lane < RL;
+    const int rr = row_ok[rt] ? rr_lane : 0;
+    const int r = rr / p.L;
+    const int l = rr - r * p.L;
+    lim[rt] = p.causal ? len - p.L + l : INT32_MAX;
+    int lo = 0, hi = p.causal && lim[rt] >= 0 && p.mask_kind == TQ_MASK_NONE ? lim[rt] + 1 : len;
+    if constexpr (GEN) {
+      mrow[rt] = b * p.m_sb + gk * p.m_sg + r * p.m_sr + l * p.m_sl + start * p.m_st;
+      if (p.mrange) {
+        const int2 mr = p.mrange[b * p.mr_sb + gk * p.mr_sg + r * p.mr_sr + l * p.mr_sl];
+        lo = mr.x;
+        hi = mr.y;
+      }
+    }
+    if (row_ok[rt]) {
+      lim_min = min(lim_min, lim[rt]);
+      wlo = min(wlo, lo);
+      whi = max(whi, hi);
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    lim_min = min(lim_min, __shfl_xor(lim_min, o, 64));
+    wlo = min(wlo, __shfl_xor(wlo, o, 64));
+    whi = max(whi, __shfl_xor(whi, o, 64));
+  }
+  lim_min = __builtin_amdgcn_readfirstlane(lim_min);
+  wlo = __builtin_amdgcn_readfirstlane(wlo);
+  whi = __builtin_amdgcn_readfirstlane(whi);
+  int2* rng = reinterpret_cast<int2*>(lds + S::RNG);
+  if (lane == 0) rng[wave] = make_int2(wlo, whi);
+  __syncthreads();
+  int blo = INT32_MAX, bhi = 0;
+#pragma unroll
+  for (int w = 0; w < kWideNW; ++w) {
+    blo = min(blo, rng[w].x);
+    bhi = max(bhi, rng[w].y);
+  }
+  bhi = min(bhi, len);
+  blo = min(blo, bhi);
+  blo = __builtin_amdgcn_readfirstlane(blo);
+  bhi = __builtin_amdgcn_readfirstlane(bhi);
+  // the block's tokens in n_splits even pieces of whole 32-token halves
+  const int piece = ((bhi - blo + p.n_splits - 1) / p.n_splits + 31) / 32 * 32;
+  const int64_t tb64 = blo + static_cast<int64_t>(split) * piece;
+  if (tb64 >= bhi) {  // no tokens: a neutral partial per row (the merge skips it)
+    for (int r = tid; r < S::ROWS; r += kWideThreads) {
+      const int rr = rb * S::ROWS + r;
+      if (rr >= RL) continue;
+      float* pm = p.pml + ((grp0 + rr / 8) * p.n_splits + split) * 16 + (rr % 8) * 2;
+      pm[0] = -INFINITY;
+      pm[1] = 0.f;
+    }
+    return;
+  }
+  const int t_begin = static_cast<int>(tb64);
+  const int t_end = min(bhi, t_begin + piece);
+  const int ntiles = (t_end - t_begin + SUB - 1) / SUB;
+  const int64_t rowbase = (static_cast<int64_t>(b) * p.Hkv + gk) * p.cap + start;
+
+  // ---- loads of this thread's units: unit e = tid + 512 u covers 8
+  // coordinates of token e / (dims / 8).  A token past the split's end reads
+  // the last one instead (its score is masked below).
+  const char* const kbase = static_cast<const char*>(p.k) + rowbase * (PACKED ? p.kpw * 4 : p.Dk * 2);
+  const char* const vbase = static_cast<const char*>(p.v) + rowbase * (PACKED ? p.vpw * 4 : p.Dv * 2);
+  const int kstride = PACKED ? p.kpw * 4 : p.Dk * 2;
+  const int vstride = PACKED ? p.vpw * 4 : p.Dv * 2;
+  const int kb = p.kbits, vb = p.vbits;
+  uint32_t kreg[S::KU][S::RW], vreg[S::VU][S::RW];
+  float nreg = 0.f;
+  auto unit_load = [&](const char* base, int stride, int bits, int pw, int dim, int c8, int tok, uint32_t (&r)[S::RW]) {
+    const char* row = base + static_cast<int64_t>(min(tok, t_end - 1)) * stride;
+    if constexpr (PACKED) {
+      // the unit's 8 * bits bits start in word w0 and end in w0 or w0 + 1
+      // (3 bits); padding units stay inside the row
+      const int w0 = min((8 * bits * c8) >> 5, pw - 1);
+      const uint32_t* rw = reinterpret_cast<const uint32_t*>(row);
+      r[0] = rw[w0];
+      r[1] = rw[min(w0 + 1, pw - 1)];
+    } else {
+      uint4 x = make_uint4(0u, 0u, 0u, 0u);
+      if (8 * c8 < dim) x = reinterpret_cast<const uint4*>(row)[c8];
+      r[0] = x.x;
+      r[1] = x.y;
+      r[2] = x.z;
+      r[3] = x.w;
+    }
+  };
+  constexpr int KC8 = S::DKP / 8, VC8 = S::DVP / 8;
+  auto load_k = [&](int i) {
+    const int t0 = t_begin + i * SUB;
+#pragma unroll
+    for (int u = 0; u < S::KU; ++u) {
+      const int e = tid + u * kWideThreads;
+      if (e < SUB * KC8) unit_load(kbase, kstride, kb, p.kpw, p.Dk, e % KC8, t0 + e / KC8, kreg[u]);
+    }
+    if constexpr (PACKED) {
+      if (tid < 2 * SUB) {  // key norms, then value norms
+        const int64_t at = rowbase + min(t0 + (tid & (SUB - 1)), t_end - 1);
+        nreg = load_norm(tid < SUB ? p.kn : p.vn, p.norm_dtype, at);
+      }
+    }
+  };
+  auto load_v = [&](int i) {
+    const int t0 = t_begin + i * SUB;
+#pragma unroll
+    for (int u = 0; u < S::VU; ++u) {
+      const int e = tid + u * kWideThreads;
+      if (e < SUB * VC8) unit_load(vbase, vstride, vb, p.vpw, p.Dv, e % VC8, t0 + e / VC8, vreg[u]);
+    }
+  };
+  load_k(0);
+  load_v(0);
+
+  // ---- query rows as prepared by wide_qprep_kernel: lane (row n, g) holds
+  // coordinates 32 s + 8 g .. + 7 (packed: hi and lo parts of q_rot * sq)
+  u32x4_t qh[RT][KS], ql[PACKED ? RT : 1][PACKED ? KS : 1];
+  float qmul[RT];  // MFMA units -> score units (log2)
+  {
+    const int64_t pair_row0 = static_cast<int64_t>(pair) * RL;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int rr = row_ok[rt] ? row_w0 + 16 * rt + n : 0;
+      const u32x4_t* src = reinterpret_cast<const u32x4_t*>(p.qhl) + (pair_row0 + rr) * (4 * KS * S::PARTS) + g;
+      const u32x4_t z = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        qh[rt][s] = src[4 * s];
+        qh[rt][s] = row_ok[rt] ? qh[rt][s] : z;
+        if constexpr (PACKED) {
+          ql[rt][s] = src[4 * KS + 4 * s];
+          ql[rt][s] = row_ok[rt] ? ql[rt][s] : z;
+        }
+      }
+      qmul[rt] = PACKED ? p.qsq[pair_row0 + rr] : 1.4426950408889634f;
+    }
+  }
+
+  // ---- pair tables: entry (a | b << bits) = (hi c_a | hi c_b << 16, lo c_a | lo c_b << 16)
+  // of the codebooks scaled by a power of two (largest magnitude in [2^12, 2^13))
+  float sv = 1.f;
+  const int kesh = kb == 4 ? 6 : 8, vesh = vb == 4 ? 6 : 8;  // log2 of an entry's bytes over its copies
+  if constexpr (PACKED) {
+    float* cbl = reinterpret_cast<float*>(lds + S::KHI);
+    if (tid < (1 << kb)) cbl[tid] = p.kcb[tid];
+    if (tid < (1 << vb)) cbl[16 + tid] = p.vcb[tid];
+    __syncthreads();
+    float kmax = 0.f, vmax = 0.f;
+    for (int i = 0; i < (1 << kb); ++i) kmax = fmaxf(kmax, fabsf(cbl[i]));
+    for (int i = 0; i < (1 << vb); ++i) vmax = fmaxf(vmax, fabsf(cbl[16 + i]));
+    const float sk = f16_split_scale(kmax);
+    sv = f16_split_scale(vmax);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) qmul[rt] = 1.4426950408889634f / (sk * qmul[rt]);
+    for (int e = tid; e < ((1 << (2 * kb + kesh)) >> 3); e += kWideThreads) {
+      const int key = e >> (kesh - 3);
+      uint32_t h0, l0, h1, l1;
+      split_f16(cbl[key & ((1 << kb) - 1)] * sk, h0, l0);
+      split_f16(cbl[key >> kb] * sk, h1, l1);
+      *reinterpret_cast<uint2*>(lds + S::KTAB + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
+    }
+    for (int e = tid; e < ((1 << (2 * vb + vesh)) >> 3); e += kWideThreads) {
+      const int key = e >> (vesh - 3);
+      uint32_t h0, l0, h1, l1;
+      split_f16(cbl[16 + (key & ((1 << vb) - 1))] * sv, h0, l0);
+      split_f16(cbl[16 + (key >> vb)] * sv, h1, l1);
+      *reinterpret_cast<uint2*>(lds + S::VTAB + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
+    }
+    __syncthreads();
+  }
+  const uint32_t ktab = S::KTAB + (lane & ((1 << (kesh - 3)) - 1)) * 8;
+  const uint32_t vtab = S::VTAB + (lane & ((1 << (vesh - 3)) - 1)) * 8;
+
+  // 8 coordinates of a unit as hi and lo parts (packed) or as stored
+  auto unit_parts = [&](const uint32_t (&r)[S::RW], int bits, int c8, uint32_t tab, int esh, uint4& hi, uint4& lo) {
+    if constexpr (PACKED) {
+      const uint32_t x = __builtin_amdgcn_alignbit(r[1], r[0], (8 * bits * c8) & 31);
+      const uint32_t kmask = (1u << (2 * bits)) - 1u;
+      uint2 e[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) e[m] = lds_at<uint2>(lds, tab + (((x >> (2 * m * bits)) & kmask) << esh));
+      hi = make_uint4(e[0].x, e[1].x, e[2].x, e[3].x);
+      lo = make_uint4(e[0].y, e[1].y, e[2].y, e[3].y);
+    } else {
+      hi = make_uint4(r[0], r[1], r[2], r[3]);
+    }
+  };
+  auto put_k = [&]() {
+#pragma unroll
+    for (int u = 0; u < S::KU; ++u) {
+      const int e = tid + u * kWideThreads;
+      if (e < SUB * KC8) {
+        const int t = e / KC8, c8 = e % KC8;
+        uint4 hi, lo;
+        unit_parts(kreg[u], kb, c8, ktab, kesh, hi, lo);
+        unsigned char* d = lds + S::KHI + ((t & ~31) + tile_kslot(t & 31)) * S::KROW + c8 * 16;
+        *reinterpret_cast<uint4*>(d) = hi;
+        if constexpr (PACKED) *reinterpret_cast<uint4*>(d + (S::KLO - S::KHI)) = lo;
+      }
+    }
+    if constexpr (PACKED)
+      if (tid < 2 * SUB) reinterpret_cast<float*>(lds + S::NRM)[tid] = nreg;
+  };
+  auto put_v = [&]() {
+#pragma unroll
+    for (int u = 0; u < S::VU; ++u) {
+      const int e = tid + u * kWideThreads;
+      if (e < SUB * VC8) {
+        const int t = e / VC8, c8 = e % VC8;
+        uint4 hi, lo;
+        unit_parts(vreg[u], vb, c8, vtab, vesh, hi, lo);
+        unsigned char* d = lds + S::VHI + (c8 >> 1) * S::VCT + (t >> 5) * 1024 + tile_vslot(t & 31) * 32 + (c8 & 1) * 16;
+        *reinterpret_cast<uint4*>(d) = hi;
+        if constexpr (PACKED) *reinterpret_cast<uint4*>(d + (S::VLO - S::VHI)) = lo;
+      }
+    }
+  };
+
+  f32x4_t O[RT][CT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) O[rt][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_row[RT];  // reference maximum of the row (log2 units)
+  float l_acc[RT];  // this lane's share of the row's sum
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    m_row[rt] = -INFINITY;
+    l_acc[rt] = 0.f;
+  }
+  int E = PACKED ? kWExp - 126 : 0;  // value norms <= 2^E (weights carry 2^-E), shared by the wave's rows
+  float vsc = ldexpf(1.f, kWExp - E);
+  float vlim = ldexpf(1.f, E);
+
+  const uint32_t ka = S::KHI + n * S::KROW + 16 * g;
+  uint32_t vtr[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) vtr[h] = S::VHI + tile_vslot(8 * g + 4 * h + (n >> 2)) * 32 + (n & 3) * 8;
+  typedef __attribute__((address_space(3))) unsigned char lds_u8;
+  typedef short s16x4v __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4v lds_s16x4;
+  lds_u8* const l3 = (lds_u8*)lds;
+  auto read_tr = [&](uint32_t off) {
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(l3 + off)));
+  };
+
+  // S^T of half hf of the step in the K slot
+  auto scores = [&](int hf, f32x4_t (&C)[RT][2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t at = ka + (32 * hf + 16 * h) * S::KROW;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) C[rt][h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const u32x4_t ah = lds_at<u32x4_t>(lds, at + 64 * s);
+        if constexpr (PACKED) {
+          const u32x4_t al = lds_at<u32x4_t>(lds, at + (S::KLO - S::KHI) + 64 * s);
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) {
+            C[rt][h] = mfma_wide<SRC>(ah, qh[rt][s], C[rt][h]);
+            C[rt][h] = mfma_wide<SRC>(ah, ql[rt][s], C[rt][h]);
+            C[rt][h] = mfma_wide<SRC>(al, qh[rt][s], C[rt][h]);
+          }
+        } else {
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) C[rt][h] = mfma_wide<SRC>(ah, qh[rt][s], C[rt][h]);
+        }
+      }
+    }
+  };
+
+  // O rows 4 g + k of this lane take the factor of row 4 g + k
+  float fac[RT];
+  bool pending = false;  // wave-uniform: fac applies between the step's halves
+  auto rescale = [&](const float (&f)[RT]) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      float ar[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ar[k] = __shfl(f[rt], 4 * g + k, 64);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) O[rt][ct][k] *= ar[k];
+    }
+  };
+
+  // softmax of half hf: tokens t0 + 8 g + j of this lane; the weights as A operands
+  auto softmax = [&](int t0, int hf, const f32x4_t (&C)[RT][2], const uint2 (&mk)[RT], u32x4_t (&A)[RT][WP]) {
+    float knv[8], vnv[8];
+    float vm = 0.f;
+    if constexpr (PACKED) {
+      const float* kn = reinterpret_cast<const float*>(lds + S::NRM) + 32 * hf + 8 * g;
+      *reinterpret_cast<float4*>(knv) = *reinterpret_cast<const float4*>(kn);
+      *reinterpret_cast<float4*>(knv + 4) = *reinterpret_cast<const float4*>(kn + 4);
+      *reinterpret_cast<float4*>(vnv) = *reinterpret_cast<const float4*>(kn + SUB);
+      *reinterpret_cast<float4*>(vnv + 4) = *reinterpret_cast<const float4*>(kn + SUB + 4);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) vm = fmaxf(vm, vnv[j]);
+    }
+    // y = n_t <q, c> in MFMA units of the row; x = y * qmul in log2 units
+    float y[RT][8];
+    bool grow = PACKED && vm > vlim;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      float ym = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        y[rt][j] = own_reg(C[rt][j >> 2][j & 3]);
+        if constexpr (PACKED) y[rt][j] *= knv[j];
+        ym = fmaxf(ym, y[rt][j]);
+      }
+      grow |= ym * qmul[rt] > m_row[rt] + kLazy;
+    }
+    bool special = t0 + 32 > t_end || t0 + 31 > lim_min;  // wave-uniform
+    if constexpr (GEN) {
+      if (p.mask_kind == TQ_MASK_BOOL) {
+        bool all = true;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) all &= mk[rt].x == 0x01010101u && mk[rt].y == 0x01010101u;
+        special |= __any(all ? 0 : 1) != 0;
+      } else if (p.mask_kind != TQ_MASK_NONE) {
+        special = true;
+      }
+    }
+    float pe[RT][8];
+    if (special || __any(grow ? 1 : 0)) {
+      // slow path: masks, a new reference maximum or norm exponent, rescale
+      float rm[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[rt][j] *= qmul[rt];
+        if (special) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const int tok = t0 + 8 * g + j;
+            if (tok > lim[rt]) y[rt][j] = -FLT_MAX;
+            if constexpr (GEN) {
+              if (p.mask_kind == TQ_MASK_BOOL) {
+                if ((((j < 4 ? mk[rt].x : mk[rt].y) >> (8 * (j & 3))) & 0xffu) == 0u) y[rt][j] = -FLT_MAX;
+              } else if (p.mask_kind != TQ_MASK_NONE) {
+                if (tok < t_end) y[rt][j] += wide_mask_add(p, mrow[rt] + tok * p.m_st);
+              }
+            }
+            if (tok >= t_end) y[rt][j] = -INFINITY;
+          }
+        }
+        rm[rt] = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) rm[rt] = fmaxf(rm[rt], y[rt][j]);
+      }
+      bool up = PACKED && vm > vlim;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) up |= rm[rt] > m_row[rt] + kLazy;
+      if (__any(up ? 1 : 0)) {
+        int e2 = E;
+        float esc = 1.f;
+        if constexpr (PACKED) {
+          const float vw = wave_max(vm);
+          if (vw > vlim) {
+            int ev;
+            frexpf(vw, &ev);
+            e2 = ev;
+          }
+          esc = ldexpf(1.f, E - e2);
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          float r = fmaxf(rm[rt], xor_lane<16>(rm[rt]));
+          {
+            const float2 hh = halves(r);
+            r = fmaxf(hh.x, hh.y);  // the row's maximum over the half
+          }
+          const float mo = m_row[rt];
+          const float mn = r > mo + kLazy ? fmaxf(mo, r) : mo;
+          const float am = mo == mn ? 1.f : (mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - mn));
+          fac[rt] = am * esc;
+          l_acc[rt] *= am;
+          m_row[rt] = mn;
+        }
+        // the step's first half rescales O here; its second half only after
+        // the first half's products, which still carry the old maximum
+        if (hf == 0)
+          rescale(fac);
+        else
+          pending = true;
+        E = e2;
+        vsc = ldexpf(1.f, kWExp - E);
+        vlim = ldexpf(1.f, E);
+      }
+      // masked keys (-FLT_MAX) weigh 1 while their whole row is masked
+      // (m = -FLT_MAX), else 0; keys past the end (-inf) always 0
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          pe[rt][j] = m_row[rt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y[rt][j] - m_row[rt]);
+    } else {
+      // every score within 2^7 of a finite reference maximum
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const float nm = -m_row[rt];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pe[rt][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[rt][j], qmul[rt], nm));
+      }
+    }
+    float vs[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) vs[j] = PACKED ? vnv[j] * vsc : vsc;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      float w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        l_acc[rt] += pe[rt][j];
+        w[j] = (PACKED || kWExp != 0) ? pe[rt][j] * vs[j] : pe[rt][j];
+      }
+#pragma unroll
+      for (int q = 0; q < WP; ++q) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (SRC == kWideBf16) {
+            const uint32_t a = f32_to_bf16_bits(w[2 * j]), c = f32_to_bf16_bits(w[2 * j + 1]);
+            A[rt][q][j] = a | (c << 16);
+            if (q + 1 < WP) {
+              w[2 * j] -= bf16_bits_to_f32(static_cast<uint16_t>(a));
+              w[2 * j + 1] -= bf16_bits_to_f32(static_cast<uint16_t>(c));
+            }
+          } else {
+            const uint32_t a = pack_f16x2(w[2 * j], w[2 * j + 1]);
+            A[rt][q][j] = a;
+            if (q + 1 < WP) {
+              w[2 * j] -= f16_bits_to_f32(static_cast<uint16_t>(a));
+              w[2 * j + 1] -= f16_bits_to_f32(static_cast<uint16_t>(a >> 16));
+            }
+          }
+        }
+      }
+    }
+  };
+
+  // O += P V of half hf of the step in the V slot
+  auto pv = [&](int hf, const u32x4_t (&A)[RT][WP]) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const uint32_t off = ct * S::VCT + hf * 1024;
+      const uint2 h0 = read_tr(vtr[0] + off);
+      const uint2 h1 = read_tr(vtr[1] + off);
+      const u32x4_t bh = {h0.x, h0.y, h1.x, h1.y};
+      if constexpr (PACKED) {
+        const uint2 g0 = read_tr(vtr[0] + off + (S::VLO - S::VHI));
+        const uint2 g1 = read_tr(vtr[1] + off + (S::VLO - S::VHI));
+        const u32x4_t bl = {g0.x, g0.y, g1.x, g1.y};
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          O[rt][ct] = mfma_wide<SRC>(A[rt][0], bh, O[rt][ct]);
+          O[rt][ct] = mfma_wide<SRC>(A[rt][0], bl, O[rt][ct]);
+          if constexpr (WP > 1) O[rt][ct] = mfma_wide<SRC>(A[rt][1], bh, O[rt][ct]);
+        }
+      } else {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int q = 0; q < WP; ++q) O[rt][ct] = mfma_wide<SRC>(A[rt][q], bh, O[rt][ct]);
+      }
+    }
+  };
+
+  // ---- K of step 0 in its slot, K of step 1 and V of step 0 loading
+  put_k();
+  if (ntiles > 1) load_k(1);
+  lds_barrier();
+  const bool lead = wave < kWideNW / 2;
+#pragma unroll 1
+  for (int i = 0; i < ntiles; ++i) {
+    const int t0 = t_begin + i * SUB;
+    const bool act = wave_live && t0 < whi && t0 + SUB > wlo;  // some row of the wave sees a token
+    u32x4_t A[H][RT][WP];
+    if (lead) {
+      put_v();
+      if (i + 1 < ntiles) load_v(i + 1);
+    }
+    if (act) {
+#pragma unroll
+      for (int hf = 0; hf < H; ++hf) {
+        uint2 mk[RT];
+        if constexpr (GEN) {
+          if (p.mask_kind == TQ_MASK_BOOL) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+              mk[rt] = wide_mask_bytes(static_cast<const uint8_t*>(p.mask) + mrow[rt], p.m_st, t0 + 32 * hf + 8 * g, len);
+          }
+        }
+        f32x4_t C[RT][2];
+        scores(hf, C);
+        softmax(t0 + 32 * hf, hf, C, mk, A[hf]);
+      }
+    }
+    if (!lead) {
+      put_v();
+      if (i + 1 < ntiles) load_v(i + 1);
+    }
+    lds_barrier();
+    if (lead && i + 1 < ntiles) {
+      put_k();
+      if (i + 2 < ntiles) load_k(i + 2);
+    }
+    if (act) {
+#pragma unroll
+      for (int hf = 0; hf < H; ++hf) {
+        if (hf > 0 && pending) {
+          rescale(fac);
+          pending = false;
+        }
+        pv(hf, A[hf]);
+      }
+    }
+    if (!lead && i + 1 < ntiles) {
+      put_k();
+      if (i + 2 < ntiles) load_k(i + 2);
+    }
+    lds_barrier();
+  }
+  // ---- partials: (o, m, l) per row, o = O * 2^E / sv (packed: in the rotated value basis)
+  if (!wave_live) return;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    float lr = l_acc[rt] + xor_lane<16>(l_acc[rt]);
+    {
+      const float2 h = halves(lr);
+      lr = h.x + h.y;
+    }
+    const int rr = row_w0 + 16 * rt + n;
+    if (g == 0 && row_ok[rt]) {
+      float* pm = p.pml + ((grp0 + rr / 8) * p.n_splits + split) * 16 + (rr % 8) * 2;
+      pm[0] = m_row[rt] * 0.6931471805599453f;  // natural-log units
+      pm[1] = lr;
+    }
+  }
+  const float osc = ldexpf(1.f, E - kWExp) / sv;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int rr = row_w0 + 16 * rt + 4 * g + k;
+      if (rr >= RL) continue;
+      float* po = p.po + (((grp0 + rr / 8) * p.n_splits + split) * 8 + rr % 8) * static_cast<int64_t>(p.Dv);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        if (16 * ct + n < p.Dv) po[16 * ct + n] = O[rt][ct][k] * osc;
+    }
+}
+
+}  // namespace tq
