@@ -7,6 +7,7 @@
 #include "tq_attn_merge.h"
 #include "tq_attn_tile.h"
 #include "tq_attn_wide_prep.h"
+#include "tq_rotate.h"
 
 namespace tq {
 namespace {
@@ -731,7 +732,9 @@ __global__ __launch_bounds__(256) void gen_merge_flat_kernel(GenParams p, I n_it
     v2 *= sg.z * p.rscale_v;
     v3 *= sg.w * p.rscale_v;
   }
-  if (p.q_dtype == TQ_DTYPE_F32) {
+  if (p.merged) {
+    *reinterpret_cast<float4*>(p.merged + o) = make_float4(v0, v1, v2, v3);
+  } else if (p.q_dtype == TQ_DTYPE_F32) {
     *reinterpret_cast<float4*>(static_cast<float*>(p.out) + o) = make_float4(v0, v1, v2, v3);
   } else {
     const bool f16 = p.q_dtype == TQ_DTYPE_F16;
@@ -831,7 +834,7 @@ GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   return gp;
 }
 
-// Workspace: [q_rot rows DkP f32 (packed)][po][pml][query words][sq rows][mask ranges]
+// Workspace: [q_rot, later merged rows, f32 (packed)][po][pml][query words][sq rows][mask ranges]
 struct WideLayout {
   int64_t po, pml, qhl, qsq, mrange, bytes;
 };
@@ -842,10 +845,10 @@ WideLayout wide_layout(int B, int Hq, int Hkv, int L, int Dk, int Dv, const GenP
   const int64_t rows = static_cast<int64_t>(B) * Hq * L;
   const int64_t parts = static_cast<int64_t>(B) * Hkv * gp.n_rg * gp.n_splits * kGenNQ;
   WideLayout w{};
-  w.po = packed ? a256(rows * round32(Dk) * 4) : 0;
+  w.po = packed ? a256(rows * std::max(round32(Dk), Dv) * 4) : 0;  // q_rot; then the merged rows
   w.pml = w.po + a256(parts * Dv * 4);
   w.qhl = w.pml + a256(parts * 2 * 4);
-  w.qsq = w.qhl + a256(rows * ks * 64 * (packed ? 2 : 1));
+  w.qsq = w.qhl + a256(rows * ks * 64 * (packed ? 2 : 1));  // packed dense queries leave it unused
   w.mrange = w.qsq + (packed ? a256(rows * 4) : 0);
   w.bytes = w.mrange + (mask ? a256(rows * 8) : 0);
   return w;
@@ -869,7 +872,7 @@ int run_wide(GenParams& p, int64_t rows, bool plain, hipStream_t st) {
   else if (wide_had_queries(p.Dk, p.k_rot_kind))
     hipLaunchKernelGGL(wide_qprep_kernel<kWideQHad>, qgrid, dim3(kWideQpThreads), 0, st, p, nr, 4 * ks);
   else
-    hipLaunchKernelGGL(wide_qprep_kernel<kWideQRows>, qgrid, dim3(kWideQpThreads), 0, st, p, nr, 4 * ks);
+    p.q_rows32 = 1;  // f32 rows already in p.qrot
   int rc = check_launch("wide_qprep_kernel");
   if (rc) return rc;
   if (p.mask_kind != TQ_MASK_NONE && !p.causal) {
@@ -977,6 +980,32 @@ void launch_qprep_mode(const GenParams& p, int64_t rows, int mode, const float* 
     case TQ_DTYPE_F16: hipLaunchKernelGGL(gen_qprep_kernel<TQ_DTYPE_F16>, grid, dim3(kGenThreads), 0, st, p, rows, mode, mat, dst); break;
     default: hipLaunchKernelGGL(gen_qprep_kernel<TQ_DTYPE_BF16>, grid, dim3(kGenThreads), 0, st, p, rows, mode, mat, dst); break;
   }
+}
+
+// q_s @ mat^T for every query row: the matrix-core rotation to d = 256, the
+// vector one beyond (gen_qprep_kernel takes 38 us for 8192 rows of 256, the
+// rotation 10 us; 6.4 and 4.0 us for 256 rows of 96, 11 and 8.3 us for 2240 of 192).
+void launch_dense_queries(const GenParams& p, int64_t rows, const float* mat, float* dst, hipStream_t st) {
+  if (p.Dk > kRotateMaxDim || rows > INT32_MAX) return launch_qprep_mode(p, rows, 2, mat, dst, st);
+  RotateArgs a{};
+  a.x = p.q;
+  a.x_sb = p.q_sb;
+  a.x_sh = p.q_sh;
+  a.x_sl = p.q_sl;
+  a.x_dtype = p.q_dtype;
+  const int es = p.q_dtype == TQ_DTYPE_F32 ? 4 : 2;
+  a.x_vec = p.Dk * es % 16 == 0 &&
+            ((reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(mat) |
+              static_cast<uintptr_t>((p.q_sb | p.q_sh | p.q_sl) * es)) & 15u) == 0;
+  a.Hq = p.Hq;
+  a.L = p.L;
+  a.scale = p.scale_q;
+  a.rows = static_cast<int>(rows);
+  a.k = a.n = p.Dk;
+  a.mat = mat;
+  a.out = dst;
+  a.out_stride = p.DkP;
+  launch_rotate_queries(a, st);
 }
 
 bool pow2(int d) { return d > 0 && (d & (d - 1)) == 0; }
@@ -1224,9 +1253,9 @@ int general_attention(const GenCall& c) {
   else if (c.k_rot_kind == TQ_ROT_HADAMARD && kb > 0)
     launch_qprep_mode(p, rows, 1, c.k_rot, p.qrot, st);
   else if (c.k_rot_kind == TQ_ROT_DENSE)
-    launch_qprep_mode(p, rows, 2, c.k_rot, p.qrot, st);
-  if (prod) launch_qprep_mode(p, rows, 2, c.projection, p.qproj, st);
-  int rc = check_launch("gen_qprep_kernel");
+    launch_dense_queries(p, rows, c.k_rot, p.qrot, st);
+  if (prod) launch_dense_queries(p, rows, c.projection, p.qproj, st);
+  int rc = check_launch("query transform");
   if (rc) return rc;
   if (tile && !wide) {
     const int64_t wgs = (rows + kTileQpRows * (kTileQpThreads / 64) - 1) / (kTileQpRows * (kTileQpThreads / 64));
@@ -1239,8 +1268,14 @@ int general_attention(const GenCall& c) {
        : tile ? launch_tile_partial(p, kb, c.v_bits, st)
               : launch_gen_partial(p, kb, plain ? 0 : c.v_bits, st);
   if (rc) return rc;
+  // dense R_V^-1: merged rows in f32 (where q_rot was), then one matrix-core
+  // rotation (gen_merge_kernel, which does both on the vector ALUs, takes 207 us
+  // for 8192 rows of 256 and 15 us for 256 rows of 96; these two 24 and 9 us)
+  const bool merge_dense = !plain && c.v_rot_kind == TQ_ROT_DENSE && c.Dv % 4 == 0 && c.Dv <= kRotateMaxDim &&
+                           (wide || c.Dv <= p.DkP) && rows <= INT32_MAX;
+  p.merged = merge_dense ? p.qrot : nullptr;
   // the flat merge takes 4 value columns per thread: plain values need Dv % 4 == 0
-  if ((plain && c.Dv % 4 == 0) || p.merge_had) {
+  if ((plain && c.Dv % 4 == 0) || p.merge_had || merge_dense) {
     const int64_t items = static_cast<int64_t>(c.B) * c.Hkv * (c.Hq / c.Hkv) * c.L * (c.Dv / 4);
     const int64_t pair_items = static_cast<int64_t>(c.Hq / c.Hkv) * c.L * (c.Dv / 4);
     // after the tile kernel, each pair's merge blocks run on the XCD whose
@@ -1253,7 +1288,17 @@ int general_attention(const GenCall& c) {
       hipLaunchKernelGGL(gen_merge_flat_kernel<int>, fgrid, dim3(256), 0, st, p, static_cast<int>(items));
     else
       hipLaunchKernelGGL(gen_merge_flat_kernel<int64_t>, fgrid, dim3(256), 0, st, p, items);
-    return check_launch("gen_merge_flat_kernel");
+    rc = check_launch("gen_merge_flat_kernel");
+    if (rc || !merge_dense) return rc;
+    RotateArgs a{};
+    a.x = p.merged;
+    a.rows = static_cast<int>(rows);
+    a.k = a.n = c.Dv;
+    a.mat = c.v_rot;
+    a.out = c.out;
+    a.out_dtype = c.q_dtype;
+    a.out_stride = c.Dv;
+    return launch_rotate_rows(a, st);
   }
   const unsigned zc = (!plain && c.v_rot_kind == TQ_ROT_DENSE) ? static_cast<unsigned>((c.Dv + 63) / 64) : 1u;
   const dim3 mgrid(static_cast<unsigned>(c.Hkv * gp.n_rg), static_cast<unsigned>(c.B), zc);

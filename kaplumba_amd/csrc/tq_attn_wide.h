@@ -27,7 +27,7 @@
 // the call before: 512 queries x 8192 tokens under a 4096-key boolean window,
 // d = 128, 3 bits: 2815 -> 170 us (vector kernel); 2 x 500 queries x 4097
 // tokens, d = 64, K3/V4: 243 -> 129 us, and 512 queries x 4096 tokens, d = 256,
-// K4/V2, dense: 540 -> 372 us (attn_mfma_kernel: decodes per 16 or 4 rows);
+// K4/V2, dense: 540 -> 165 us (attn_mfma_kernel: decodes per 16 or 4 rows);
 // 512 queries x 8192 plain bf16 tokens, d = 128: 345 -> 170 us
 // (attn_plain_kernel: reads K/V per 16 rows).  Partial kernels alone: 156, 119,
 // 119 and 172 us.
@@ -320,8 +320,10 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
   load_k(0);
   load_v(0);
 
-  // ---- query rows as prepared by wide_qprep_kernel: lane (row n, g) holds
-  // coordinates 32 s + 8 g .. + 7 (packed: hi and lo parts of q_rot * sq)
+  // ---- query rows: lane (row n, g) holds coordinates 32 s + 8 g .. + 7.
+  // Packed keys: hi and lo parts of q_rot * sq, sq a power of two that brings
+  // the row's largest magnitude into [2^12, 2^13); from wide_qprep_kernel, or
+  // (dense rotation) formed here from the f32 rows of the rotation kernel.
   u32x4_t qh[RT][KS], ql[PACKED ? RT : 1][PACKED ? KS : 1];
   float qmul[RT];  // MFMA units -> score units (log2)
   {
@@ -329,18 +331,53 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const int rr = row_ok[rt] ? row_w0 + 16 * rt + n : 0;
-      const u32x4_t* src = reinterpret_cast<const u32x4_t*>(p.qhl) + (pair_row0 + rr) * (4 * KS * S::PARTS) + g;
-      const u32x4_t z = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        qh[rt][s] = src[4 * s];
-        qh[rt][s] = row_ok[rt] ? qh[rt][s] : z;
+      bool rows32 = false;
+      if constexpr (PACKED) rows32 = p.q_rows32 != 0;
+      if (rows32) {
         if constexpr (PACKED) {
-          ql[rt][s] = src[4 * KS + 4 * s];
-          ql[rt][s] = row_ok[rt] ? ql[rt][s] : z;
+          const float* src = p.qrot + (pair_row0 + rr) * p.DkP + 8 * g;
+          float v[KS][8];
+          float mx = 0.f;
+#pragma unroll
+          for (int s = 0; s < KS; ++s) {
+            const bool in = 32 * s < p.DkP;  // uniform: whole steps past the row are zero
+            const float4 a = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0));
+            const float4 c = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0) + 4);
+            const bool live = in && row_ok[rt];
+            v[s][0] = live ? a.x : 0.f, v[s][1] = live ? a.y : 0.f, v[s][2] = live ? a.z : 0.f, v[s][3] = live ? a.w : 0.f;
+            v[s][4] = live ? c.x : 0.f, v[s][5] = live ? c.y : 0.f, v[s][6] = live ? c.z : 0.f, v[s][7] = live ? c.w : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[s][e]));
+          }
+          mx = fmaxf(mx, xor_lane<16>(mx));
+          const float2 hm = halves(mx);
+          const float sq = f16_split_scale(fmaxf(hm.x, hm.y));
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              uint32_t h0, l0, h1, l1;
+              split_f16(v[s][2 * e] * sq, h0, l0);
+              split_f16(v[s][2 * e + 1] * sq, h1, l1);
+              qh[rt][s][e] = h0 | (h1 << 16);
+              ql[rt][s][e] = l0 | (l1 << 16);
+            }
+          qmul[rt] = sq;
         }
+      } else {
+        const u32x4_t* src = reinterpret_cast<const u32x4_t*>(p.qhl) + (pair_row0 + rr) * (4 * KS * S::PARTS) + g;
+        const u32x4_t z = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          qh[rt][s] = src[4 * s];
+          qh[rt][s] = row_ok[rt] ? qh[rt][s] : z;
+          if constexpr (PACKED) {
+            ql[rt][s] = src[4 * KS + 4 * s];
+            ql[rt][s] = row_ok[rt] ? ql[rt][s] : z;
+          }
+        }
+        qmul[rt] = PACKED ? p.qsq[pair_row0 + rr] : 1.4426950408889634f;
       }
-      qmul[rt] = PACKED ? p.qsq[pair_row0 + rr] : 1.4426950408889634f;
     }
   }
 

@@ -9,15 +9,15 @@ namespace tq {
 // Query rows for the wide kernel: words of 8 halves, word w holding
 // coordinates 8 w .. + 7, zeros past Dk.  Packed keys: q_rot times sq, a power
 // of two that brings the row's largest magnitude into [2^12, 2^13), as 4 KS
-// hi words then 4 KS lo words; q_rot = H(s * q_s) / sqrt(Dk) formed here
-// (kWideQHad, Dk = 64, 128 or 256), or read from p.qrot (kWideQRows, written
-// by gen_qprep_kernel).  Plain keys (kWideQPlain): q_s as it is, in the type it
-// shares with the cache.  q_s = round_qdtype(q * scale).
+// hi words then 4 KS lo words; q_rot = H(s * q_s) / sqrt(Dk) (kWideQHad, Dk = 64,
+// 128 or 256; other rotations reach the wide kernel as f32 rows).  Plain keys
+// (kWideQPlain): q_s as it is, in the type it shares with the cache.
+// q_s = round_qdtype(q * scale).
 // 16 lanes per row, lane j words j and j + 16, so the butterflies run over
 // coordinate bits 0-2 in registers, 3-6 across the lanes of a DPP row and 7
 // between a lane's two words.
 constexpr int kWideQpThreads = 256;
-enum WideQ { kWideQPlain = 0, kWideQHad = 1, kWideQRows = 2 };
+enum WideQ { kWideQPlain = 0, kWideQHad = 1 };
 
 template <int MODE>
 __global__ __launch_bounds__(kWideQpThreads) void wide_qprep_kernel(GenParams p, int rows, int words) {
@@ -29,17 +29,7 @@ __global__ __launch_bounds__(kWideQpThreads) void wide_qprep_kernel(GenParams p,
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[u][e] = 0.f;
-  if constexpr (MODE == kWideQRows) {
-    const float4* src = reinterpret_cast<const float4*>(p.qrot + static_cast<int64_t>(row) * p.DkP);  // zero past Dk
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int w = j + 16 * u;
-      if (w < words && 8 * w < p.DkP) {
-        *reinterpret_cast<float4*>(v[u]) = src[2 * w];
-        *reinterpret_cast<float4*>(v[u] + 4) = src[2 * w + 1];
-      }
-    }
-  } else {
+  {
     const int l = row % p.L;
     const int bh = row / p.L;
     const int64_t qo = static_cast<int64_t>(bh / p.Hq) * p.q_sb + static_cast<int64_t>(bh % p.Hq) * p.q_sh + l * p.q_sl;
