@@ -88,6 +88,14 @@ int launch_append_dense_kv(const AppendArgs& k, const AppendArgs& v, int dim, in
 // (tq_append_general.hip), for the dims the matrix-core kernels do not take.
 int launch_append_dense_general(const AppendArgs& a, int dim, int bits, int x_dtype, hipStream_t st);
 
+// Dense rotation of few vectors at dims that are multiples of 8 up to 256
+// (tq_append_few.hip): one side (sides = 1, v unused) or both in one launch, any
+// widths.  append_few_path: whether a call of n_vec vectors a side takes it;
+// paired: the other way is one append_dense_kv_kernel launch.
+bool append_few_path(int64_t n_vec, int dim, int sides, bool paired);
+int launch_append_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
+                      hipStream_t st);
+
 struct DequantGeneralArgs {
   const uint32_t* packed;
   const void* norms;

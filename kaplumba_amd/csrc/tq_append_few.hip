@@ -1,0 +1,280 @@
+// Dense-rotation append of few vectors (decode and verify steps, short chunks)
+// on v_mfma_f32_16x16x32_bf16, keys and values in one launch.
+//
+// Semantics and arithmetic as tq_append_dense.hip: y * max(n, eps) = x @ R^T from
+// bf16 pieces that sum to the f32 operands (R three; x one for bf16, two for
+// f16, three for f32), products whose orders add up to more than 2 skipped,
+// sums in f32; indices by strict compares against mid * max(n, eps).  Norms
+// take the shared tree, the dim zero-padded to whole 32-element groups, so they
+// are bit-exact.
+//
+// A workgroup takes 16 vectors and 64 coordinates (whole words at every width)
+// of one side.  Each of 4 waves owns 16 coordinates and splits their rows of R
+// straight into B fragments: no LDS, one round trip of loads; the norm is
+// formed by every wave.  Indices meet in LDS for the packing.
+#include "tq_append.h"
+
+namespace tq {
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4_t mfma_bf16(u32x4_t a, u32x4_t b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0,
+                                                 0, 0);
+}
+
+// Eight f32 values as NP bf16 pieces each (round to nearest even, exact remainders).
+template <int NP>
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4_t (&w)[NP]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = v[2 * j], b = v[2 * j + 1];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const bf16x2_t x = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+      const uint32_t u = __builtin_bit_cast(uint32_t, x);
+      w[p][j] = u;
+      a = __fsub_rn(a, __uint_as_float(u << 16));
+      b = __fsub_rn(b, __uint_as_float(u & 0xffff0000u));
+    }
+  }
+}
+
+__device__ __forceinline__ float halves_add(float x) {  // x of lanes l and l ^ 32
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+constexpr int kFewThreads = 256;
+constexpr int kFewCoords = 64;              // coordinates per workgroup
+constexpr int kFewMaxDim = 256;
+constexpr int kFewIdxRow = kFewCoords + 4;  // bytes per vector's indices in LDS
+
+// KS: 32-element steps that hold the dim (a multiple of 8)
+template <int KS, int XDT>
+__global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, AppendArgs va, int D, int kbits, int vbits,
+                                                                int n_vec) {
+  constexpr int NX = XDT == TQ_DTYPE_BF16 ? 1 : (XDT == TQ_DTYPE_F16 ? 2 : 3);
+  __shared__ __align__(16) uint8_t s_idx[16 * kFewIdxRow];
+  const bool key = blockIdx.z == 0;
+  const AppendArgs a = select_args(key, ka, va);
+  const int bits = key ? kbits : vbits;
+  const int nmid = (1 << bits) - 1;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15;
+  const int g = lane >> 4;
+
+  // ---- loads: this wave's rows of R (coordinates past D read the last row and
+  // are not stored), then the 16 vectors (past the end: the last one, not
+  // stored).  D % 8 == 0, so whole 8-element pieces lie inside D or past it.
+  const int s0 = blockIdx.y * kFewCoords;  // the workgroup's first coordinate
+  const int coord = s0 + 16 * wave + n;
+  float4 rv[KS][2];
+  {
+    const float* row = a.rot + static_cast<int64_t>(min(coord, D - 1)) * D;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int k = min(32 * s + 8 * g, D - 8);
+      rv[s][0] = *reinterpret_cast<const float4*>(row + k);
+      rv[s][1] = *reinterpret_cast<const float4*>(row + k + 4);
+    }
+  }
+  const int vec = min(static_cast<int>(blockIdx.x) * 16 + n, n_vec - 1);
+  const int l = vec % a.L;
+  const int bh = vec / a.L;
+  const int64_t xoff = static_cast<int64_t>(bh / a.H) * a.sb + static_cast<int64_t>(bh % a.H) * a.sh + l * a.sl;
+  const int64_t out_row = static_cast<int64_t>(bh) * a.cap + a.offset + l;
+  u32x4_t xr[KS][XDT == TQ_DTYPE_F32 ? 2 : 1];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int k = min(32 * s + 8 * g, D - 8);
+    if constexpr (XDT == TQ_DTYPE_F32) {
+      const u32x4_t* src = reinterpret_cast<const u32x4_t*>(static_cast<const float*>(a.x) + xoff + k);
+      xr[s][0] = src[0];
+      xr[s][1] = src[1];
+    } else {
+      xr[s][0] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.x) + xoff + k);
+    }
+  }
+  float mid[15];
+#pragma unroll
+  for (int m = 0; m < 15; ++m) mid[m] = a.mid[min(m, nmid - 1)];
+
+  // ---- pieces of x and the norm.  Lane (vector n, g) holds elements 32 s + 8 g
+  // + e: the tree's folds at 16 and 8 run across lanes 32 and 16 apart, those at
+  // 4, 2, 1 in registers, group sums pairwise.
+  u32x4_t xp[KS][NX];
+  float gs[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) gs[q] = 0.f;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    float v[8];
+    const bool in = 32 * s + 8 * g < D;
+#pragma unroll
+    for (int h = 0; h < (XDT == TQ_DTYPE_F32 ? 2 : 1); ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xr[s][h][e] = in ? xr[s][h][e] : 0u;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (XDT == TQ_DTYPE_F32) {
+        v[e] = __uint_as_float(xr[s][e >> 2][e & 3]);
+      } else {
+        const uint16_t u = static_cast<uint16_t>(xr[s][0][e >> 1] >> (16 * (e & 1)));
+        v[e] = XDT == TQ_DTYPE_F16 ? f16_bits_to_f32(u) : bf16_bits_to_f32(u);
+      }
+    }
+    if constexpr (XDT == TQ_DTYPE_BF16)
+      xp[s][0] = xr[s][0];
+    else
+      split8<NX>(v, xp[s]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float q = halves_add(__fmul_rn(v[e], v[e]));
+      q = __fadd_rn(q, xor_lane<16>(q));
+      v[e] = q;
+    }
+#pragma unroll
+    for (int w = 4; w >= 1; w >>= 1)
+#pragma unroll
+      for (int e = 0; e < w; ++e) v[e] = __fadd_rn(v[e], v[e + w]);
+    gs[s] = v[0];
+  }
+#pragma unroll
+  for (int w = 1; w < 8; w <<= 1)
+#pragma unroll
+    for (int q = 0; q < 8; q += 2 * w) gs[q] = __fadd_rn(gs[q], gs[q + w]);  // groups past the dim add exact zeros
+  const float nrm = sqrt_rn(gs[0]);
+  const float den = fmaxf(nrm, kNormEps);
+  if (blockIdx.y == 0 && wave == 0 && g == 0 && static_cast<int>(blockIdx.x) * 16 + n < n_vec) {
+    if (a.norm_dtype == TQ_DTYPE_F16)
+      static_cast<uint16_t*>(a.norms)[out_row] = f32_to_f16_bits(nrm);
+    else
+      static_cast<float*>(a.norms)[out_row] = nrm;
+  }
+  float dj[4];  // of result rows 4 g + j
+#pragma unroll
+  for (int j = 0; j < 4; ++j) dj[j] = __shfl(den, 4 * g + j, 64);
+
+  // ---- products and indices: lane (coordinate n, g) holds vectors 4 g + j
+  f32x4_t acc[3];  // one chain per piece of R
+#pragma unroll
+  for (int p = 0; p < 3; ++p) acc[p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const float4 r0 = rv[s][0], r1 = rv[s][1];
+    const float r[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+    u32x4_t w[3];
+    split8<3>(r, w);
+#pragma unroll
+    for (int p = 2; p >= 0; --p)
+#pragma unroll
+      for (int q = NX - 1; q >= 0; --q)
+        if (q + p <= 2) acc[p] = mfma_bf16(xp[s][q], w[p], acc[p]);
+  }
+  uint32_t idx[4] = {0u, 0u, 0u, 0u};
+  float y[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] = __fadd_rn(__fadd_rn(acc[2][j], acc[1][j]), acc[0][j]);
+#pragma unroll
+  for (int m = 0; m < 15; ++m) {
+    if (m >= nmid) break;  // uniform
+#pragma unroll
+    for (int j = 0; j < 4; ++j) idx[j] += y[j] > __fmul_rn(mid[m], dj[j]) ? 1u : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) s_idx[(4 * g + j) * kFewIdxRow + 16 * wave + n] = static_cast<uint8_t>(idx[j]);
+  __syncthreads();
+
+  // ---- pack: thread (vector, word); LSB-first, zeros past the last coordinate
+  const int pw = (D * bits + 31) / 32;
+  const int v = tid >> 4;
+  const int w = tid & 15;                     // word of the slice: 2 bits of them
+  const int pword = blockIdx.y * 2 * bits + w;
+  const int gv = static_cast<int>(blockIdx.x) * 16 + v;
+  if (w < 2 * bits && pword < pw && gv < n_vec) {
+    const uint8_t* row = s_idx + v * kFewIdxRow;
+    const int dl = D - s0;  // coordinates of the slice that exist
+    uint32_t word = 0;
+    if (bits == 3) {
+      const int ca = 32 * w / 3, cb = min(min(dl, kFewCoords) - 1, (32 * w + 31) / 3);
+      for (int c = ca; c <= cb; ++c) {
+        const int sh = 3 * c - 32 * w;  // negative for a field straddling the word's start
+        const uint32_t q = row[c];
+        word |= sh >= 0 ? q << sh : q >> -sh;
+      }
+    } else {
+      // 32 / bits coordinates per word, four bytes at a time
+      const int per = 32 / bits;
+      for (int c = 0; c < per; c += 4) {
+        if (per * w + c >= dl) break;
+        const uint32_t q = *reinterpret_cast<const uint32_t*>(row + per * w + c);
+        const uint32_t f = (q & 0xffu) | ((q >> 8 & 0xffu) << bits) | ((q >> 16 & 0xffu) << (2 * bits)) | ((q >> 24) << (3 * bits));
+        word |= f << (c * bits);
+      }
+    }
+    const int vl = gv % a.L;
+    const int vbh = gv / a.L;
+    a.packed[(static_cast<int64_t>(vbh) * a.cap + a.offset + vl) * pw + pword] = word;
+  }
+}
+
+template <int KS>
+int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
+               hipStream_t st) {
+  const int n_vec = k.B * k.H * k.L;
+  const dim3 grid(static_cast<unsigned>((n_vec + 15) / 16), static_cast<unsigned>((dim + kFewCoords - 1) / kFewCoords),
+                  static_cast<unsigned>(sides));
+  switch (x_dtype) {
+    case TQ_DTYPE_F32:
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F32>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
+      break;
+    case TQ_DTYPE_F16:
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
+      break;
+    default:
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_BF16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
+      break;
+  }
+  return check_launch("append_few_kernel");
+}
+
+}  // namespace
+
+// The line between this kernel and those that share a split of R among many
+// vectors, in workgroups (16 vectors x 64 coordinates x side).  K + V, 8 heads,
+// bf16, us before -> here.  Against one paired launch: d = 64 about equal
+// (4.1-5.0 -> 4.4-4.9), so it keeps that; d = 128 8.6 -> 5.4 at 16 workgroups,
+// 10.9 -> 7.5 at 512, 11.0 -> 11.1 at 1024; d = 256 8.9 -> 7.8 at 8, 12.0 -> 10.6
+// at 512, 12.2 -> 18.4 at 1024.  Against a launch a side (other width pairs):
+// d = 64 8.3 -> 4.7 at 2, 10.4 -> 8.3 at 1024; d = 128 18.2 -> 5.6 at 4; d = 256
+// 18.1 -> 8.1 at 8, 23.9 -> 18.1 at 1024, 24.2 -> 31.3 at 2048.  Against the
+// vector kernel (dims that are no 64, 128, 256): d = 96 26 -> 5.1 at 4, 33 -> 16
+// at 2048, d = 192 43 -> 6.1 at 6, 76 -> 33 at 3072: always.
+bool append_few_path(int64_t n_vec, int dim, int sides, bool paired) {
+  if (dim % 8 != 0 || dim < 8 || dim > kFewMaxDim || n_vec >= (int64_t(1) << 31) - 16) return false;
+  const int64_t wgs = (n_vec + 15) / 16 * ((dim + kFewCoords - 1) / kFewCoords) * sides;
+  if (dim != 64 && dim != 128 && dim != 256) return true;
+  return paired ? dim > 64 && wgs <= 512 : wgs <= 512 * sides;
+}
+
+int launch_append_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
+                      hipStream_t st) {
+  switch ((dim + 31) / 32) {
+    case 1:
+    case 2: return launch_few<2>(k, v, sides, dim, kbits, vbits, x_dtype, st);
+    case 3: return launch_few<3>(k, v, sides, dim, kbits, vbits, x_dtype, st);
+    case 4: return launch_few<4>(k, v, sides, dim, kbits, vbits, x_dtype, st);
+    case 5:
+    case 6: return launch_few<6>(k, v, sides, dim, kbits, vbits, x_dtype, st);
+    default: return launch_few<8>(k, v, sides, dim, kbits, vbits, x_dtype, st);
+  }
+}
+
+}  // namespace tq

@@ -1,0 +1,39 @@
+"""The dense-rotation append of few vectors (tq_append_few.hip), keys and values
+in one call: every dim class, width pair and input type, vector counts at the
+edges of its 16-vector groups.  Bar of test_append_general_gpu: norms bit-exact,
+indices equal to the oracle's but within its band of a midpoint (each y is a
+sum of exact piece products in f32, no longer than that band's d / 4 + 2 ulps),
+nothing written outside the appended rows."""
+import numpy as np
+import pytest
+import torch
+
+from kaplumba_amd import ops
+from tests.test_append_general_gpu import _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [8, 40, 64, 72, 96, 128, 160, 192, 248, 256])
+@pytest.mark.parametrize("kb,vb", [(3, 3), (4, 2), (1, 3), (2, 1)])
+@pytest.mark.parametrize("xdt,B,H,L", [("bf16", 1, 1, 1), ("f16", 2, 3, 5), ("f32", 1, 2, 8), ("bf16", 3, 1, 11)])
+def test_few_vectors_keys_and_values(device, d, kb, vb, xdt, B, H, L):
+    rng = np.random.default_rng(d + 10 * kb + L)
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[xdt]
+    # strided input: heads and tokens swapped, as a projection leaves them
+    xs = [torch.from_numpy(rng.standard_normal((B, L, H, d)).astype(np.float32)).to(dt).to(device).transpose(1, 2)
+          for _ in range(2)]
+    codecs = [ops.Codec(d, b, s, rotation="dense") for b, s in ((kb, 0), (vb, 1))]
+    cap, off = L + 6, 3
+    packed = [torch.full((B, H, cap, c.packed_width), 0x5a5a5a5a, dtype=torch.int32, device=device).view(torch.uint32)
+              for c in codecs]
+    norms = [torch.full((B, H, cap), -7.0, dtype=torch.float32, device=device) for _ in codecs]
+    ops.append_quantize_kv(xs[0], xs[1], codecs[0], codecs[1], packed[0], norms[0], packed[1], norms[1], off)
+    for x, c, p, n, b, s in zip(xs, codecs, packed, norms, (kb, vb), (0, 1)):
+        gp, gn = p.cpu().numpy().astype(np.uint32), n.cpu().numpy()
+        assert _check(x.float().cpu().numpy(), b, d, s, gp[:, :, off:off + L], gn[:, :, off:off + L]) <= 2
+        assert (np.delete(gp, np.s_[off:off + L], axis=2) == 0x5a5a5a5a).all()
+        assert (np.delete(gn, np.s_[off:off + L], axis=2) == -7.0).all()
+        used = d * b % 32
+        if used:  # bits past the last coordinate are zero
+            assert not (gp[:, :, off:off + L, -1] >> used).any()
