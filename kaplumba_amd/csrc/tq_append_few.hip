@@ -12,6 +12,13 @@
 // of one side.  Each of 4 waves owns 16 coordinates and splits their rows of R
 // straight into B fragments: no LDS, one round trip of loads; the norm is
 // formed by every wave.  Indices meet in LDS for the packing.
+//
+// Ties.  Sums in another order than the vector kernel's (tq_append_general.hip)
+// may put a coordinate within an ulp of a midpoint on its other side.  Where a
+// coordinate lies within a margin of a threshold that is above both
+// kernels' rounding, its index comes from the vector kernel's own arithmetic
+// (IEEE division, four fused chains), so the two agree bit for bit: one
+// coordinate in 10^4 or fewer, a branch that a wave takes now and then.
 #include "tq_append.h"
 
 namespace tq {
@@ -52,12 +59,16 @@ __device__ __forceinline__ float halves_add(float x) {  // x of lanes l and l ^ 
 constexpr int kFewThreads = 256;
 constexpr int kFewCoords = 64;              // coordinates per workgroup
 constexpr int kFewMaxDim = 256;
+// Margin of a tie in ulps of 1 per unit of |x| |R_i|: a margin of one already
+// gave the vector kernel's words over 65 million coordinates of 6 dims.
+constexpr float kTieUlps = 4;
+constexpr int kFewTunedVecs = 512;          // vectors a side at d = 64, 128, 256
 constexpr int kFewIdxRow = kFewCoords + 4;  // bytes per vector's indices in LDS
 
 // KS: 32-element steps that hold the dim (a multiple of 8)
 template <int KS, int XDT>
 __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, AppendArgs va, int D, int kbits, int vbits,
-                                                                int n_vec) {
+                                                                int n_vec, bool exact_ties) {
   constexpr int NX = XDT == TQ_DTYPE_BF16 ? 1 : (XDT == TQ_DTYPE_F16 ? 2 : 3);
   __shared__ __align__(16) uint8_t s_idx[16 * kFewIdxRow];
   const bool key = blockIdx.z == 0;
@@ -163,6 +174,7 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
   for (int j = 0; j < 4; ++j) dj[j] = __shfl(den, 4 * g + j, 64);
 
   // ---- products and indices: lane (coordinate n, g) holds vectors 4 g + j
+  float r2 = 0.f;  // squared length of this lane's row of R
   f32x4_t acc[3];  // one chain per piece of R
 #pragma unroll
   for (int p = 0; p < 3; ++p) acc[p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -170,6 +182,8 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
   for (int s = 0; s < KS; ++s) {
     const float4 r0 = rv[s][0], r1 = rv[s][1];
     const float r[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r2 = __builtin_fmaf(r[e], r[e], r2);
     u32x4_t w[3];
     split8<3>(r, w);
 #pragma unroll
@@ -178,15 +192,73 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
       for (int q = NX - 1; q >= 0; --q)
         if (q + p <= 2) acc[p] = mfma_bf16(xp[s][q], w[p], acc[p]);
   }
+  // |x . R_i| sums to at most |x| |R_i|; clamped tail pieces only add to r2
+  r2 += xor_lane<16>(r2);
+  r2 = halves_add(r2);
+  const float margin = kTieUlps * 0x1p-24f * __builtin_amdgcn_sqrtf(r2);
   uint32_t idx[4] = {0u, 0u, 0u, 0u};
   float y[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) y[j] = __fadd_rn(__fadd_rn(acc[2][j], acc[1][j]), acc[0][j]);
+  bool tie[4] = {false, false, false, false};
 #pragma unroll
   for (int m = 0; m < 15; ++m) {
     if (m >= nmid) break;  // uniform
 #pragma unroll
-    for (int j = 0; j < 4; ++j) idx[j] += y[j] > __fmul_rn(mid[m], dj[j]) ? 1u : 0u;
+    for (int j = 0; j < 4; ++j) {
+      const float d = y[j] - __fmul_rn(mid[m], dj[j]);
+      idx[j] += d > 0.f ? 1u : 0u;
+      tie[j] |= fabsf(d) <= margin * dj[j];
+    }
+  }
+  if (exact_ties && __any(tie[0] | tie[1] | tie[2] | tie[3])) {
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j) {
+      const bool mine = j == 0 ? tie[0] : j == 1 ? tie[1] : j == 2 ? tie[2] : tie[3];
+      if (!__any(mine)) continue;
+      const int tv = min(static_cast<int>(blockIdx.x) * 16 + 4 * g + j, n_vec - 1);
+      const int tl = tv % a.L;
+      const int tbh = tv / a.L;
+      const int64_t tx = static_cast<int64_t>(tbh / a.H) * a.sb + static_cast<int64_t>(tbh % a.H) * a.sh + tl * a.sl;
+      const float* row = a.rot + static_cast<int64_t>(min(coord, D - 1)) * D;
+      const float td = j == 0 ? dj[0] : j == 1 ? dj[1] : j == 2 ? dj[2] : dj[3];
+      float c[4] = {0.f, 0.f, 0.f, 0.f};
+      // 32 elements at a time, in whole 8-element pieces (those past D add u = 0)
+#pragma unroll 1
+      for (int k0 = 0; k0 < D; k0 += 32) {
+        float u[32], r[32];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int k = min(k0 + 8 * q, D - 8);
+          *reinterpret_cast<float4*>(r + 8 * q) = *reinterpret_cast<const float4*>(row + k);
+          *reinterpret_cast<float4*>(r + 8 * q + 4) = *reinterpret_cast<const float4*>(row + k + 4);
+          if constexpr (XDT == TQ_DTYPE_F32) {
+            const float* xs = static_cast<const float*>(a.x) + tx + k;
+            *reinterpret_cast<float4*>(u + 8 * q) = *reinterpret_cast<const float4*>(xs);
+            *reinterpret_cast<float4*>(u + 8 * q + 4) = *reinterpret_cast<const float4*>(xs + 4);
+          } else {
+            const uint4 h = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.x) + tx + k);
+            const uint32_t w[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const uint16_t b16 = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
+              u[8 * q + e] = XDT == TQ_DTYPE_F16 ? f16_bits_to_f32(b16) : bf16_bits_to_f32(b16);
+            }
+          }
+        }
+        div_by_norm<XDT>(u, td, u);
+#pragma unroll
+        for (int e = 0; e < 32; ++e)
+          if (k0 + (e & ~7) < D) c[e & 3] = __builtin_fmaf(u[e], r[e], c[e & 3]);
+      }
+      const float ty = __fadd_rn(__fadd_rn(c[0], c[1]), __fadd_rn(c[2], c[3]));
+      uint32_t ti = 0;
+#pragma unroll
+      for (int m = 0; m < 15; ++m)
+        if (m < nmid) ti += ty > mid[m] ? 1u : 0u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) idx[q] = (q == j && mine) ? ti : idx[q];
+    }
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) s_idx[(4 * g + j) * kFewIdxRow + 16 * wave + n] = static_cast<uint8_t>(idx[j]);
@@ -229,17 +301,18 @@ template <int KS>
 int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
                hipStream_t st) {
   const int n_vec = k.B * k.H * k.L;
+  const bool ties = dim != 64 && dim != 128 && dim != 256;  // the dims of the vector kernel
   const dim3 grid(static_cast<unsigned>((n_vec + 15) / 16), static_cast<unsigned>((dim + kFewCoords - 1) / kFewCoords),
                   static_cast<unsigned>(sides));
   switch (x_dtype) {
     case TQ_DTYPE_F32:
-      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F32>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F32>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec, ties);
       break;
     case TQ_DTYPE_F16:
-      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec, ties);
       break;
     default:
-      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_BF16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_BF16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec, ties);
       break;
   }
   return check_launch("append_few_kernel");
@@ -250,18 +323,19 @@ int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int
 // The line between this kernel and those that share a split of R among many
 // vectors, in workgroups (16 vectors x 64 coordinates x side).  K + V, 8 heads,
 // bf16, us before -> here.  Against one paired launch: d = 64 about equal
-// (4.1-5.0 -> 4.4-4.9), so it keeps that; d = 128 8.6 -> 5.4 at 16 workgroups,
-// 10.9 -> 7.5 at 512, 11.0 -> 11.1 at 1024; d = 256 8.9 -> 7.8 at 8, 12.0 -> 10.6
-// at 512, 12.2 -> 18.4 at 1024.  Against a launch a side (other width pairs):
-// d = 64 8.3 -> 4.7 at 2, 10.4 -> 8.3 at 1024; d = 128 18.2 -> 5.6 at 4; d = 256
-// 18.1 -> 8.1 at 8, 23.9 -> 18.1 at 1024, 24.2 -> 31.3 at 2048.  Against the
-// vector kernel (dims that are no 64, 128, 256): d = 96 26 -> 5.1 at 4, 33 -> 16
-// at 2048, d = 192 43 -> 6.1 at 6, 76 -> 33 at 3072: always.
+// (4.1-5.0 -> 4.4-4.9), so it keeps that; d = 128 8.6 -> 5.6 at 16 workgroups,
+// 10.8 -> 6.0 at 128; d = 256 8.9 -> 7.8 at 8, 11.8 -> 8.6 at 256.  Against a
+// launch a side (other width pairs): d = 64 8.4 -> 5.2 at 2, 10.2 -> 5.4 at 64;
+// d = 128 18.2 -> 6.0 at 4; d = 256 18 -> 8.2 at 8, 23.5 -> 9.0 at 256.  Against
+// the vector kernel (dims that are no 64, 128, 256), ties included: d = 96 26 ->
+// 5.2 at 4, 33 -> 21 at 2048, d = 192 43 -> 6.7 at 6, 77 -> 42 at 3072: always.
 bool append_few_path(int64_t n_vec, int dim, int sides, bool paired) {
   if (dim % 8 != 0 || dim < 8 || dim > kFewMaxDim || n_vec >= (int64_t(1) << 31) - 16) return false;
   const int64_t wgs = (n_vec + 15) / 16 * ((dim + kFewCoords - 1) / kFewCoords) * sides;
   if (dim != 64 && dim != 128 && dim != 256) return true;
-  return paired ? dim > 64 && wgs <= 512 : wgs <= 512 * sides;
+  // the matrix-core kernels round their sums in their own order, so their ties
+  // fall otherwise than here: up to a verify step's vectors only
+  return n_vec <= kFewTunedVecs && (paired ? dim > 64 && wgs <= 512 : wgs <= 512 * sides);
 }
 
 int launch_append_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
