@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "tq_append.h"
+#include "tq_rotate.h"
 
 namespace tq {
 
@@ -443,39 +444,96 @@ struct DequantArgs {
   float* out;
 };
 
-// One block per vector; D threads (64..256).  Test/API path, not hot.
-__global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
-  __shared__ float y[256];
-  const int64_t vec = blockIdx.x;  // (b*H + h)*T + t
-  const int t = static_cast<int>(vec % a.T);
-  const int64_t bh = vec / a.T;
-  const int64_t row = bh * a.cap + t;
-  const int i = threadIdx.x;
-  const uint32_t* w = a.packed + row * a.PW;
-  const int pos = i * a.bits;
-  uint32_t idx = w[pos >> 5] >> (pos & 31);
-  if ((pos & 31) + a.bits > 32) idx |= w[(pos >> 5) + 1] << (32 - (pos & 31));
-  idx &= (1u << a.bits) - 1u;
-  y[i] = a.cb[idx];
-  __syncthreads();
-  float r;
-  if (a.rot_kind == TQ_ROT_HADAMARD) {
-    for (int hstep = 1; hstep < a.D; hstep <<= 1) {
-      float mine = y[i];
-      float other = y[i ^ hstep];
-      __syncthreads();
-      y[i] = (i & hstep) ? __fsub_rn(other, mine) : __fadd_rn(mine, other);
-      __syncthreads();
-    }
-    r = __fmul_rn(__fmul_rn(y[i], a.scale), a.rot[i]);
-  } else {
-    // x = y @ R : x[i] = sum_j y[j] R[j][i]
-    float acc = 0.f;
-    for (int j = 0; j < a.D; ++j) acc = fmaf(y[j], a.rot[static_cast<int64_t>(j) * a.D + i], acc);
-    r = acc;
+// Hadamard rotation, D = 4 LV coordinates: LV lanes per vector, four coordinates
+// each, UN vectors per lane with every load issued first (4, or 1 while the
+// vectors do not fill the chip).  Butterflies at
+// distances 1 and 2 in registers, then across lanes, in ascending order (the
+// sums of _rht_inverse, turboquant_cache.py:3564-3575).  Bound by the f32
+// output: 16-byte stores, a vector's row contiguous.  K of 8 x 4096 vectors of
+// 128: one thread per coordinate with barriers between the stages took 18 us,
+// this 7.5 (17 MB written).
+constexpr int kDqThreads = 256;
+template <int LV, int UN, typename I>
+__global__ __launch_bounds__(kDqThreads) void dequant_rht_kernel(DequantArgs a, I n_vec) {
+  constexpr int VPB = kDqThreads / LV;
+  __shared__ float s_cb[16];
+  const int tid = threadIdx.x;
+  const int lane = tid % LV;
+  const I v0 = static_cast<I>(blockIdx.x) * (VPB * UN) + tid / LV;
+  const int bit = 4 * lane * a.bits;
+  const int w0 = bit >> 5;
+  const int w1 = min(w0 + 1, a.PW - 1);
+  uint32_t lo[UN], hi[UN];
+  float nrm[UN];
+#pragma unroll
+  for (int u = 0; u < UN; ++u) {
+    const I vec = min(v0 + u * VPB, n_vec - 1);
+    const I bh = vec / static_cast<I>(a.T);
+    const int64_t row = static_cast<int64_t>(bh) * a.cap + (vec - bh * static_cast<I>(a.T));
+    lo[u] = a.packed[row * a.PW + w0];
+    hi[u] = a.packed[row * a.PW + w1];
+    nrm[u] = load_norm(a.norms, a.norm_dtype, row);
   }
-  const float nrm = load_norm(a.norms, a.norm_dtype, row);
-  a.out[vec * a.D + i] = nrm * r;
+  const float4 sg = reinterpret_cast<const float4*>(a.rot)[lane];
+  if (tid < (1 << a.bits)) s_cb[tid] = a.cb[tid];
+  __syncthreads();
+  const uint32_t mask = (1u << a.bits) - 1u;
+#pragma unroll
+  for (int u = 0; u < UN; ++u) {
+    const uint32_t x = __builtin_amdgcn_alignbit(hi[u], lo[u], bit & 31);
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = s_cb[(x >> (e * a.bits)) & mask];
+    const float a0 = __fadd_rn(y[0], y[1]), a1 = __fsub_rn(y[0], y[1]);
+    const float a2 = __fadd_rn(y[2], y[3]), a3 = __fsub_rn(y[2], y[3]);
+    y[0] = __fadd_rn(a0, a2);
+    y[2] = __fsub_rn(a0, a2);
+    y[1] = __fadd_rn(a1, a3);
+    y[3] = __fsub_rn(a1, a3);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = y[e];
+#define TQ_DQ_STAGE(HB)                                             \
+  if constexpr (LV > HB) {                                          \
+    const float o = xor_lane<HB>(v);                                \
+    v = (lane & HB) ? __fsub_rn(o, v) : __fadd_rn(v, o);            \
+  }
+      TQ_DQ_STAGE(1)
+      TQ_DQ_STAGE(2)
+      TQ_DQ_STAGE(4)
+      TQ_DQ_STAGE(8)
+      TQ_DQ_STAGE(16)
+#undef TQ_DQ_STAGE
+      if constexpr (LV > 32) {
+        const float o = __shfl_xor(v, 32, 64);
+        v = (lane & 32) ? __fsub_rn(o, v) : __fadd_rn(v, o);
+      }
+      y[e] = __fmul_rn(v, a.scale);
+    }
+    const I vec = v0 + u * VPB;
+    if (vec < n_vec)
+      reinterpret_cast<float4*>(a.out)[static_cast<int64_t>(vec) * LV + lane] =
+          make_float4(nrm[u] * __fmul_rn(y[0], sg.x), nrm[u] * __fmul_rn(y[1], sg.y), nrm[u] * __fmul_rn(y[2], sg.z),
+                      nrm[u] * __fmul_rn(y[3], sg.w));
+  }
+}
+
+template <int LV, int UN>
+int launch_dequant_rht_un(const DequantArgs& a, int64_t n, hipStream_t st) {
+  constexpr int per = kDqThreads / LV * UN;
+  const dim3 grid(static_cast<unsigned>((n + per - 1) / per));
+  if (n < (int64_t(1) << 31) - per)
+    hipLaunchKernelGGL((dequant_rht_kernel<LV, UN, int>), grid, dim3(kDqThreads), 0, st, a, static_cast<int>(n));
+  else
+    hipLaunchKernelGGL((dequant_rht_kernel<LV, UN, int64_t>), grid, dim3(kDqThreads), 0, st, a, n);
+  return check_launch("dequant_rht_kernel");
+}
+
+template <int LV>
+int launch_dequant_rht(const DequantArgs& a, int64_t n, hipStream_t st) {
+  // four vectors per lane once that still leaves four workgroups to a CU
+  if (n >= static_cast<int64_t>(16) * device_cu_count() * (kDqThreads / LV)) return launch_dequant_rht_un<LV, 4>(a, n, st);
+  return launch_dequant_rht_un<LV, 1>(a, n, st);
 }
 
 }  // namespace tq
@@ -705,16 +763,23 @@ extern "C" int tq_dequantize(const uint32_t* packed, const void* norms, int norm
   if (n == 0) return TQ_OK;
   if (!packed || !norms || !codebook || !rot || !out)
     return fail(TQ_ERR_INVALID_ARGUMENT, "dequantize: null pointer");
-  if (dim < 32 || dim > 256 || (dim & (dim - 1))) {
-    const DequantGeneralArgs g{packed, norms, norm_dtype, B, H, T, dim, bits,
-                               tq_packed_width(dim, bits), capacity, codebook, rot_kind, rot,
-                               static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(dim))), out};
-    return launch_dequant_general(g, n, static_cast<hipStream_t>(stream));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int pw = tq_packed_width(dim, bits);
+  const float scale = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(dim)));
+  if (rot_kind == TQ_ROT_HADAMARD && dim >= 32 && dim <= 256 && aligned16(rot) && aligned16(out)) {
+    const DequantArgs a{packed, norms, norm_dtype, B, H, T, dim, bits, pw, capacity, codebook, rot_kind, rot, scale, out};
+    switch (dim) {
+      case 32: return launch_dequant_rht<8>(a, n, st);
+      case 64: return launch_dequant_rht<16>(a, n, st);
+      case 128: return launch_dequant_rht<32>(a, n, st);
+      default: return launch_dequant_rht<64>(a, n, st);
+    }
   }
-  DequantArgs a{packed, norms, norm_dtype, B, H, T, dim, bits, tq_packed_width(dim, bits),
-                capacity, codebook, rot_kind, rot,
-                static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(dim))), out};
-  hipLaunchKernelGGL(dequant_kernel, dim3(static_cast<unsigned>(n)), dim3(dim), 0,
-                     static_cast<hipStream_t>(stream), a);
-  return check_launch("dequant_kernel");
+  const DequantGeneralArgs g{packed, norms, norm_dtype, B, H, T, dim, bits, pw, capacity, codebook, rot_kind, rot, scale, out};
+  // the matrix-core kernel shares a split of R among 128 vectors (us of one
+  // workgroup per vector -> this: 1024 vectors d = 128 6.2 -> 6.8, d = 256 11.5 ->
+  // 10.1; 2048 7.1 -> 6.9 and 22.9 -> 10.5; 32768 76 -> 11.8 and 264 -> 36)
+  if (rot_kind == TQ_ROT_DENSE && dim <= kRotateMaxDim && n >= kDequantDenseMin && n < (int64_t(1) << 31) - 128)
+    return launch_dequant_dense(g, static_cast<int>(n), st);
+  return launch_dequant_general(g, n, st);
 }

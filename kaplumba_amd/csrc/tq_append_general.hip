@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void dequant_general_kernel(DequantGeneralArgs
   const int64_t row = bh * a.cap + t;
   const int D = a.D;
   const uint32_t* w = a.packed + row * a.PW;
-  for (int d = threadIdx.x; d < D; d += 256) {
+  for (int d = threadIdx.x; d < D; d += blockDim.x) {
     const int bit = d * a.bits;
     const int wi = bit >> 5;
     const int sh = bit & 31;
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void dequant_general_kernel(DequantGeneralArgs
   float* out = a.out + vec * D;
   if (a.rot_kind == TQ_ROT_HADAMARD) {
     for (int hs = 1; hs < D; hs <<= 1) {
-      for (int k = threadIdx.x; k < D / 2; k += 256) {
+      for (int k = threadIdx.x; k < D / 2; k += blockDim.x) {
         const int i0 = (k / hs) * 2 * hs + (k % hs);
         const float p = s_y[i0];
         const float q = s_y[i0 + hs];
@@ -270,10 +270,10 @@ __global__ __launch_bounds__(256) void dequant_general_kernel(DequantGeneralArgs
       }
       __syncthreads();
     }
-    for (int d = threadIdx.x; d < D; d += 256) out[d] = n * (s_y[d] * a.scale * a.rot[d]);
+    for (int d = threadIdx.x; d < D; d += blockDim.x) out[d] = n * (s_y[d] * a.scale * a.rot[d]);
     return;
   }
-  for (int j = threadIdx.x; j < D; j += 256) {
+  for (int j = threadIdx.x; j < D; j += blockDim.x) {
     float acc = 0.f;
     for (int d = 0; d < D; ++d) acc = __builtin_fmaf(s_y[d], a.rot[static_cast<int64_t>(d) * D + j], acc);
     out[j] = n * acc;
@@ -335,7 +335,8 @@ int launch_prod_residual_dense(const AppendArgs& a, int dim, int mb, int x_dtype
 }
 
 int launch_dequant_general(const DequantGeneralArgs& a, int64_t n_vec, hipStream_t st) {
-  hipLaunchKernelGGL(dequant_general_kernel, dim3(static_cast<unsigned>(n_vec)), dim3(256), 0, st, a);
+  const unsigned threads = a.D > 192 ? 256u : static_cast<unsigned>((a.D + 63) / 64 * 64);  // a coordinate each
+  hipLaunchKernelGGL(dequant_general_kernel, dim3(static_cast<unsigned>(n_vec)), dim3(threads), 0, st, a);
   return check_launch("dequant_general_kernel");
 }
 

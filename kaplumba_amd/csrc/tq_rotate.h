@@ -1,6 +1,7 @@
 // Dense rotations of many f32 or query rows on the matrix cores.
 #pragma once
 
+#include "tq_append.h"
 #include "tq_common.h"
 
 namespace tq {
@@ -27,5 +28,9 @@ constexpr int kRotateMaxDim = 256;
 int launch_rotate_queries(const RotateArgs& a, hipStream_t st);
 // out = x @ mat for f32 rows x (k = n <= 256, a multiple of 4, rows and x 16-byte aligned)
 int launch_rotate_rows(const RotateArgs& a, hipStream_t st);
+
+// out[vec] = norm * (codebook[idx] @ R) for n packed vectors of any dim up to 256
+constexpr int kDequantDenseMin = 2048;
+int launch_dequant_dense(const DequantGeneralArgs& a, int n, hipStream_t st);
 
 }  // namespace tq

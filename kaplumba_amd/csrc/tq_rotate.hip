@@ -13,6 +13,8 @@
 // rotate_few_kernel: for few rows a workgroup takes 16 rows and 64 columns, a
 // wave one 16-column tile whose pieces it splits straight into registers: no
 // LDS, one round trip of loads.  Latency-bound.
+#include <algorithm>
+
 #include "tq_rotate.h"
 
 namespace tq {
@@ -297,7 +299,132 @@ int launch_any(const RotateArgs& a, hipStream_t st) {
   }
 }
 
+// Dequantize with the dense rotation: rotate_kernel's products with the rows
+// decoded from packed indices (the three pieces of every codebook level in an
+// LDS table), scaled by the vector's norm.  A workgroup walks 128-vector tiles
+// with one split of its 64 columns of R.
+template <int KS>
+__global__ __launch_bounds__(512) void dequant_dense_kernel(DequantGeneralArgs a, int n_vec) {
+  __shared__ u32x4_t s_m[3 * 4 * KS * 64];  // [piece][16-column tile][k step][lane]
+  __shared__ uint2 s_cb[16];                // pieces 0 | 1 << 16, 2 of a level
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int n = lane & 15;
+  const int g = lane >> 4;
+  const int c0 = blockIdx.y * 64;
+  const int D = a.D;
+  RotateArgs ra{};
+  ra.k = ra.n = D;
+  ra.mat = a.rot;
+  constexpr int FR = 4 * KS * 64;
+  constexpr int FPT = (FR + 511) / 512;
+  float m[FPT][8];
+#pragma unroll
+  for (int i = 0; i < FPT; ++i) {
+    const int f = min(tid + 512 * i, FR - 1);
+    fragment_load<false, true>(ra, c0 + 16 * (f / (64 * KS)) + (f & 15), 32 * ((f >> 6) % KS) + 8 * ((f >> 4) & 3), m[i]);
+  }
+  if (tid < (1 << a.bits)) {
+    float v[8] = {a.cb[tid], 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    u32x4_t w[3];
+    split8<3>(v, w);
+    s_cb[tid] = make_uint2((w[0][0] & 0xffffu) | (w[1][0] << 16), w[2][0] & 0xffffu);
+  }
+#pragma unroll
+  for (int i = 0; i < FPT; ++i) {
+    const int f = tid + 512 * i;
+    if (FR % 512 != 0 && f >= FR) break;  // whole waves
+    fragment_zero(ra, c0 + 16 * (f / (64 * KS)) + (f & 15), 32 * ((f >> 6) % KS) + 8 * ((f >> 4) & 3), m[i]);
+    u32x4_t w[3];
+    split8<3>(m[i], w);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) s_m[p * FR + f] = w[p];
+  }
+  __syncthreads();
+  const int bits = a.bits;
+  const int sh = (8 * g * bits) & 31;
+  const uint32_t mask = (1u << bits) - 1u;
+#pragma unroll 1
+  for (int r0 = blockIdx.x * kRotateRows + 16 * (tid >> 6); r0 < n_vec; r0 += gridDim.x * kRotateRows) {
+    // the fragments stay in LDS: hoisted out of the loop they spill
+    asm volatile("" ::: "memory");
+    // lane (vector n, g): coordinates 32 s + 8 g .. + 7, 8 * bits bits from word
+    // s * bits + (8 g bits) / 32 on; words past the row's last are not read
+    // (their coordinates meet zero rows of R)
+    const int vec = min(r0 + n, n_vec - 1);
+    const int bh = vec / a.T;
+    const uint32_t* row = a.packed + (static_cast<int64_t>(bh) * a.cap + (vec - bh * a.T)) * a.PW;
+    uint32_t x[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int w = s * bits + ((8 * g * bits) >> 5);
+      x[s] = __builtin_amdgcn_alignbit(row[min(w + 1, a.PW - 1)], row[min(w, a.PW - 1)], sh);
+    }
+    float nrm[4];
+    int vj[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      vj[j] = r0 + 4 * g + j;
+      const int v = min(vj[j], n_vec - 1);
+      const int vbh = v / a.T;
+      nrm[j] = load_norm(a.norms, a.norm_dtype, static_cast<int64_t>(vbh) * a.cap + (v - vbh * a.T));
+    }
+    f32x4_t acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      u32x4_t xp[3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint2 u = s_cb[(x[s] >> (2 * e * bits)) & mask];
+        const uint2 v = s_cb[(x[s] >> ((2 * e + 1) * bits)) & mask];
+        xp[0][e] = __builtin_amdgcn_perm(v.x, u.x, 0x05040100u);
+        xp[1][e] = __builtin_amdgcn_perm(v.x, u.x, 0x07060302u);
+        xp[2][e] = __builtin_amdgcn_perm(v.y, u.y, 0x05040100u);
+      }
+#pragma unroll
+      for (int mp = 2; mp >= 0; --mp)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const u32x4_t b = s_m[mp * FR + (t * KS + s) * 64 + lane];
+#pragma unroll
+          for (int q = 2; q >= 0; --q)
+            if (q + mp <= 2) acc[t] = mfma_bf16(xp[q], b, acc[t]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int col = c0 + 16 * t + n;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (vj[j] < n_vec && col < D) a.out[static_cast<int64_t>(vj[j]) * D + col] = nrm[j] * acc[t][j];
+    }
+  }
+}
+
+template <int KS>
+int launch_dequant_ks(const DequantGeneralArgs& a, int n, hipStream_t st) {
+  const int gy = (a.D + 63) / 64;
+  const int tiles = (n + kRotateRows - 1) / kRotateRows;
+  const int gx = std::min(tiles, std::max(1, 2 * device_cu_count() / gy));
+  hipLaunchKernelGGL(dequant_dense_kernel<KS>, dim3(static_cast<unsigned>(gx), static_cast<unsigned>(gy)), dim3(512), 0, st, a, n);
+  return check_launch("dequant_dense_kernel");
+}
+
 }  // namespace
+
+int launch_dequant_dense(const DequantGeneralArgs& a, int n, hipStream_t st) {
+  switch ((a.D + 31) / 32) {
+    case 1:
+    case 2: return launch_dequant_ks<2>(a, n, st);
+    case 3: return launch_dequant_ks<3>(a, n, st);
+    case 4: return launch_dequant_ks<4>(a, n, st);
+    case 5:
+    case 6: return launch_dequant_ks<6>(a, n, st);
+    default: return launch_dequant_ks<8>(a, n, st);
+  }
+}
 
 int launch_rotate_queries(const RotateArgs& a, hipStream_t st) {
   switch (a.x_dtype) {
