@@ -661,6 +661,9 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
       for (int j = 0; j < 8; ++j) {
         l_acc[rt] += pe[rt][j];
         w[j] = (PACKED || kWExp != 0) ? pe[rt][j] * vs[j] : pe[rt][j];
+        // in a register of its own: the product folded into the f16 conversion
+        // rounds once, and the low part would belong to another high part
+        if constexpr (WP > 1) w[j] = own_reg(w[j]);
       }
 #pragma unroll
       for (int q = 0; q < WP; ++q) {
