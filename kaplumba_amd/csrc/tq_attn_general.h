@@ -165,5 +165,8 @@ bool wide_call(const GenCall& c);
 int launch_wide_packed(const GenParams& p, bool f32_weights, hipStream_t st);
 int launch_wide_f16(const GenParams& p, bool f32_weights, hipStream_t st);
 int launch_wide_bf16(const GenParams& p, bool f32_weights, hipStream_t st);
+int launch_narrow_packed(const GenParams& p, hipStream_t st);
+int launch_narrow_f16(const GenParams& p, hipStream_t st);
+int launch_narrow_bf16(const GenParams& p, hipStream_t st);
 
 }  // namespace tq

@@ -6,6 +6,7 @@
 #include "tq_attn_general.h"
 #include "tq_attn_merge.h"
 #include "tq_attn_tile.h"
+#include "tq_attn_narrow.h"
 #include "tq_attn_wide_prep.h"
 #include "tq_rotate.h"
 
@@ -806,6 +807,8 @@ GenPlan tile_plan(int B, int Hq, int Hkv, int L, int64_t T) {
 // the partials' way through memory (written, then read by the merge, at about
 // 4 TB/s).  Microseconds per token measured on the prefill shapes.
 constexpr int kWideMaxSplits = 32;
+constexpr int kNarrowMaxSplits = 64;
+constexpr double kNarrowTokenUs = 2.5e-5;  // per token and padded dim of one workgroup
 
 GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   GenPlan gp{};
@@ -831,6 +834,34 @@ GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   }
   gp.n_splits = static_cast<int>(best);
   gp.chunk = 0;  // each block splits the tokens its rows see (in the kernel)
+  return gp;
+}
+
+// The narrow kernel's plan: 16-row groups, splits with the least estimated time
+// (see wide_plan; a workgroup's 8 waves take 256 tokens at a time).
+GenPlan narrow_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
+  GenPlan gp{};
+  int ks = 0, ct = 0;
+  wide_dims(Dk, Dv, ks, ct);
+  const int64_t rows = static_cast<int64_t>(Hq / Hkv) * L;
+  gp.n_rg = static_cast<int>((rows + kGenNQ - 1) / kGenNQ);
+  const int64_t blocks = static_cast<int64_t>(B) * Hkv * ((rows + kNarrowRows - 1) / kNarrowRows);
+  const int64_t cus = device_cu_count();
+  const double token_us = (32 * ks + 16 * ct) * kNarrowTokenUs;
+  const double merge_us = static_cast<double>(B) * Hq * L * Dv * 8 / 4e6;  // per split
+  int64_t best = 1;
+  double best_cost = 0;
+  for (int64_t ns = 1; ns <= kNarrowMaxSplits && (ns == 1 || (T + ns - 1) / ns >= 128); ++ns) {
+    const double cost =
+        static_cast<double>((blocks * ns + cus - 1) / cus) * (static_cast<double>((T + ns - 1) / ns) * token_us + 6) +
+        static_cast<double>(ns) * merge_us;
+    if (ns == 1 || cost < best_cost) {
+      best = ns;
+      best_cost = cost;
+    }
+  }
+  gp.n_splits = static_cast<int>(best);
+  gp.chunk = 0;
   return gp;
 }
 
@@ -862,7 +893,7 @@ bool wide_had_queries(int Dk, int rot_kind) {
 // Prepares the queries (and mask ranges) and runs the wide kernel over p,
 // whose workspace pointers follow wide_layout; general: the weights were f32
 // in the vector kernel.
-int run_wide(GenParams& p, int64_t rows, bool plain, hipStream_t st) {
+int run_wide(GenParams& p, int64_t rows, bool plain, bool narrow, hipStream_t st) {
   int ks = 0, ct = 0;
   wide_dims(p.Dk, p.Dv, ks, ct);
   const dim3 qgrid(static_cast<unsigned>((rows + kWideQpThreads / 16 - 1) / (kWideQpThreads / 16)));
@@ -875,7 +906,8 @@ int run_wide(GenParams& p, int64_t rows, bool plain, hipStream_t st) {
     p.q_rows32 = 1;  // f32 rows already in p.qrot
   int rc = check_launch("wide_qprep_kernel");
   if (rc) return rc;
-  if (p.mask_kind != TQ_MASK_NONE && !p.causal) {
+  // (few rows over few tokens: the range kernel costs more than it saves)
+  if (p.mask_kind != TQ_MASK_NONE && !p.causal && (!narrow || p.T >= 1024)) {
     // one range per distinct mask row: axes the mask is broadcast along share
     // theirs (per-sequence windows keep the batch axis)
     const bool bb = p.B > 1 && (p.m_sb != 0 || p.seq_lens || p.seq_starts);
@@ -890,6 +922,10 @@ int run_wide(GenParams& p, int64_t rows, bool plain, hipStream_t st) {
     if (rc) return rc;
   } else {
     p.mrange = nullptr;
+  }
+  if (narrow) {
+    if (!plain) return launch_narrow_packed(p, st);
+    return p.key_kind == kGenPlainBf16 ? launch_narrow_bf16(p, st) : launch_narrow_f16(p, st);
   }
   // the vector kernel's f32 weights: array masks and the dims it alone served
   const bool pow2dim = p.Dk == p.Dv && (p.Dk == 64 || p.Dk == 128 || p.Dk == 256);
@@ -1021,39 +1057,69 @@ bool wide_rows_path(int kv_kind, int Dk, int Dv, int rows) {
   return (kv_kind == TQ_KV_PACKED || kv_kind == TQ_KV_PLAIN) && rows >= kWideMinRows && wide_dims(Dk, Dv, ks, ct);
 }
 
-// Work from which the wide kernel is the faster one, in query row x token x
-// (Dk + Dv) products of 2^28 (its set-up, and the partials of the splits that
-// fill the chip, cost 10-15 us).  Measured crossovers against the kernel that
-// would run instead, 2 and 8 kv heads, 64-1024 rows each, 256-4352 tokens:
-// tuned kernels at d = 64: 0.85-1.0x up to 5, 1.15x at 17; plain d = 128:
-// 0.65-1.15x at 2, 1.15x from 4; d = 256: 0.76-1.0x at 0.3-1, 1.3x from 1.25;
-// vector kernel with dense queries 0.8x at 0.4, 1.0x at 0.75, 1.1x from 1.5;
-// its other calls (masks, plain caches of other dims) 1.05x and more from the
-// smallest on.
+// Shapes, types and alignment that the wide and narrow kernels take: packed
+// MSE caches, or plain ones in the queries' type with whole 16-byte rows.
+static bool mfma_operands(const GenCall& c) {
+  int ks = 0, ct = 0;
+  if (c.kv_kind != TQ_KV_PACKED && c.kv_kind != TQ_KV_PLAIN) return false;
+  if (!wide_dims(c.Dk, c.Dv, ks, ct)) return false;
+  if (c.capacity > INT32_MAX || static_cast<int64_t>(c.B) * c.Hq * c.L >= (int64_t(1) << 30)) return false;
+  return c.kv_kind == TQ_KV_PACKED ||
+         (c.q_dtype == c.kv_dtype && c.Dk % 8 == 0 && c.Dv % 8 == 0 &&
+          ((reinterpret_cast<uintptr_t>(c.k) | reinterpret_cast<uintptr_t>(c.v)) & 15u) == 0);
+}
+
+// Whether a plan fits the call's workspace and one launch of the merge.
+static bool mfma_fits(const GenCall& c, const GenPlan& gp) {
+  return static_cast<int64_t>(c.Hkv) * gp.n_rg <= 65535 && c.B <= 65535 &&
+         c.workspace_bytes >= wide_layout(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, gp, c.kv_kind == TQ_KV_PACKED,
+                                          c.mask_kind != TQ_MASK_NONE).bytes;
+}
+
+// Calls of the vector kernel that the narrow one takes instead.
+static bool narrow_call(const GenCall& c) {
+  const int64_t T = std::max<int64_t>(c.max_tokens, 1);
+  return mfma_operands(c) && mfma_fits(c, narrow_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T));
+}
+
+// Whether the wide kernel is the faster one, by work (query row x token x
+// (Dk + Dv) products of 2^28) and query rows of the whole call: its set-up and
+// the partials of the splits that fill the chip cost 10-15 us, and few rows
+// leave most of a block's products empty at every length.  Measured against
+// the kernel that would run instead, time there / time here, 144-16384 rows:
+//   tuned, d = 64 / 128 plain: 512 rows 0.4-0.9x up to 18, 1024 rows 0.7-1.2x up
+//     to 20; 1536 rows and more: 0.8-1.7x at 10-12, 0.98-2.1x at 18-20.
+//   tuned, d = 256: packed 0.85-1.2x at 1.3, 0.94-1.8x at 2, 1.02-1.6x at 2.5,
+//     1.36-4.4x from 5; plain 1.27-2.1x at 1.3, up to 11x at 20.
+//   others against the narrow kernel (it walks the cache once per 16 rows):
+//     packed Dv 256 (where the narrow kernel spills) 1.13-1.9x from 0.6; 192 /
+//     128: 0.71-1.18x at 256-512 rows, 0.93-1.3x from 1024; other dims 0.56-0.97x
+//     at 256-512 rows; from 1024 rows 0.8-1.2x at 4, 0.97-1.7x at 8, 1.02-1.9x at
+//     16-32.  Masks that keep every key 0.97-1.6x at 8, 1.07-2.2x at 16-32; a
+//     window of 300 keys 0.6-0.8x up to 4096 rows, 0.95-1.4x from 8192 at any work
+//     (its work is not known here, so masks of few rows wait until 16); plain
+//     Dv 256: 0.8-1.2x at 512 rows, 0.8-1.9x from 1024 rows and 2.
 bool wide_pays(const GenCall& c) {
-  const double work = static_cast<double>(c.B) * c.Hq * c.L * static_cast<double>(c.max_tokens) * (c.Dk + c.Dv) / (1 << 28);
+  const double rows = static_cast<double>(c.B) * c.Hq * c.L;
+  const double work = rows * static_cast<double>(c.max_tokens) * (c.Dk + c.Dv) / (1 << 28);
   const bool plain = c.kv_kind == TQ_KV_PLAIN;
-  const bool tuned = c.mask_kind == TQ_MASK_NONE && c.Dk == c.Dv && (plain || c.k_rot_kind == c.v_rot_kind);
-  if (tuned && c.Dk == 64) return work >= 6;
-  if (tuned && c.Dk == 128) return work >= 4;
-  if (tuned && c.Dk == 256) return work >= 1.25;
-  return plain || c.k_rot_kind == TQ_ROT_HADAMARD || work >= 1;
+  const bool masked = c.mask_kind != TQ_MASK_NONE;
+  const bool tuned = !masked && c.Dk == c.Dv && (plain || c.k_rot_kind == c.v_rot_kind);
+  if (tuned && (c.Dk == 64 || c.Dk == 128)) return rows >= 1536 && work >= 16;
+  if (tuned && c.Dk == 256) return work >= (plain ? 1.25 : 2.5);
+  if (c.Dv > 128 && !plain) return work >= 0.5;
+  if (rows < 1024) return false;
+  if (c.Dv > 128) return work >= 2;
+  if (c.Dk > 128) return work >= 1;
+  return work >= (masked ? (rows < 8192 ? 16 : 4) : 8);
 }
 
 bool wide_call(const GenCall& c) {
   const int rows = (c.Hq / c.Hkv) * c.L;
   if (!wide_rows_path(c.kv_kind, c.Dk, c.Dv, rows) || !wide_pays(c)) return false;
   if (c.mask_kind == TQ_MASK_NONE && tile_rows_path(c.kv_kind, c.Dk, c.Dv, rows)) return false;
-  if (c.capacity > INT32_MAX || static_cast<int64_t>(c.B) * c.Hq * c.L >= (int64_t(1) << 30)) return false;
-  if (c.kv_kind == TQ_KV_PLAIN &&
-      (c.q_dtype != c.kv_dtype || c.Dk % 8 || c.Dv % 8 ||
-       ((reinterpret_cast<uintptr_t>(c.k) | reinterpret_cast<uintptr_t>(c.v)) & 15u)))
-    return false;
   const int64_t T = std::max<int64_t>(c.max_tokens, 1);
-  const GenPlan gp = wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T);
-  return static_cast<int64_t>(c.Hkv) * gp.n_rg <= 65535 && c.B <= 65535 &&
-         c.workspace_bytes >= wide_layout(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, gp, c.kv_kind == TQ_KV_PACKED,
-                                          c.mask_kind != TQ_MASK_NONE).bytes;
+  return mfma_operands(c) && mfma_fits(c, wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T));
 }
 
 int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod,
@@ -1061,8 +1127,11 @@ int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, i
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || Dk <= 0 || Dv <= 0 || Hq % Hkv) return 0;
   T = std::max<int64_t>(T, 1);
   int64_t wide = 0;
+  int ks = 0, ct = 0;
+  if (!without_wide && wide_dims(Dk, Dv, ks, ct))
+    wide = wide_layout(B, Hq, Hkv, L, Dk, Dv, narrow_plan(B, Hq, Hkv, L, Dk, Dv, T), true, true).bytes;
   if (!without_wide && wide_rows_path(TQ_KV_PACKED, Dk, Dv, (Hq / Hkv) * L))
-    wide = wide_layout(B, Hq, Hkv, L, Dk, Dv, wide_plan(B, Hq, Hkv, L, Dk, Dv, T), true, true).bytes;
+    wide = std::max(wide, wide_layout(B, Hq, Hkv, L, Dk, Dv, wide_plan(B, Hq, Hkv, L, Dk, Dv, T), true, true).bytes);
   GenPlan gp = gen_plan(B, Hq, Hkv, L, T);
   const int64_t rows = static_cast<int64_t>(B) * Hq * L;
   int64_t tile_q = 0;  // the tile kernel's prepared query rows
@@ -1135,8 +1204,10 @@ int general_attention(const GenCall& c) {
   const bool tile = c.kv_kind == TQ_KV_PACKED && c.mask_kind == TQ_MASK_NONE &&
                     tile_rows_path(c.kv_kind, c.Dk, c.Dv, (c.Hq / c.Hkv) * c.L) &&
                     static_cast<int64_t>(c.B) * c.Hq * c.L < (int64_t(1) << 30);
-  const bool wide = wide_call(c);
-  const GenPlan gp = wide   ? wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T)
+  const bool narrow = !tile && !wide_call(c) && narrow_call(c);
+  const bool wide = narrow || wide_call(c);  // either matrix-core kernel: they share layout and preparation
+  const GenPlan gp = narrow ? narrow_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T)
+                     : wide ? wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T)
                      : tile ? tile_plan(c.B, c.Hq, c.Hkv, c.L, T)
                             : gen_plan(c.B, c.Hq, c.Hkv, c.L, T);
   if (static_cast<int64_t>(c.Hkv) * gp.n_rg > 65535 || c.B > 65535)
@@ -1264,7 +1335,7 @@ int general_attention(const GenCall& c) {
     rc = check_launch("gen_tile_qprep_kernel");
     if (rc) return rc;
   }
-  rc = wide   ? run_wide(p, rows, plain, st)
+  rc = wide   ? run_wide(p, rows, plain, narrow, st)
        : tile ? launch_tile_partial(p, kb, c.v_bits, st)
               : launch_gen_partial(p, kb, plain ? 0 : c.v_bits, st);
   if (rc) return rc;

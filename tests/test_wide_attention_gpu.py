@@ -17,10 +17,21 @@ from tests.test_general_attention_gpu import packed_case
 pytestmark = pytest.mark.gpu
 
 
-def kv_heads(least, need, B, rows, T, dk, dv):
-    """kv heads that bring rows x T x (dk + dv) products to ``need`` x 2^28, from
-    which the wide kernel takes the call (wide_pays in tq_attn_general.hip)."""
-    return max(least, math.ceil(1.02 * need * 2 ** 28 / (B * rows * T * (dk + dv))))
+def kv_heads(least, B, rows, T, dk, dv, tuned=False, plain=False, masked=False):
+    """kv heads (``rows`` query rows each) from which the wide kernel takes the
+    call: wide_pays in tq_attn_general.hip, in rows of the call and products of 2^28."""
+    if tuned and dk in (64, 128):
+        all_rows, work = 1536, 16
+    elif tuned and dk == 256:
+        all_rows, work = 0, 1.25 if plain else 2.5
+    elif dv > 128:
+        all_rows, work = (1024, 2) if plain else (0, 0.5)
+    elif dk > 128:
+        all_rows, work = 1024, 1
+    else:
+        all_rows, work = (8192, 4) if masked else (1024, 8)
+    return max(least, math.ceil(all_rows / (B * rows)),
+               math.ceil(1.02 * work * 2 ** 28 / (B * rows * T * (dk + dv))))
 
 
 @pytest.mark.parametrize("dk,krot,dv,vrot,kb,vb", [
@@ -43,8 +54,7 @@ def kv_heads(least, need, B, rows, T, dk, dv):
     (4, 2, 70, 1029, [1029, 611], [3, 600])])     # 280 rows; a window shorter than the queries
 def test_wide_packed(device, dk, krot, dv, vrot, kb, vb, R, Hkv, L, T, lengths, starts):
     B = 1 if lengths is None else len(lengths)
-    need = {64: 6, 256: 1.25}.get(dk, 1) if dk == dv and krot == vrot else 1
-    Hkv = kv_heads(Hkv, need, B, R * L, T, dk, dv)
+    Hkv = kv_heads(Hkv, B, R * L, T, dk, dv, tuned=dk == dv and krot == vrot)
     Hq = R * Hkv
     packed_case(device, 40 + dk + dv + L, B, Hq, Hkv, L, T, dk, dv, kb, vb, krot, vrot,
                 qdt="f16" if L == 43 else "bf16", lengths=lengths, starts=starts,
@@ -56,15 +66,17 @@ def test_wide_packed(device, dk, krot, dv, vrot, kb, vb, R, Hkv, L, T, lengths, 
 def test_wide_window_mask(device, d, W, L, T):
     """A sliding window's rows see a band of keys; rows of one block end at different keys."""
     m = create_causal_mask(L, offset=T - L, window_size=W).numpy()
-    packed_case(device, 900 + d + W, 1, 4, 2, L, T, d, d, 3, 3, causal=False, mask_np=m)
+    Hkv = kv_heads(2, 1, 2 * L, T, d, d, masked=True)
+    packed_case(device, 900 + d + W, 1, 2 * Hkv, Hkv, L, T, d, d, 3, 3, causal=False, mask_np=m)
 
 
 @pytest.mark.parametrize("shape", ["2d", "4d", "5d", "keys"])
 def test_wide_bool_mask_shapes_and_empty_rows(device, shape):
     """Rows that keep nothing average every value of their window; a row that
     keeps one key takes it, wherever it lies; a mask broadcast along keys."""
-    B, Hq, Hkv, L, T = 2, 8, 2, 33, 600
-    R = Hq // Hkv
+    B, R, L, T = 2, 4, 33, 600
+    Hkv = kv_heads(2, B, R * L, T, 128, 128, masked=True)
+    Hq = R * Hkv
     rng = np.random.default_rng(77)
     full = {"2d": (L, T), "4d": (B, Hkv, L, T), "5d": (B, Hkv, R, L, T), "keys": (L, 1)}[shape]
     m = rng.random(full) < 0.4
@@ -84,7 +96,9 @@ def test_wide_bool_mask_shapes_and_empty_rows(device, shape):
 @pytest.mark.parametrize("causal", [False, True])
 def test_wide_additive_mask(device, dt, causal):
     """Additive entries, the type's lowest value among them (finite: a row of it is uniform)."""
-    B, Hq, Hkv, L, T = 1, 4, 2, 50, 333
+    B, L, T = 1, 50, 333
+    Hkv = kv_heads(2, B, 2 * L, T, 64, 64, masked=True)
+    Hq = 2 * Hkv
     rng = np.random.default_rng(78)
     tdt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[dt]
     m = O.round_to_dtype(rng.normal(0, 2.0, size=(L, T)).astype(np.float32), dt)
@@ -104,7 +118,7 @@ def test_wide_minus_infinity_mask(device):
     keep = rng.random((L, T)) < 0.2
     keep[:, 11] = True
     add = np.where(keep, 0.0, -np.inf).astype(np.float32)
-    Hkv = kv_heads(2, 1, 1, 2 * L, T, 96, 96)
+    Hkv = kv_heads(2, 1, 2 * L, T, 96, 96, masked=True)
     packed_case(device, 930, 1, 2 * Hkv, Hkv, L, T, 96, 96, 3, 3, "dense", "dense", causal=False, mask_np=keep,
                 mask_t=torch.from_numpy(add).to(device))
 
@@ -115,8 +129,7 @@ def test_wide_minus_infinity_mask(device):
                                                       (2, 2, 48, 400, None, 45)])
 def test_wide_plain(device, kvdt, dk, dv, R, Hkv, L, T, lengths, window):
     B = 1 if lengths is None else len(lengths)
-    if dk == dv and not window:
-        Hkv = kv_heads(Hkv, {64: 6, 128: 4, 256: 1.25}.get(dk, 0), B, R * L, T, dk, dv)
+    Hkv = kv_heads(Hkv, B, R * L, T, dk, dv, tuned=dk == dv and not window, plain=True, masked=bool(window))
     Hq = R * Hkv
     rng = np.random.default_rng(dk + dv + L)
     k = O.round_to_dtype(rng.standard_normal((B, Hkv, T, dk)).astype(np.float32), kvdt)
