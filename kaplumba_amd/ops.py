@@ -32,12 +32,15 @@ def _opt_tensor(x, dtype):
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # torch.cuda.current_stream(t.device).cuda_stream without its Stream object: a
+    # short decode step waits for the host, and asks three times (with the plain
+    # checks of _check_append_buffers and _require_device: 43.0 -> 34.9 us a step)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _require_device(*ts: torch.Tensor) -> None:
     for t in ts:
-        if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+        if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise ValueError("TurboQuant kernels need ROCm device tensors "
                              f"(got {getattr(t, 'device', type(t))}); there is no CPU path")
 
@@ -56,7 +59,7 @@ class Codec:
     seed: int
     rotation: str = "auto"
     codebook_kind: str = "beta"
-    _dev: Dict[str, Dict[str, torch.Tensor]] = field(default_factory=dict, repr=False)
+    _dev: Dict[torch.device, Dict[str, torch.Tensor]] = field(default_factory=dict, repr=False)
 
     def __post_init__(self) -> None:
         pow2 = self.dim > 0 and (self.dim & (self.dim - 1)) == 0
@@ -82,8 +85,7 @@ class Codec:
         return cbmod.rotation_matrix(self.dim, self.seed)
 
     def device_tensors(self, device: torch.device) -> Dict[str, torch.Tensor]:
-        key = str(device)
-        d = self._dev.get(key)
+        d = self._dev.get(device)
         if d is None:
             d = {
                 "rot": torch.from_numpy(np.array(self.rot_host, dtype=np.float32, order="C")).to(device),
@@ -91,7 +93,7 @@ class Codec:
                 "midpoints": torch.from_numpy(
                     self.midpoints.copy() if self.midpoints.size else np.zeros(1, np.float32)).to(device),
             }
-            self._dev[key] = d
+            self._dev[device] = d
         return d
 
 
@@ -132,8 +134,8 @@ def _check_append_buffers(x: torch.Tensor, codec: Codec, packed: torch.Tensor,
     if packed.shape != (B, H, cap, codec.packed_width) or norms.shape != (B, H, cap):
         raise ValueError(f"buffer shapes {tuple(packed.shape)}/{tuple(norms.shape)} "
                          f"do not match ({B}, {H}, cap, {codec.packed_width})")
-    es = x.element_size()
-    if x.data_ptr() % 16 or any((s * es) % 16 for s in x.stride()[:3]):
+    sb, sh, sl, _ = x.stride()
+    if (x.data_ptr() | (sb | sh | sl) * x.element_size()) & 15:
         x = x.contiguous()
     return x
 
@@ -264,7 +266,9 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     (see _RETIRED_WORKSPACES); ``reserve_workspace`` sizes it once before
     graph capture.
     """
-    key = (str(device), torch.cuda.current_stream(device).cuda_stream)
+    stream = (torch.cuda.current_stream(device).cuda_stream if device.index is None
+              else torch._C._cuda_getCurrentRawStream(device.index))
+    key = (device, stream)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:
@@ -281,6 +285,7 @@ def reserve_workspace(device, B: int, Hq: int, Hkv: int, L: int, dim: int,
     caller will run (for example before capturing decode graphs for several
     batch sizes), so no later call on that stream replaces it.  Returns bytes."""
     device = torch.device(device)
+    torch.cuda.init()
     nbytes = int(_lib.load().tq_attention_workspace_size(B, Hq, Hkv, L, dim, max_tokens))
     _workspace(device, nbytes)
     return nbytes
