@@ -472,6 +472,14 @@ int launch_dense_kv_bits(int kbits, int vbits, const AppendArgs& k, const Append
     case 1 * 8 + 2: return launch_dense_kv_pair<D, 1, 2, XDT>(k, v, st);
     case 2 * 8 + 3: return launch_dense_kv_pair<D, 2, 3, XDT>(k, v, st);
     case 3 * 8 + 4: return launch_dense_kv_pair<D, 3, 4, XDT>(k, v, st);
+    // wider keys (K4/V2, K2/V1 and their neighbours).  K + V, bf16, us of a launch
+    // a side -> one launch, K4/V2: 1024 vectors a side d = 64 10.0 -> 6.4, d = 128
+    // 22.5 -> 13.5, d = 256 23.3 -> 13.0; 65536: 11.5 -> 11.4, 26.6 -> 24.8, 78 -> 75
+    // (few tiles leave most CUs idle, and the sides fill them together; K2/V1 alike)
+    case 2 * 8 + 1: return launch_dense_kv_pair<D, 2, 1, XDT>(k, v, st);
+    case 3 * 8 + 2: return launch_dense_kv_pair<D, 3, 2, XDT>(k, v, st);
+    case 4 * 8 + 3: return launch_dense_kv_pair<D, 4, 3, XDT>(k, v, st);
+    case 4 * 8 + 2: return launch_dense_kv_pair<D, 4, 2, XDT>(k, v, st);
   }
   return -1;
 }

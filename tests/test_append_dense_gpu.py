@@ -190,3 +190,25 @@ def test_dense_whole_tiles_batched(device, dtype):
     flips = _check(xt.float().cpu().numpy(), bits, d, 0, gp[:, :, 3:3 + L], norms.cpu().numpy()[:, :, 3:3 + L])
     assert flips <= 2
     assert not gp[:, :, :3].any() and not gp[:, :, 3 + L:].any()
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("kb,vb", [(2, 1), (3, 2), (4, 3), (4, 2)])
+@pytest.mark.parametrize("dtype,L", [(torch.bfloat16, 521), (torch.float16, 1031)])
+def test_dense_wider_keys_one_launch(device, d, kb, vb, dtype, L):
+    """Keys and values of unlike widths in one launch: the words of one launch a
+    side (the same arithmetic), over a ragged last tile, nothing else written."""
+    g = torch.Generator().manual_seed(d + kb)
+    xs = [torch.randn(1, 3, L, d, generator=g).to(dtype).to(device) for _ in range(2)]
+    codecs = [ops.Codec(d, b, s, rotation="dense") for s, b in enumerate((kb, vb))]
+
+    def buffers():
+        return [(torch.full((1, 3, L + 6, c.packed_width), 0x5a5a5a5a, dtype=torch.int32, device=device)
+                 .view(torch.uint32), torch.full((1, 3, L + 6), -7.0, device=device)) for c in codecs]
+
+    both, apart = buffers(), buffers()
+    ops.append_quantize_kv(*xs, *codecs, *both[0], *both[1], 3)
+    for x, c, (p, n) in zip(xs, codecs, apart):
+        ops.append_quantize(x, c, p, n, 3)
+    for (p, n), (wp, wn) in zip(both, apart):
+        assert torch.equal(p.view(torch.int32), wp.view(torch.int32)) and torch.equal(n, wn)
