@@ -779,7 +779,7 @@ extern "C" int tq_dequantize(const uint32_t* packed, const void* norms, int norm
   // the matrix-core kernel shares a split of R among 128 vectors (us of one
   // workgroup per vector -> this: 1024 vectors d = 128 6.2 -> 6.8, d = 256 11.5 ->
   // 10.1; 2048 7.1 -> 6.9 and 22.9 -> 10.5; 32768 76 -> 11.8 and 264 -> 36)
-  if (rot_kind == TQ_ROT_DENSE && dim <= kRotateMaxDim && n >= kDequantDenseMin && n < (int64_t(1) << 31) - 128)
+  if (rot_kind == TQ_ROT_DENSE && dim <= kRotateMaxDim && n >= kDequantDenseMin && n <= kMaxTiledRows)
     return launch_dequant_dense(g, static_cast<int>(n), st);
   return launch_dequant_general(g, n, st);
 }

@@ -1022,7 +1022,7 @@ void launch_qprep_mode(const GenParams& p, int64_t rows, int mode, const float* 
 // vector one beyond (gen_qprep_kernel takes 38 us for 8192 rows of 256, the
 // rotation 10 us; 6.4 and 4.0 us for 256 rows of 96, 11 and 8.3 us for 2240 of 192).
 void launch_dense_queries(const GenParams& p, int64_t rows, const float* mat, float* dst, hipStream_t st) {
-  if (p.Dk > kRotateMaxDim || rows > INT32_MAX) return launch_qprep_mode(p, rows, 2, mat, dst, st);
+  if (p.Dk > kRotateMaxDim || rows > kMaxTiledRows) return launch_qprep_mode(p, rows, 2, mat, dst, st);
   RotateArgs a{};
   a.x = p.q;
   a.x_sb = p.q_sb;
@@ -1343,7 +1343,7 @@ int general_attention(const GenCall& c) {
   // rotation (gen_merge_kernel, which does both on the vector ALUs, takes 207 us
   // for 8192 rows of 256 and 15 us for 256 rows of 96; these two 24 and 9 us)
   const bool merge_dense = !plain && c.v_rot_kind == TQ_ROT_DENSE && c.Dv % 4 == 0 && c.Dv <= kRotateMaxDim &&
-                           (wide || c.Dv <= p.DkP) && rows <= INT32_MAX;
+                           (wide || c.Dv <= p.DkP) && rows <= kMaxTiledRows;
   p.merged = merge_dense ? p.qrot : nullptr;
   // the flat merge takes 4 value columns per thread: plain values need Dv % 4 == 0
   if ((plain && c.Dv % 4 == 0) || p.merge_had || merge_dense) {

@@ -3,6 +3,7 @@
 
 #include "tq_append.h"
 #include "tq_common.h"
+#include "tq_tiles.h"
 
 namespace tq {
 
@@ -24,6 +25,7 @@ struct RotateArgs {
 
 constexpr int kRotateMaxDim = 256;
 
+// At most kMaxTiledRows rows or vectors.
 // q_rot = round_qdtype(q * scale) @ mat^T into f32 rows (k = n <= 256)
 int launch_rotate_queries(const RotateArgs& a, hipStream_t st);
 // out = x @ mat for f32 rows x (k = n <= 256, a multiple of 4, rows and x 16-byte aligned)

@@ -176,7 +176,7 @@ __device__ __forceinline__ void store_tiles(const RotateArgs& a, int r0, int g, 
   }
 }
 
-constexpr int kRotateRows = 128;  // rows per rotate_kernel workgroup
+constexpr int kRotateRows = kTileRows128;  // rows per rotate_kernel workgroup
 
 template <int KS, int XT>
 __global__ __launch_bounds__(512) void rotate_kernel(RotateArgs a) {
@@ -272,7 +272,7 @@ int launch_ks(const RotateArgs& a, hipStream_t st) {
   const int cols = XT == kFromF32Rows ? a.n : a.out_stride;
   const unsigned gy = static_cast<unsigned>((cols + 63) / 64);
   // 128 rows per workgroup where that still gives one to most CUs
-  const unsigned gx = static_cast<unsigned>((a.rows + kRotateRows - 1) / kRotateRows);
+  const unsigned gx = static_cast<unsigned>(tiles_of(a.rows));
   const bool vec = XT == kFromF32Rows || a.x_vec;
   if (vec && static_cast<int64_t>(gx) * gy >= device_cu_count() / 2)
     hipLaunchKernelGGL((rotate_kernel<KS, XT>), dim3(gx, gy), dim3(512), 0, st, a);
@@ -286,8 +286,8 @@ int launch_ks(const RotateArgs& a, hipStream_t st) {
 template <int XT>
 int launch_any(const RotateArgs& a, hipStream_t st) {
   if (a.rows <= 0) return TQ_OK;
-  if (a.k < 4 || a.n < 1 || a.k > kRotateMaxDim || a.n > kRotateMaxDim || a.out_stride > kRotateMaxDim)
-    return fail(TQ_ERR_UNSUPPORTED, "rotate: %d x %d", a.k, a.n);
+  if (a.rows > kMaxTiledRows || a.k < 4 || a.n < 1 || a.k > kRotateMaxDim || a.n > kRotateMaxDim || a.out_stride > kRotateMaxDim)
+    return fail(TQ_ERR_UNSUPPORTED, "rotate: %d rows, %d x %d", a.rows, a.k, a.n);
   switch ((a.k + 31) / 32) {
     case 1:
     case 2: return launch_ks<2, XT>(a, st);
@@ -344,8 +344,9 @@ __global__ __launch_bounds__(512) void dequant_dense_kernel(DequantGeneralArgs a
   const int bits = a.bits;
   const int sh = (8 * g * bits) & 31;
   const uint32_t mask = (1u << bits) - 1u;
-#pragma unroll 1
-  for (int r0 = blockIdx.x * kRotateRows + 16 * (tid >> 6); r0 < n_vec; r0 += gridDim.x * kRotateRows) {
+  walk_tiles(n_vec, blockIdx.x, gridDim.x, [&](int tile0) {
+    const int r0 = tile0 + 16 * (tid >> 6);
+    if (r0 >= n_vec) return;  // a wave past the end
     // the fragments stay in LDS: hoisted out of the loop they spill
     asm volatile("" ::: "memory");
     // lane (vector n, g): coordinates 32 s + 8 g .. + 7, 8 * bits bits from word
@@ -400,14 +401,13 @@ __global__ __launch_bounds__(512) void dequant_dense_kernel(DequantGeneralArgs a
       for (int j = 0; j < 4; ++j)
         if (vj[j] < n_vec && col < D) a.out[static_cast<int64_t>(vj[j]) * D + col] = nrm[j] * acc[t][j];
     }
-  }
+  });
 }
 
 template <int KS>
 int launch_dequant_ks(const DequantGeneralArgs& a, int n, hipStream_t st) {
   const int gy = (a.D + 63) / 64;
-  const int tiles = (n + kRotateRows - 1) / kRotateRows;
-  const int gx = std::min(tiles, std::max(1, 2 * device_cu_count() / gy));
+  const int gx = std::min(tiles_of(n), std::max(1, 2 * device_cu_count() / gy));
   hipLaunchKernelGGL(dequant_dense_kernel<KS>, dim3(static_cast<unsigned>(gx), static_cast<unsigned>(gy)), dim3(512), 0, st, a, n);
   return check_launch("dequant_dense_kernel");
 }
