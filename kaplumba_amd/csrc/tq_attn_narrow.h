@@ -58,8 +58,8 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
   using S = NarrowShape<KS, CT, SRC>;
   constexpr bool PACKED = S::PACKED;
   constexpr int WP = SRC == kWideBf16 ? 3 : 2;
-  constexpr float kLazy = 7.f;
-  constexpr int kWExp = SRC != kWideBf16 ? 8 : 0;  // weights carry 2^kWExp
+  constexpr float kLazy = kWideLazy;
+  constexpr int kWExp = SRC != kWideBf16 ? 8 : 0;  // the largest weights carry 2^kWExp
   constexpr int SUB = 32;
   __shared__ __align__(16) unsigned char lds[S::BYTES];
   const int tid = threadIdx.x;
@@ -276,10 +276,7 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
   f32x4_t O[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) O[ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_row = -INFINITY, l_acc = 0.f;
-  int E = PACKED ? kWExp - 126 : 0;
-  float vsc = ldexpf(1.f, kWExp - E);
-  float vlim = ldexpf(1.f, E);
+  WideRow row = {-INFINITY, 0.f, PACKED ? 0x1p126f : static_cast<float>(1 << kWExp)};
   unsigned char* const tile = lds + S::TILE + wave * S::WAVE;
   const uint32_t tile_off = S::TILE + wave * S::WAVE;
   uint32_t vtr[2];
@@ -301,7 +298,6 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
     if (p.mask_kind == TQ_MASK_BOOL)
       mk = wide_mask_bytes(static_cast<const uint8_t*>(p.mask) + mrow, p.m_st, t0 + 8 * g, len);
     float knv[8], vnv[8];
-    float vm = 0.f;
     if constexpr (PACKED) {
       float* nt = reinterpret_cast<float*>(tile + S::VBYTES);
       nt[lane] = nreg;
@@ -310,8 +306,6 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
       *reinterpret_cast<float4*>(knv + 4) = *reinterpret_cast<const float4*>(nt + 8 * g + 4);
       *reinterpret_cast<float4*>(vnv) = *reinterpret_cast<const float4*>(nt + 32 + 8 * g);
       *reinterpret_cast<float4*>(vnv + 4) = *reinterpret_cast<const float4*>(nt + 32 + 8 * g + 4);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) vm = fmaxf(vm, vnv[j]);
     }
     // ---- scores S^T = K Q^T, tiles h of 16 tokens
     f32x4_t C[2];
@@ -354,51 +348,40 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
         ym = fmaxf(ym, y[j]);
       }
     }
-    if (__any((PACKED && vm > vlim) || ym > m_row + kLazy ? 1 : 0)) {
-      // a new reference maximum or norm exponent: rescale
-      int e2 = E;
-      float esc = 1.f;
-      if constexpr (PACKED) {
-        const float vw = wave_max(vm);
-        if (vw > vlim) {
-          int ev;
-          frexpf(vw, &ev);
-          e2 = ev;
-        }
-        esc = ldexpf(1.f, E - e2);
+    float fo = 1.f;  // factor of the row's O
+    bool moved = __any(ym > row.m + kLazy ? 1 : 0);
+    if (moved) fo = wide_row_rise<PACKED>(row, ym);
+    float w[8];
+    float wm = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float pe = row.m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y[j] - row.m);
+      row.l += pe;
+      w[j] = PACKED ? pe * vnv[j] : pe;
+      wm = fmaxf(wm, w[j]);
+    }
+    if constexpr (PACKED) {
+      if (__any(wm * row.vsc > kWideTop ? 1 : 0)) {
+        fo *= wide_row_drop<kWExp>(row, wm, kWideTop);
+        moved = true;
       }
-      float r = fmaxf(ym, xor_lane<16>(ym));
-      {
-        const float2 hh = halves(r);
-        r = fmaxf(hh.x, hh.y);  // the row's maximum over the sub-chunk
-      }
-      const float mo = m_row;
-      const float mn = r > mo + kLazy ? fmaxf(mo, r) : mo;
-      const float am = mo == mn ? 1.f : (mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - mn));
-      const float ao = am * esc;
-      l_acc *= am;
+    }
+    if (moved) {
       float ar[4];  // O rows 4 g + k of this lane take the factor of row 4 g + k
 #pragma unroll
-      for (int k = 0; k < 4; ++k) ar[k] = __shfl(ao, 4 * g + k, 64);
+      for (int k = 0; k < 4; ++k) ar[k] = __shfl(fo, 4 * g + k, 64);
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int k = 0; k < 4; ++k) O[ct][k] *= ar[k];
-      m_row = mn;
-      E = e2;
-      vsc = ldexpf(1.f, kWExp - E);
-      vlim = ldexpf(1.f, E);
     }
     u32x4_t A[WP];
     {
-      float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float pe = m_row == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y[j] - m_row);
-        l_acc += pe;
         // in a register of its own: the product folded into the f16 conversion
         // rounds once, and the low part would belong to another high part
-        w[j] = own_reg(PACKED ? pe * (vnv[j] * vsc) : pe * vsc);
+        w[j] = own_reg(w[j] * row.vsc);
       }
 #pragma unroll
       for (int q = 0; q < WP; ++q)
@@ -453,20 +436,22 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
   }
 
   // ---- the waves' partials meet in LDS: o scaled to the value basis, (m, l)
-  float lr = l_acc + xor_lane<16>(l_acc);
+  float lr = row.l + xor_lane<16>(row.l);
   {
     const float2 h = halves(lr);
     lr = h.x + h.y;
   }
-  const float osc = ldexpf(1.f, E - kWExp) / sv;
+  float osc[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) osc[k] = __shfl(1.f / row.vsc, 4 * g + k, 64) / sv;
   __syncthreads();
   float* s_o = reinterpret_cast<float*>(lds) + wave * 16 * S::DVP;
   float2* s_ml = reinterpret_cast<float2*>(lds + S::OML);
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) s_o[(4 * g + k) * S::DVP + 16 * ct + n] = O[ct][k] * osc;
-  if (g == 0) s_ml[wave * 16 + n] = make_float2(m_row, lr);
+    for (int k = 0; k < 4; ++k) s_o[(4 * g + k) * S::DVP + 16 * ct + n] = O[ct][k] * osc[k];
+  if (g == 0) s_ml[wave * 16 + n] = make_float2(row.m, lr);
   __syncthreads();
   const int rows = min(kNarrowRows, RL - row0);
   for (int e = tid; e < rows * S::DVP; e += S::NT) {

@@ -33,8 +33,8 @@
 // 119 and 172 us.
 //
 // Weight pieces WP.  1: f16 weights, as the other packed kernels.  More where
-// the general vector kernel held weights in f32: f16 hi + lo (2; weights
-// carry 2^8 so the lo parts stay normal), bf16 hi + mid + lo (3); plain bf16
+// the general vector kernel held weights in f32: f16 hi + lo (2; under a power
+// of two that keeps the lo parts normal), bf16 hi + mid + lo (3); plain bf16
 // layers always take hi + lo (2), as attn_plain_kernel.  Scores: packed keys
 // K_hi Q_hi + K_hi Q_lo + K_lo Q_hi (f32-class); plain keys are exact in
 // their type and so are the queries, which share it: one product.
@@ -149,14 +149,80 @@ __device__ __forceinline__ float wide_mask_add(const GenParams& p, int64_t off) 
   return (t == -INFINITY && m != -INFINITY) ? -FLT_MAX : t;
 }
 
+// Scores grow by up to 2^kWideLazy past a row's reference maximum before it moves.
+constexpr float kWideLazy = 7.f;
+constexpr float kWideTop = 32768.f;  // bound of scaled weights, whole in f16
+
+// Row state of the online softmax, one row per 16-lane column (lanes n + 16 g):
+// m reference maximum (log2 units), l this lane's share of the sum, vsc the power
+// of two that the weights p * n_t of packed values carry as f16 pieces (plain: p).
+//
+// Where the weights are f32-class (wide_general), vsc follows the row's own: it
+// drops when one passes 2^15 under it and rises with the maximum (what O holds
+// shrinks then).  A token of huge norm that the row masks or hardly weighs (a
+// padded or corrupt one) so costs the others no bits; a scale by the norms lost
+// all of them from 2^30 on.  One-piece weights keep the tuned kernels' rule, one
+// scale for all rows, of the largest norm met (a scale a row: prefill of d = 64,
+// which keeps every token of its window, 128.0 -> 131.4 us).
+struct WideRow {
+  float m, l, vsc;
+};
+
+__device__ __forceinline__ float wide_row_max(float x) {  // over the row's four lanes
+  x = fmaxf(x, xor_lane<16>(x));
+  const float2 h = halves(x);
+  return fmaxf(h.x, h.y);
+}
+
+// The row meets scores of maximum rm (this lane's): moves m where it has to.
+// Returns the factor of O.
+template <bool PACKED>
+__device__ __forceinline__ float wide_row_rise(WideRow& w, float rm) {
+  const float r = wide_row_max(rm);
+  const float mo = w.m;
+  const float mn = r > mo + kWideLazy ? fmaxf(mo, r) : mo;
+  const float am = mo == mn ? 1.f : (mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - mn));
+  w.l *= am;
+  w.m = mn;
+  float f = am;
+  if constexpr (PACKED) {
+    if (am == 0.f) {  // nothing is held any more (so far only masked keys, or far below)
+      w.vsc = 0x1p126f;
+    } else if (am < 1.f) {  // the whole part of the shrinkage goes to vsc, up to 2^126
+      int e = 0;
+      frexpf(w.vsc, &e);
+      const int up = min(static_cast<int>(mn - mo), 127 - e);
+      w.vsc = ldexpf(w.vsc, up);
+      f = ldexpf(am, up);
+    }
+  }
+  return f;
+}
+
+// The row's weights (or norms) reach wm (this lane's): where that passes top under
+// vsc, brings it to 2^WEXP.  Returns the factor of O.
+template <int WEXP>
+__device__ __forceinline__ float wide_row_drop(WideRow& w, float wm, float top) {
+  const float x = wide_row_max(wm);
+  float f = 1.f;
+  if (x * w.vsc > top) {
+    int e = 0;
+    frexpf(x, &e);
+    const float v = ldexpf(1.f, max(WEXP - e, -120));
+    f = v / w.vsc;
+    w.vsc = v;
+  }
+  return f;
+}
+
 template <int KS, int CT, int RT, int SRC, int WP>
 __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int n_blocks) {
   using S = WideShape<KS, CT, RT, SRC, WP>;
   constexpr bool PACKED = S::PACKED;
   constexpr bool GEN = wide_general<SRC, WP>();
   constexpr int SUB = S::SUB, H = S::H;
-  constexpr float kLazy = 7.f;
-  constexpr int kWExp = (SRC != kWideBf16 && WP > 1) ? 8 : 0;  // weights carry 2^kWExp
+  constexpr float kLazy = kWideLazy;
+  constexpr int kWExp = (SRC != kWideBf16 && WP > 1) ? (PACKED ? 4 : 8) : 0;  // the largest weights carry 2^kWExp
   __shared__ __align__(16) unsigned char lds[S::BYTES];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -466,16 +532,12 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) O[rt][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_row[RT];  // reference maximum of the row (log2 units)
-  float l_acc[RT];  // this lane's share of the row's sum
+  WideRow row[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    m_row[rt] = -INFINITY;
-    l_acc[rt] = 0.f;
-  }
-  int E = PACKED ? kWExp - 126 : 0;  // value norms <= 2^E (weights carry 2^-E), shared by the wave's rows
-  float vsc = ldexpf(1.f, kWExp - E);
-  float vlim = ldexpf(1.f, E);
+  for (int rt = 0; rt < RT; ++rt) row[rt] = WideRow{-INFINITY, 0.f, PACKED ? 0x1p126f : static_cast<float>(1 << kWExp)};
+
+  constexpr float kOneTop = static_cast<float>(1 << kWExp);
+  float vlim = 0.f;  // one-piece weights: norms up to here need no new scale
 
   const uint32_t ka = S::KHI + n * S::KROW + 16 * g;
   uint32_t vtr[2];
@@ -546,7 +608,7 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
     }
     // y = n_t <q, c> in MFMA units of the row; x = y * qmul in log2 units
     float y[RT][8];
-    bool grow = PACKED && vm > vlim;
+    bool grow = PACKED && !GEN && vm > vlim;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       float ym = -INFINITY;
@@ -556,8 +618,8 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
         if constexpr (PACKED) y[rt][j] *= knv[j];
         ym = fmaxf(ym, y[rt][j]);
       }
-      grow |= ym * qmul[rt] > m_row[rt] + kLazy;
-    }
+      grow |= ym * qmul[rt] > row[rt].m + kLazy;
+          }
     bool special = t0 + 32 > t_end || t0 + 31 > lim_min;  // wave-uniform
     if constexpr (GEN) {
       if (p.mask_kind == TQ_MASK_BOOL) {
@@ -570,8 +632,17 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
       }
     }
     float pe[RT][8];
+    bool moved = false;
+    // the step's first half rescales O at once; its second half only after the
+    // first half's products, which still carry the old scale
+    auto scale_moved = [&]() {
+      if (hf == 0)
+        rescale(fac);
+      else
+        pending = true;
+    };
     if (special || __any(grow ? 1 : 0)) {
-      // slow path: masks, a new reference maximum or norm exponent, rescale
+      // slow path: masks, a new reference maximum
       float rm[RT];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
@@ -596,44 +667,26 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
 #pragma unroll
         for (int j = 0; j < 8; ++j) rm[rt] = fmaxf(rm[rt], y[rt][j]);
       }
-      bool up = PACKED && vm > vlim;
+      bool up = false;
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) up |= rm[rt] > m_row[rt] + kLazy;
+      for (int rt = 0; rt < RT; ++rt) up |= rm[rt] > row[rt].m + kLazy;
+      if constexpr (PACKED && !GEN) up |= vm > vlim;
       if (__any(up ? 1 : 0)) {
-        int e2 = E;
-        float esc = 1.f;
-        if constexpr (PACKED) {
-          const float vw = wave_max(vm);
-          if (vw > vlim) {
-            int ev;
-            frexpf(vw, &ev);
-            e2 = ev;
-          }
-          esc = ldexpf(1.f, E - e2);
-        }
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          float r = fmaxf(rm[rt], xor_lane<16>(rm[rt]));
-          {
-            const float2 hh = halves(r);
-            r = fmaxf(hh.x, hh.y);  // the row's maximum over the half
+        for (int rt = 0; rt < RT; ++rt) fac[rt] = wide_row_rise<PACKED && GEN>(row[rt], rm[rt]);
+        if constexpr (PACKED && !GEN) {
+          const float f = wide_row_drop<kWExp>(row[0], wave_max(vm), kOneTop);
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) {
+            fac[rt] *= f;
+            row[rt].vsc = row[0].vsc;
           }
-          const float mo = m_row[rt];
-          const float mn = r > mo + kLazy ? fmaxf(mo, r) : mo;
-          const float am = mo == mn ? 1.f : (mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - mn));
-          fac[rt] = am * esc;
-          l_acc[rt] *= am;
-          m_row[rt] = mn;
+          vlim = kOneTop / row[0].vsc;
         }
-        // the step's first half rescales O here; its second half only after
-        // the first half's products, which still carry the old maximum
-        if (hf == 0)
-          rescale(fac);
+        if constexpr (PACKED && GEN)
+          moved = true;
         else
-          pending = true;
-        E = e2;
-        vsc = ldexpf(1.f, kWExp - E);
-        vlim = ldexpf(1.f, E);
+          scale_moved();
       }
       // masked keys (-FLT_MAX) weigh 1 while their whole row is masked
       // (m = -FLT_MAX), else 0; keys past the end (-inf) always 0
@@ -641,26 +694,61 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          pe[rt][j] = m_row[rt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y[rt][j] - m_row[rt]);
+          pe[rt][j] = row[rt].m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y[rt][j] - row[rt].m);
     } else {
       // every score within 2^7 of a finite reference maximum
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        const float nm = -m_row[rt];
+        const float nm = -row[rt].m;
 #pragma unroll
         for (int j = 0; j < 8; ++j) pe[rt][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[rt][j], qmul[rt], nm));
       }
     }
-    float vs[8];
+    float vs[8];  // one scale for all rows: with n_t in one factor
 #pragma unroll
-    for (int j = 0; j < 8; ++j) vs[j] = PACKED ? vnv[j] * vsc : vsc;
+    for (int j = 0; j < 8; ++j) vs[j] = PACKED && !GEN ? vnv[j] * row[0].vsc : row[0].vsc;
+    if constexpr (PACKED && GEN) {
+      // no weight passes 2^15 while the norms, times the 2^7 that a score may
+      // stand above its reference, do not: one compare a row
+      bool near = false;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) near |= vm * row[rt].vsc > kWideTop / 128.f;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          row[rt].l += pe[rt][j];
+          pe[rt][j] *= vnv[j];
+        }
+      if (__any(near ? 1 : 0)) {
+        float wm[RT];
+        bool over = false;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          wm[rt] = 0.f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) wm[rt] = fmaxf(wm[rt], pe[rt][j]);
+          over |= wm[rt] * row[rt].vsc > kWideTop;
+        }
+        if (__any(over ? 1 : 0)) {
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) {
+            const float f = wide_row_drop<kWExp>(row[rt], wm[rt], kWideTop);
+            fac[rt] = moved ? fac[rt] * f : f;
+          }
+          moved = true;
+        }
+      }
+      if (moved) scale_moved();
+    }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        l_acc[rt] += pe[rt][j];
-        w[j] = (PACKED || kWExp != 0) ? pe[rt][j] * vs[j] : pe[rt][j];
+        if constexpr (!(PACKED && GEN)) row[rt].l += pe[rt][j];
+        w[j] = pe[rt][j];
+        if constexpr (PACKED || kWExp != 0) w[j] *= PACKED && GEN ? row[rt].vsc : vs[j];
         // in a register of its own: the product folded into the f16 conversion
         // rounds once, and the low part would belong to another high part
         if constexpr (WP > 1) w[j] = own_reg(w[j]);
@@ -771,11 +859,11 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
     }
     lds_barrier();
   }
-  // ---- partials: (o, m, l) per row, o = O * 2^E / sv (packed: in the rotated value basis)
+  // ---- partials: (o, m, l) per row, o = O / (vsc sv) (packed: in the rotated value basis)
   if (!wave_live) return;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    float lr = l_acc[rt] + xor_lane<16>(l_acc[rt]);
+    float lr = row[rt].l + xor_lane<16>(row[rt].l);
     {
       const float2 h = halves(lr);
       lr = h.x + h.y;
@@ -783,15 +871,15 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
     const int rr = row_w0 + 16 * rt + n;
     if (g == 0 && row_ok[rt]) {
       float* pm = p.pml + ((grp0 + rr / 8) * p.n_splits + split) * 16 + (rr % 8) * 2;
-      pm[0] = m_row[rt] * 0.6931471805599453f;  // natural-log units
+      pm[0] = row[rt].m * 0.6931471805599453f;  // natural-log units
       pm[1] = lr;
     }
   }
-  const float osc = ldexpf(1.f, E - kWExp) / sv;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
+      const float osc = (PACKED && GEN ? __shfl(1.f / row[rt].vsc, 4 * g + k, 64) : 1.f / row[0].vsc) / sv;
       const int rr = row_w0 + 16 * rt + 4 * g + k;
       if (rr >= RL) continue;
       float* po = p.po + (((grp0 + rr / 8) * p.n_splits + split) * 8 + rr % 8) * static_cast<int64_t>(p.Dv);
