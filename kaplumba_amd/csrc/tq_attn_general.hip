@@ -890,9 +890,15 @@ bool wide_had_queries(int Dk, int rot_kind) {
   return rot_kind == TQ_ROT_HADAMARD && (Dk == 64 || Dk == 128 || Dk == 256);
 }
 
+// Calls that only the vector kernel served before, with weights in f32: array
+// masks, other dims, K / V dims or rotations that differ.
+bool vector_weights(int mask_kind, int Dk, int Dv, bool plain, int k_rot_kind, int v_rot_kind) {
+  const bool pow2dim = Dk == Dv && (Dk == 64 || Dk == 128 || Dk == 256);
+  return mask_kind != TQ_MASK_NONE || !pow2dim || (!plain && k_rot_kind != v_rot_kind);
+}
+
 // Prepares the queries (and mask ranges) and runs the wide kernel over p,
-// whose workspace pointers follow wide_layout; general: the weights were f32
-// in the vector kernel.
+// whose workspace pointers follow wide_layout.
 int run_wide(GenParams& p, int64_t rows, bool plain, bool narrow, hipStream_t st) {
   int ks = 0, ct = 0;
   wide_dims(p.Dk, p.Dv, ks, ct);
@@ -927,9 +933,7 @@ int run_wide(GenParams& p, int64_t rows, bool plain, bool narrow, hipStream_t st
     if (!plain) return launch_narrow_packed(p, st);
     return p.key_kind == kGenPlainBf16 ? launch_narrow_bf16(p, st) : launch_narrow_f16(p, st);
   }
-  // the vector kernel's f32 weights: array masks and the dims it alone served
-  const bool pow2dim = p.Dk == p.Dv && (p.Dk == 64 || p.Dk == 128 || p.Dk == 256);
-  const bool f32_weights = p.mask_kind != TQ_MASK_NONE || !pow2dim || (!plain && p.k_rot_kind != p.v_rot_kind);
+  const bool f32_weights = vector_weights(p.mask_kind, p.Dk, p.Dv, plain, p.k_rot_kind, p.v_rot_kind);
   if (!plain) return launch_wide_packed(p, f32_weights, st);
   return p.key_kind == kGenPlainBf16 ? launch_wide_bf16(p, f32_weights, st) : launch_wide_f16(p, f32_weights, st);
 }
@@ -1058,10 +1062,16 @@ bool wide_rows_path(int kv_kind, int Dk, int Dv, int rows) {
 }
 
 // Shapes, types and alignment that the wide and narrow kernels take: packed
-// MSE caches, or plain ones in the queries' type with whole 16-byte rows.
+// MSE caches, or plain ones in the queries' type with whole 16-byte rows.  f32
+// queries over packed caches keep the vector kernel's f32 arithmetic where it
+// served them: operands in two f16 pieces have 22 bits, and the errors of f32
+// outputs were 1.1-1.7 times larger (16-bit outputs round both alike).
 static bool mfma_operands(const GenCall& c) {
   int ks = 0, ct = 0;
   if (c.kv_kind != TQ_KV_PACKED && c.kv_kind != TQ_KV_PLAIN) return false;
+  if (c.q_dtype == TQ_DTYPE_F32 &&
+      vector_weights(c.mask_kind, c.Dk, c.Dv, c.kv_kind == TQ_KV_PLAIN, c.k_rot_kind, c.v_rot_kind))
+    return false;
   if (!wide_dims(c.Dk, c.Dv, ks, ct)) return false;
   if (c.capacity > INT32_MAX || static_cast<int64_t>(c.B) * c.Hq * c.L >= (int64_t(1) << 30)) return false;
   return c.kv_kind == TQ_KV_PACKED ||
