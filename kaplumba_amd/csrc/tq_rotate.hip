@@ -4,7 +4,12 @@
 // f32-class products: M and f32 rows go into three bf16 pieces (24
 // significand bits), f16 queries into two, bf16 queries into one; all pieces
 // of an entry sum to it exactly, products whose orders add up to more than 2
-// are below f32 resolution and skipped, sums run in f32.
+// are below f32 resolution and skipped, sums run in f32, in one chain per order:
+// a matrix product may round its accumulator by up to 4 units of 2^-24 of the
+// sum of magnitudes (measured), and the main chain so meets one of them per 32
+// terms instead of up to six.  Error of a reconstruction at d = 64 / 256 with all
+// orders in one chain 0.9e-7 / 2.2e-7, so 0.5e-7 / 0.8e-7; f32 chains of d terms
+// 1.5e-7 / 2.9e-7.
 //
 // rotate_kernel: a workgroup takes 128 rows and 64 columns.  It splits its 64
 // columns of M once into LDS, in B-fragment order (conflict-free 16-byte
@@ -45,6 +50,15 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4_t (&w)[NP]) {
       b = __fsub_rn(b, __uint_as_float(u & 0xffff0000u));
     }
   }
+}
+
+// The product's sum from its chains, one per order of the pieces' product: the
+// main chain is rounded once per step only.
+__device__ __forceinline__ f32x4_t sum_orders(f32x4_t o0, f32x4_t o1, f32x4_t o2) {
+  f32x4_t y;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] = __fadd_rn(__fadd_rn(o2[j], o1[j]), o0[j]);
+  return y;
 }
 
 constexpr int kFromF32Rows = -1;  // XT: contiguous f32 rows; else the queries' TQ_DTYPE_*
@@ -214,21 +228,25 @@ __global__ __launch_bounds__(512) void rotate_kernel(RotateArgs a) {
   x.split(a, g, xp);
   __syncthreads();
 
-  f32x4_t acc[4];
+  f32x4_t acc[3][4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int o = 0; o < 3; ++o)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[o][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < KS; ++s)
 #pragma unroll
-    for (int mp = 2; mp >= 0; --mp)  // smallest terms of a step first
+    for (int mp = 2; mp >= 0; --mp)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const u32x4_t b = s_m[mp * FR + (t * KS + s) * 64 + lane];
 #pragma unroll
         for (int q = X::NX - 1; q >= 0; --q)
-          if (q + mp <= 2) acc[t] = mfma_bf16(xp[s][q], b, acc[t]);
+          if (q + mp <= 2) acc[q + mp][t] = mfma_bf16(xp[s][q], b, acc[q + mp][t]);
       }
-  store_tiles<X::QUERY, 4>(a, r0, g, c0 + n, acc);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[0][t] = sum_orders(acc[0][t], acc[1][t], acc[2][t]);
+  store_tiles<X::QUERY, 4>(a, r0, g, c0 + n, acc[0]);
 }
 
 template <int KS, int XT, bool VEC>
@@ -247,7 +265,7 @@ __global__ __launch_bounds__(256) void rotate_few_kernel(RotateArgs a) {
   x.load(a, r0, n, g);
   u32x4_t xp[KS][X::NX];
   x.split(a, g, xp);
-  f32x4_t acc[3];  // one chain per piece of M, the smallest terms added first
+  f32x4_t acc[3];
 #pragma unroll
   for (int p = 0; p < 3; ++p) acc[p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -259,11 +277,9 @@ __global__ __launch_bounds__(256) void rotate_few_kernel(RotateArgs a) {
     for (int p = 2; p >= 0; --p)
 #pragma unroll
       for (int q = X::NX - 1; q >= 0; --q)
-        if (q + p <= 2) acc[p] = mfma_bf16(xp[s][q], w[p], acc[p]);
+        if (q + p <= 2) acc[q + p] = mfma_bf16(xp[s][q], w[p], acc[q + p]);
   }
-  f32x4_t y[1];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) y[0][j] = (acc[2][j] + acc[1][j]) + acc[0][j];
+  const f32x4_t y[1] = {sum_orders(acc[0], acc[1], acc[2])};
   store_tiles<X::QUERY, 1>(a, r0, g, col, y);
 }
 
@@ -370,9 +386,11 @@ __global__ __launch_bounds__(512) void dequant_dense_kernel(DequantGeneralArgs a
       const int vbh = v / a.T;
       nrm[j] = load_norm(a.norms, a.norm_dtype, static_cast<int64_t>(vbh) * a.cap + (v - vbh * a.T));
     }
-    f32x4_t acc[4];
+    f32x4_t acc[3][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int o = 0; o < 3; ++o)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[o][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       u32x4_t xp[3];
@@ -391,15 +409,16 @@ __global__ __launch_bounds__(512) void dequant_dense_kernel(DequantGeneralArgs a
           const u32x4_t b = s_m[mp * FR + (t * KS + s) * 64 + lane];
 #pragma unroll
           for (int q = 2; q >= 0; --q)
-            if (q + mp <= 2) acc[t] = mfma_bf16(xp[q], b, acc[t]);
+            if (q + mp <= 2) acc[q + mp][t] = mfma_bf16(xp[q], b, acc[q + mp][t]);
         }
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int col = c0 + 16 * t + n;
+      const f32x4_t y = sum_orders(acc[0][t], acc[1][t], acc[2][t]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (vj[j] < n_vec && col < D) a.out[static_cast<int64_t>(vj[j]) * D + col] = nrm[j] * acc[t][j];
+        if (vj[j] < n_vec && col < D) a.out[static_cast<int64_t>(vj[j]) * D + col] = nrm[j] * y[j];
     }
   });
 }
