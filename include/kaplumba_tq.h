@@ -90,8 +90,11 @@ int tq_append_quantize(const void* x, int x_dtype, int B, int H, int L, int dim,
  * destination; the shape (B, H, L, dim), x_dtype, rot_kind, norm_dtype,
  * capacity and offset are shared.  F16 / BF16 input at dim 64 / 128 / 256
  * with equal widths or v_bits = k_bits + 1 (the x.5-bit split) runs both
- * sides in one kernel launch, for either rotation; other cases run the two
- * quantizers one after the other.  Results are identical either way.
+ * sides in one kernel launch, for either rotation; the dense rotation does so
+ * too for k_bits / v_bits of 2/1, 3/2, 4/3 and 4/2, and for every input at the
+ * other dims up to 256 that are multiples of 8; other cases run the two
+ * quantizers one after the other.  Results are identical either way, and a
+ * vector's words do not depend on the other vectors of the call.
  */
 int tq_append_quantize_kv(const void* k_x, const void* v_x, int x_dtype, int B, int H, int L,
                           int dim, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_l,

@@ -80,19 +80,20 @@ __device__ __forceinline__ void div_by_norm(const float (&x)[32], float den, flo
 
 // Dense-rotation quantizer on the matrix cores (tq_append_dense.hip).
 int launch_append_dense(const AppendArgs& a, int dim, int bits, int x_dtype, hipStream_t st);
-// Keys and values in one launch (16-bit input, dim 64 / 128 / 256, equal
-// widths or v_bits = k_bits + 1); returns -1 for other cases.
+// Keys and values in one launch: 16-bit input at dim 64 / 128 / 256 with equal
+// widths, values one bit wider, or the wider keys of 2/1, 3/2, 4/3 and 4/2 (the
+// splits that caches use; the other pairs, and f32 input, take a launch a side),
+// and every call of append_few_path.  Returns -1 for other cases.
 int launch_append_dense_kv(const AppendArgs& k, const AppendArgs& v, int dim, int kbits, int vbits,
                            int x_dtype, hipStream_t st);
 // Dense rotation at any dim (multiples of 8 up to 512) on the vector ALUs
 // (tq_append_general.hip), for the dims the matrix-core kernels do not take.
 int launch_append_dense_general(const AppendArgs& a, int dim, int bits, int x_dtype, hipStream_t st);
 
-// Dense rotation of few vectors at dims that are multiples of 8 up to 256
+// Dense rotation at dims that are multiples of 8 up to 256 but not 64, 128 or 256
 // (tq_append_few.hip): one side (sides = 1, v unused) or both in one launch, any
-// widths.  append_few_path: whether a call of n_vec vectors a side takes it;
-// paired: the other way is one append_dense_kv_kernel launch.
-bool append_few_path(int64_t n_vec, int dim, int sides, bool paired);
+// widths.  append_few_path: whether a call of n_vec vectors a side takes it.
+bool append_few_path(int64_t n_vec, int dim);
 int launch_append_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
                       hipStream_t st);
 

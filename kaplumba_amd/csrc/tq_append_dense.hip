@@ -498,8 +498,7 @@ int launch_append_dense_kv(const AppendArgs& k, const AppendArgs& v, int dim, in
                            int x_dtype, hipStream_t st) {
   if ((reinterpret_cast<uintptr_t>(k.rot) & 15u) != 0 || (reinterpret_cast<uintptr_t>(v.rot) & 15u) != 0)
     return fail(TQ_ERR_INVALID_ARGUMENT, "append: dense rotation matrix must be 16-byte aligned");
-  const bool paired = x_dtype != TQ_DTYPE_F32 && (kbits == vbits || kbits + 1 == vbits);
-  if (append_few_path(static_cast<int64_t>(k.B) * k.H * k.L, dim, 2, paired))
+  if (append_few_path(static_cast<int64_t>(k.B) * k.H * k.L, dim))
     return launch_append_few(k, v, 2, dim, kbits, vbits, x_dtype, st);
   switch (dim) {
     case 64: return launch_dense_kv_dim<64>(x_dtype, kbits, vbits, k, v, st);
@@ -523,7 +522,7 @@ int launch_append_dense_signs(const AppendArgs& a, int dim, hipStream_t st) {
 int launch_append_dense(const AppendArgs& a, int dim, int bits, int x_dtype, hipStream_t st) {
   if ((reinterpret_cast<uintptr_t>(a.rot) & 15u) != 0)
     return fail(TQ_ERR_INVALID_ARGUMENT, "append: dense rotation matrix must be 16-byte aligned");
-  if (append_few_path(static_cast<int64_t>(a.B) * a.H * a.L, dim, 1, false))
+  if (append_few_path(static_cast<int64_t>(a.B) * a.H * a.L, dim))
     return launch_append_few(a, a, 1, dim, bits, bits, x_dtype, st);
   switch (dim) {
     case 64: return launch_dense_dim<64>(a, bits, x_dtype, st);

@@ -1,4 +1,6 @@
-// Dense-rotation append of few vectors (decode and verify steps, short chunks)
+// Dense-rotation append at dims that are multiples of 8 up to 256, but not 64, 128
+// or 256 (those take tq_append_dense.hip at every size: its sums run in another
+// order, and a vector's words must not depend on how many are appended with it),
 // on v_mfma_f32_16x16x32_bf16, keys and values in one launch.
 //
 // Semantics and arithmetic as tq_append_dense.hip: y * max(n, eps) = x @ R^T from
@@ -62,13 +64,12 @@ constexpr int kFewMaxDim = 256;
 // Margin of a tie in ulps of 1 per unit of |x| |R_i|: a margin of one already
 // gave the vector kernel's words over 65 million coordinates of 6 dims.
 constexpr float kTieUlps = 4;
-constexpr int kFewTunedVecs = 512;          // vectors a side at d = 64, 128, 256
 constexpr int kFewIdxRow = kFewCoords + 4;  // bytes per vector's indices in LDS
 
 // KS: 32-element steps that hold the dim (a multiple of 8)
 template <int KS, int XDT>
 __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, AppendArgs va, int D, int kbits, int vbits,
-                                                                int n_vec, bool exact_ties) {
+                                                                int n_vec) {
   constexpr int NX = XDT == TQ_DTYPE_BF16 ? 1 : (XDT == TQ_DTYPE_F16 ? 2 : 3);
   __shared__ __align__(16) uint8_t s_idx[16 * kFewIdxRow];
   const bool key = blockIdx.z == 0;
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
       tie[j] |= fabsf(d) <= margin * dj[j];
     }
   }
-  if (exact_ties && __any(tie[0] | tie[1] | tie[2] | tie[3])) {
+  if (__any(tie[0] | tie[1] | tie[2] | tie[3])) {
 #pragma unroll 1
     for (int j = 0; j < 4; ++j) {
       const bool mine = j == 0 ? tie[0] : j == 1 ? tie[1] : j == 2 ? tie[2] : tie[3];
@@ -301,18 +302,17 @@ template <int KS>
 int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,
                hipStream_t st) {
   const int n_vec = k.B * k.H * k.L;
-  const bool ties = dim != 64 && dim != 128 && dim != 256;  // the dims of the vector kernel
   const dim3 grid(static_cast<unsigned>((n_vec + 15) / 16), static_cast<unsigned>((dim + kFewCoords - 1) / kFewCoords),
                   static_cast<unsigned>(sides));
   switch (x_dtype) {
     case TQ_DTYPE_F32:
-      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F32>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec, ties);
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F32>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
       break;
     case TQ_DTYPE_F16:
-      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec, ties);
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_F16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
       break;
     default:
-      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_BF16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec, ties);
+      hipLaunchKernelGGL((append_few_kernel<KS, TQ_DTYPE_BF16>), grid, dim3(kFewThreads), 0, st, k, v, dim, kbits, vbits, n_vec);
       break;
   }
   return check_launch("append_few_kernel");
@@ -320,22 +320,12 @@ int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int
 
 }  // namespace
 
-// The line between this kernel and those that share a split of R among many
-// vectors, in workgroups (16 vectors x 64 coordinates x side).  K + V, 8 heads,
-// bf16, us before -> here.  Against one paired launch: d = 64 about equal
-// (4.1-5.0 -> 4.4-4.9), so it keeps that; d = 128 8.6 -> 5.6 at 16 workgroups,
-// 10.8 -> 6.0 at 128; d = 256 8.9 -> 7.8 at 8, 11.8 -> 8.6 at 256.  Against a
-// launch a side (other width pairs): d = 64 8.4 -> 5.2 at 2, 10.2 -> 5.4 at 64;
-// d = 128 18.2 -> 6.0 at 4; d = 256 18 -> 8.2 at 8, 23.5 -> 9.0 at 256.  Against
-// the vector kernel (dims that are no 64, 128, 256), ties included: d = 96 26 ->
-// 5.2 at 4, 33 -> 21 at 2048, d = 192 43 -> 6.7 at 6, 77 -> 42 at 3072: always.
-bool append_few_path(int64_t n_vec, int dim, int sides, bool paired) {
-  if (dim % 8 != 0 || dim < 8 || dim > kFewMaxDim || n_vec >= (int64_t(1) << 31) - 16) return false;
-  const int64_t wgs = (n_vec + 15) / 16 * ((dim + kFewCoords - 1) / kFewCoords) * sides;
-  if (dim != 64 && dim != 128 && dim != 256) return true;
-  // the matrix-core kernels round their sums in their own order, so their ties
-  // fall otherwise than here: up to a verify step's vectors only
-  return n_vec <= kFewTunedVecs && (paired ? dim > 64 && wgs <= 512 : wgs <= 512 * sides);
+// Every count of vectors: K + V, 8 heads, bf16, us in the vector kernel -> here, ties
+// included: d = 96 26 -> 5.2 at 4 workgroups (16 vectors x 64 coordinates x side),
+// 33 -> 21 at 2048; d = 192 43 -> 6.7 at 6, 77 -> 42 at 3072.
+bool append_few_path(int64_t n_vec, int dim) {
+  return dim % 8 == 0 && dim >= 8 && dim <= kFewMaxDim && dim != 64 && dim != 128 && dim != 256 &&
+         n_vec < (int64_t(1) << 31) - 16;
 }
 
 int launch_append_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int kbits, int vbits, int x_dtype,

@@ -1,5 +1,5 @@
-"""The dense-rotation append of few vectors (tq_append_few.hip), keys and values
-in one call: every dim class, width pair and input type, vector counts at the
+"""The dense-rotation append at dims that are no 64, 128 or 256 (tq_append_few.hip),
+keys and values in one call, and few vectors at those dims: every dim class, width pair and input type, vector counts at the
 edges of its 16-vector groups.  Bar of test_append_general_gpu: norms bit-exact,
 indices equal to the oracle's but within its band of a midpoint (each y is a
 sum of exact piece products in f32, no longer than that band's d / 4 + 2 ulps),
@@ -37,3 +37,45 @@ def test_few_vectors_keys_and_values(device, d, kb, vb, xdt, B, H, L):
         used = d * b % 32
         if used:  # bits past the last coordinate are zero
             assert not (gp[:, :, off:off + L, -1] >> used).any()
+
+
+def midpoints_on(x, rot, rng, count, off=0):
+    """Sorted thresholds (f32) on rotated coordinates of random vectors, ``off`` f32 steps away."""
+    u = x.astype(np.float64).reshape(-1, x.shape[-1])
+    u = u / np.linalg.norm(u, axis=1, keepdims=True)
+    v, i = rng.integers(0, u.shape[0], count), rng.integers(0, u.shape[1], count)
+    y = np.einsum("cd,cd->c", u[v], rot.astype(np.float64)[i]).astype(np.float32)
+    return np.sort(y + off * np.spacing(y))
+
+
+@pytest.mark.parametrize("d", [64, 128, 256, 96])
+@pytest.mark.parametrize("xdt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("kb,vb", [(4, 4), (4, 2), (3, 4)])
+def test_words_do_not_depend_on_the_call(device, d, xdt, kb, vb):
+    """The words of a vector on a threshold are the same whether it is appended
+    with thousands of others, with few or alone, as one side or both."""
+    rng = np.random.default_rng(d + kb)
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[xdt]
+    H, L = 4, 640
+    xs = [torch.from_numpy(rng.standard_normal((1, H, L, d)).astype(np.float32)).to(dt).to(device) for _ in range(2)]
+    codecs = [ops.Codec(d, b, s, rotation="dense") for b, s in ((kb, 0), (vb, 1))]
+
+    def buffers(n):
+        return [(torch.zeros((1, H, n, c.packed_width), dtype=torch.uint32, device=device),
+                 torch.zeros((1, H, n), device=device)) for c in codecs]
+
+    for trial in range(12):
+        for c, x in zip(codecs, xs):
+            m = midpoints_on(x[:, :, :100].float().cpu().numpy(), np.array(c.rot_host), rng, (1 << c.bits) - 1)
+            c.device_tensors(x.device)["midpoints"] = torch.from_numpy(m).to(device)
+        whole = buffers(L)
+        ops.append_quantize_kv(*xs, *codecs, *whole[0], *whole[1], 0)
+        for n in (1, 7, 100):
+            part = [x[:, :, :n] for x in xs]
+            both, single = buffers(n), buffers(n)
+            ops.append_quantize_kv(*part, *codecs, *both[0], *both[1], 0)
+            for x, c, s, b, w in zip(part, codecs, single, both, whole):
+                ops.append_quantize(x, c, *s, 0)
+                for got in (s, b):
+                    assert torch.equal(got[0].view(torch.int32), w[0][:, :, :n].view(torch.int32)), (trial, n)
+                    assert torch.equal(got[1], w[1][:, :, :n])
