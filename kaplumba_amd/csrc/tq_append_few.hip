@@ -16,11 +16,11 @@
 // formed by every wave.  Indices meet in LDS for the packing.
 //
 // Ties.  Sums in another order than the vector kernel's (tq_append_general.hip)
-// may put a coordinate within an ulp of a midpoint on its other side.  Where a
-// coordinate lies within a margin of a threshold that is above both
-// kernels' rounding, its index comes from the vector kernel's own arithmetic
-// (IEEE division, four fused chains), so the two agree bit for bit: one
-// coordinate in 10^4 or fewer, a branch that a wave takes now and then.
+// may put a coordinate within some ulps of a midpoint on its other side.  Where a
+// coordinate lies within the bound of both kernels' rounding of a threshold
+// (tie_units), its index comes from the vector kernel's own arithmetic (IEEE
+// division, four fused chains), so the two agree bit for bit: one coordinate in
+// 3000 (d = 96, 4 bits), a branch that one wave in twelve takes.
 #include "tq_append.h"
 
 namespace tq {
@@ -61,10 +61,22 @@ __device__ __forceinline__ float halves_add(float x) {  // x of lanes l and l ^ 
 constexpr int kFewThreads = 256;
 constexpr int kFewCoords = 64;              // coordinates per workgroup
 constexpr int kFewMaxDim = 256;
-// Margin of a tie in ulps of 1 per unit of |x| |R_i|: a margin of one already
-// gave the vector kernel's words over 65 million coordinates of 6 dims.
-constexpr float kTieUlps = 4;
 constexpr int kFewIdxRow = kFewCoords + 4;  // bytes per vector's indices in LDS
+
+// How far the two kernels' sums of one coordinate can lie apart, in units of
+// 2^-24 |x| |R_i| (sum_k |x_k R_ik| <= |x| |R_i|).  Vector kernel: D / 4 fused adds a
+// chain, the two adds of the chains and the division, one unit each.  Here: a
+// product rounds by up to 4 units of its accumulator and terms (3.7 the largest over
+// 5e5 random and one-signed ones, and the terms count once in all), so 4 per step
+// of the main chain and 4; the other chains, 2^-8 of it, one; two adds, the
+// threshold's product and the skipped terms one each.
+constexpr float tie_units(int D, int steps) { return D / 4 + 3 + 4 * steps + 4 + 1 + 4; }
+
+// Orders a wave's own LDS accesses (the LDS serves a wave in order).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 // KS: 32-element steps that hold the dim (a multiple of 8)
 template <int KS, int XDT>
@@ -72,6 +84,7 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
                                                                 int n_vec) {
   constexpr int NX = XDT == TQ_DTYPE_BF16 ? 1 : (XDT == TQ_DTYPE_F16 ? 2 : 3);
   __shared__ __align__(16) uint8_t s_idx[16 * kFewIdxRow];
+  __shared__ uint8_t s_tie[kFewThreads / 64][256];  // per wave: vector << 4 | coordinate
   const bool key = blockIdx.z == 0;
   const AppendArgs a = select_args(key, ka, va);
   const int bits = key ? kbits : vbits;
@@ -176,7 +189,7 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
 
   // ---- products and indices: lane (coordinate n, g) holds vectors 4 g + j
   float r2 = 0.f;  // squared length of this lane's row of R
-  f32x4_t acc[3];  // one chain per piece of R
+  f32x4_t acc[3];  // one chain per order of the piece products
 #pragma unroll
   for (int p = 0; p < 3; ++p) acc[p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -191,12 +204,12 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
     for (int p = 2; p >= 0; --p)
 #pragma unroll
       for (int q = NX - 1; q >= 0; --q)
-        if (q + p <= 2) acc[p] = mfma_bf16(xp[s][q], w[p], acc[p]);
+        if (q + p <= 2) acc[q + p] = mfma_bf16(xp[s][q], w[p], acc[q + p]);
   }
   // |x . R_i| sums to at most |x| |R_i|; clamped tail pieces only add to r2
   r2 += xor_lane<16>(r2);
   r2 = halves_add(r2);
-  const float margin = kTieUlps * 0x1p-24f * __builtin_amdgcn_sqrtf(r2);
+  const float margin = tie_units(D, KS) * 0x1p-24f * __builtin_amdgcn_sqrtf(r2);
   uint32_t idx[4] = {0u, 0u, 0u, 0u};
   float y[4];
 #pragma unroll
@@ -212,57 +225,53 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
       tie[j] |= fabsf(d) <= margin * dj[j];
     }
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) s_idx[(4 * g + j) * kFewIdxRow + 16 * wave + n] = static_cast<uint8_t>(idx[j]);
   if (__any(tie[0] | tie[1] | tie[2] | tie[3])) {
-#pragma unroll 1
+    // the wave's ties as a list, then four lanes a tie, one per chain of the vector kernel
+    int ties = 0;
+#pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const bool mine = j == 0 ? tie[0] : j == 1 ? tie[1] : j == 2 ? tie[2] : tie[3];
-      if (!__any(mine)) continue;
-      const int tv = min(static_cast<int>(blockIdx.x) * 16 + 4 * g + j, n_vec - 1);
-      const int tl = tv % a.L;
-      const int tbh = tv / a.L;
-      const int64_t tx = static_cast<int64_t>(tbh / a.H) * a.sb + static_cast<int64_t>(tbh % a.H) * a.sh + tl * a.sl;
-      const float* row = a.rot + static_cast<int64_t>(min(coord, D - 1)) * D;
-      const float td = j == 0 ? dj[0] : j == 1 ? dj[1] : j == 2 ? dj[2] : dj[3];
-      float c[4] = {0.f, 0.f, 0.f, 0.f};
-      // 32 elements at a time, in whole 8-element pieces (those past D add u = 0)
+      const uint64_t set = __ballot(tie[j] ? 1 : 0);
+      const int at = ties + __builtin_popcountll(set & ((uint64_t(1) << lane) - 1));
+      if (tie[j]) s_tie[wave][at] = static_cast<uint8_t>((4 * g + j) << 4 | n);
+      ties += __builtin_popcountll(set);
+    }
+    wave_lds_order();
 #pragma unroll 1
-      for (int k0 = 0; k0 < D; k0 += 32) {
-        float u[32], r[32];
+    for (int t0 = 0; t0 < ties; t0 += 16) {
+      const int code = s_tie[wave][min(t0 + (lane >> 2), ties - 1)];
+      const int tv = code >> 4;
+      const int tn = code & 15;
+      const int gv = min(static_cast<int>(blockIdx.x) * 16 + tv, n_vec - 1);
+      const int bh = gv / a.L;
+      const int64_t tx = static_cast<int64_t>(bh / a.H) * a.sb + static_cast<int64_t>(bh % a.H) * a.sh +
+                         (gv - bh * a.L) * a.sl + (lane & 3);
+      const float* row = a.rot + static_cast<int64_t>(min(s0 + 16 * wave + tn, D - 1)) * D + (lane & 3);
+      const float td = __shfl(den, tv, 64);
+      float c = 0.f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int k = min(k0 + 8 * q, D - 8);
-          *reinterpret_cast<float4*>(r + 8 * q) = *reinterpret_cast<const float4*>(row + k);
-          *reinterpret_cast<float4*>(r + 8 * q + 4) = *reinterpret_cast<const float4*>(row + k + 4);
-          if constexpr (XDT == TQ_DTYPE_F32) {
-            const float* xs = static_cast<const float*>(a.x) + tx + k;
-            *reinterpret_cast<float4*>(u + 8 * q) = *reinterpret_cast<const float4*>(xs);
-            *reinterpret_cast<float4*>(u + 8 * q + 4) = *reinterpret_cast<const float4*>(xs + 4);
-          } else {
-            const uint4 h = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.x) + tx + k);
-            const uint32_t w[4] = {h.x, h.y, h.z, h.w};
+      for (int s = 0; s < KS; ++s) {  // 32 elements, 8 of this chain; D is a multiple of 8
+        float u[8], r[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const uint16_t b16 = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
-              u[8 * q + e] = XDT == TQ_DTYPE_F16 ? f16_bits_to_f32(b16) : bf16_bits_to_f32(b16);
-            }
-          }
+        for (int e = 0; e < 8; ++e) {
+          const int k = min(32 * s + 4 * e, D - 4);
+          u[e] = load_elem<XDT>(a.x, tx + k);
+          r[e] = row[k];
         }
-        div_by_norm<XDT>(u, td, u);
 #pragma unroll
-        for (int e = 0; e < 32; ++e)
-          if (k0 + (e & ~7) < D) c[e & 3] = __builtin_fmaf(u[e], r[e], c[e & 3]);
+        for (int e = 0; e < 8; ++e)
+          if (32 * s + 4 * e < D) c = __builtin_fmaf(__fdiv_rn(u[e], td), r[e], c);
       }
-      const float ty = __fadd_rn(__fadd_rn(c[0], c[1]), __fadd_rn(c[2], c[3]));
+      c = __fadd_rn(c, xor_lane<1>(c));
+      const float ty = __fadd_rn(c, xor_lane<2>(c));
       uint32_t ti = 0;
 #pragma unroll
       for (int m = 0; m < 15; ++m)
         if (m < nmid) ti += ty > mid[m] ? 1u : 0u;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) idx[q] = (q == j && mine) ? ti : idx[q];
+      if ((lane & 3) == 0) s_idx[tv * kFewIdxRow + 16 * wave + tn] = static_cast<uint8_t>(ti);
     }
   }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) s_idx[(4 * g + j) * kFewIdxRow + 16 * wave + n] = static_cast<uint8_t>(idx[j]);
   __syncthreads();
 
   // ---- pack: thread (vector, word); LSB-first, zeros past the last coordinate
@@ -320,9 +329,9 @@ int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int
 
 }  // namespace
 
-// Every count of vectors: K + V, 8 heads, bf16, us in the vector kernel -> here, ties
-// included: d = 96 26 -> 5.2 at 4 workgroups (16 vectors x 64 coordinates x side),
-// 33 -> 21 at 2048; d = 192 43 -> 6.7 at 6, 77 -> 42 at 3072.
+// Every count of vectors: K + V, 8 heads, bf16, 3 bits, us in the vector kernel ->
+// here, ties included (one costs its workgroup 2.5 us at d = 96, 5 at 192): d = 96
+// 26 -> 4.9 for 8 vectors a side, 33 -> 13.5 for 4096; d = 192 43 -> 6.4 and 77 -> 28.
 bool append_few_path(int64_t n_vec, int dim) {
   return dim % 8 == 0 && dim >= 8 && dim <= kFewMaxDim && dim != 64 && dim != 128 && dim != 256 &&
          n_vec < (int64_t(1) << 31) - 16;

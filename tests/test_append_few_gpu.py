@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import tq_oracle as O
 from kaplumba_amd import ops
 from tests.test_append_general_gpu import _check
 
@@ -79,3 +80,43 @@ def test_words_do_not_depend_on_the_call(device, d, xdt, kb, vb):
                 for got in (s, b):
                     assert torch.equal(got[0].view(torch.int32), w[0][:, :, :n].view(torch.int32)), (trial, n)
                     assert torch.equal(got[1], w[1][:, :, :n])
+
+
+def vector_kernel_sums(x, den, rot):
+    """y of the vector kernel (tq_append_general.hip) in its own f32 arithmetic: u = x / den, four chains of
+    fused adds (coordinates k mod 4 in order), added in pairs.  An 80-bit add of the exact product stands for
+    the fused one."""
+    u = (x / den[..., None]).astype(np.float32)
+    c = []
+    for s in range(4):
+        acc = np.zeros(u.shape[:-1] + (rot.shape[0],), np.float32)
+        for k in range(s, u.shape[-1], 4):
+            acc = (u[..., k:k + 1].astype(np.longdouble) * rot[:, k].astype(np.longdouble) + acc).astype(np.float32)
+        c.append(acc)
+    return (c[0] + c[1]) + (c[2] + c[3])
+
+
+@pytest.mark.parametrize("d", [8, 40, 96, 192, 248])
+@pytest.mark.parametrize("xdt", ["bf16", "f16", "f32"])
+def test_ties_are_the_vector_kernels(device, d, xdt):
+    """Thresholds placed on coordinates as the vector kernel computes them, and one f32 step below: every index
+    is that kernel's, bit for bit.  (Without the branch for ties about a third of the coordinates on a
+    threshold come out on the other side.)"""
+    rng = np.random.default_rng(d)
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[xdt]
+    N = 33
+    x = torch.from_numpy(rng.standard_normal((1, 1, N, d)).astype(np.float32)).to(dt).to(device)
+    codec = ops.Codec(d, 4, 0, rotation="dense")
+    p = torch.zeros((1, 1, N, codec.packed_width), dtype=torch.uint32, device=device)
+    n = torch.zeros((1, 1, N), device=device)
+    ops.append_quantize(x, codec, p, n, 0)
+    y = vector_kernel_sums(x.float().cpu().numpy()[0, 0], n.cpu().numpy()[0, 0], np.array(codec.rot_host, np.float32))
+    for trial in range(16):
+        m = np.sort(rng.choice(y.reshape(-1), 15, replace=False))
+        if trial % 2:
+            m = np.nextafter(m, np.float32(-np.inf))
+        codec.device_tensors(x.device)["midpoints"] = torch.from_numpy(m).to(device)
+        ops.append_quantize(x, codec, p, n, 0)
+        want = (y[..., None] > m).sum(-1)
+        got = O.unpack_lowbit(p.cpu().numpy().astype(np.uint32)[0, 0], 4, d)
+        assert np.array_equal(got, want), np.argwhere(got != want)[:4]
