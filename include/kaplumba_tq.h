@@ -175,7 +175,8 @@ int tq_prod_dequantize(const void* norms, const uint32_t* mse_packed, const void
 /*
  * Bytes of workspace tq_attention() / tq_attention_ranged() need for this
  * problem (split-K partials and rotated queries).  max_tokens is the largest
- * per-sequence cache length.  tq_attention_prod_workspace_size() is the same
+ * per-sequence cache length.  The size grows with B, L and max_tokens: it also
+ * serves every problem with fewer sequences, queries or tokens.  tq_attention_prod_workspace_size() is the same
  * for tq_attention_prod (its general-kernel shapes add a projected-query
  * region).
  */
@@ -279,7 +280,7 @@ int tq_attention_prod(const void* q, int q_dtype, int B, int Hq, int Hkv, int L,
 
 /*
  * Bytes of workspace tq_attention_general() needs (rotated and projected
- * queries, split partials).
+ * queries, split partials); grows with B, L and max_tokens as above.
  */
 int64_t tq_attention_general_workspace_size(int B, int Hq, int Hkv, int L, int k_dim, int v_dim,
                                             int64_t max_tokens);

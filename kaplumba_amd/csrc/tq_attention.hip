@@ -163,30 +163,46 @@ using namespace tq;
 
 namespace {
 
-// Workspace of one attention call: the larger of the tuned kernels' layout
+// Least workspace of one attention call: the larger of the tuned kernels' layout
 // (either cache kind) and the general kernels' (the shapes outside the tuned
-// ones); Prod keys add a projected-query region to the latter.
-int64_t attention_workspace_bytes(int B, int Hq, int Hkv, int L, int dim, int64_t max_tokens, bool prod,
-                                  bool without_wide = false) {
+// ones).
+int64_t attention_workspace_bytes(int B, int Hq, int Hkv, int L, int dim, int64_t max_tokens) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || dim <= 0 || max_tokens < 0 || Hq % Hkv)
     return 0;
   const int64_t T = std::max<int64_t>(max_tokens, 1);
   const int64_t tuned =
       std::max(workspace_bytes(plan_splits(B, Hq, Hkv, L, T, dim, true), B, Hq, Hkv, L, dim),
                workspace_bytes(plan_splits(B, Hq, Hkv, L, T, dim, false), B, Hq, Hkv, L, dim));
-  return std::max(tuned, general_workspace_bytes(B, Hq, Hkv, L, dim, dim, T, prod, without_wide));
+  return std::max(tuned, general_workspace_bytes(B, Hq, Hkv, L, dim, dim, T, false));
+}
+
+// Bytes with which every kernel takes this problem and every one with fewer
+// sequences, query rows or tokens; Prod keys add a projected-query region.
+int64_t attention_workspace_bound(int B, int Hq, int Hkv, int L, int dim, int64_t max_tokens, bool prod) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || dim <= 0 || max_tokens < 0 || Hq % Hkv)
+    return 0;
+  const int64_t T = std::max<int64_t>(max_tokens, 1);
+  // plan_splits: ceil(target / base) splits of base row groups, fewer for few
+  // tokens, more where a chunk is at its largest
+  SplitPlan sp = plan_splits(B, Hq, Hkv, L, T, dim, true);
+  const int64_t base = static_cast<int64_t>(B) * Hkv * sp.n_rg;
+  const int64_t parts = std::max(std::min(base * ((T + 255) / 256), base + device_cu_count()),
+                                 base * ((T + kMaxChunk - 1) / kMaxChunk)) * sp.nq;
+  const int64_t rows = static_cast<int64_t>(B) * Hq * L;
+  const int64_t tuned = align256(rows * dim * 4) + align256(parts * dim * 4) + align256(parts * 2 * 4);
+  return std::max(tuned, general_workspace_bound(B, Hq, Hkv, L, dim, dim, T, prod));
 }
 
 }  // namespace
 
 extern "C" int64_t tq_attention_workspace_size(int B, int Hq, int Hkv, int L, int dim,
                                                int64_t max_tokens) {
-  return attention_workspace_bytes(B, Hq, Hkv, L, dim, max_tokens, false);
+  return attention_workspace_bound(B, Hq, Hkv, L, dim, max_tokens, false);
 }
 
 extern "C" int64_t tq_attention_prod_workspace_size(int B, int Hq, int Hkv, int L, int dim,
                                                     int64_t max_tokens) {
-  return attention_workspace_bytes(B, Hq, Hkv, L, dim, max_tokens, true);
+  return attention_workspace_bound(B, Hq, Hkv, L, dim, max_tokens, true);
 }
 
 namespace {
@@ -530,7 +546,7 @@ extern "C" int tq_attention_noalloc(const void* q, int q_dtype, int B, int Hq, i
                 B, Hq, Hkv, L, dim);
   if (B == 0) return TQ_OK;
   // the wide kernel runs where its own need fits too; no problem is refused for it
-  const int64_t need = attention_workspace_bytes(B, Hq, Hkv, L, dim, max_tokens, false, true);
+  const int64_t need = attention_workspace_bytes(B, Hq, Hkv, L, dim, max_tokens);
   if (need > kScratchBytes)
     return fail(TQ_ERR_WORKSPACE, "attention (no-alloc): the problem needs %lld bytes of scratch, "
                 "above the static %lld; use tq_attention with a caller workspace",

@@ -114,12 +114,15 @@ bool tile_rows_path(int kv_kind, int Dk, int Dv, int rows);
 constexpr int kWideMinRows = 64;
 bool wide_rows_path(int kv_kind, int Dk, int Dv, int rows);
 
-// Workspace bytes of the general path for this problem, whichever of its
-// kernels runs; without_wide: of the kernels before the wide one, which takes
-// a call only where its own need fits (callers with fixed scratch keep every
-// problem they had).
+// Workspace bytes of the general path's kernels before the wide and narrow ones,
+// which take a call only where their own need fits: the least a call must bring.
 int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T,
-                                bool prod, bool without_wide = false);
+                                bool prod);
+
+// Bytes with which every kernel of the general path takes this problem and every
+// smaller one (fewer sequences, query rows or tokens).
+int64_t general_workspace_bound(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T,
+                                bool prod);
 
 // Arguments of one general attention call (validated by general_attention).
 struct GenCall {

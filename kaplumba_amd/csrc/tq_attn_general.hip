@@ -808,6 +808,17 @@ GenPlan tile_plan(int B, int Hq, int Hkv, int L, int64_t T) {
 // 4 TB/s).  Microseconds per token measured on the prefill shapes.
 constexpr int kWideMaxSplits = 32;
 constexpr int kNarrowMaxSplits = 64;
+// Bytes of split partials that a plan may take beyond those of one split: eight
+// rounds of workgroups over the chip (256 wide ones of 128 KiB each, or narrow ones
+// of 16 KiB).  Only calls of more rows than that feel it; with it the workspace
+// sizes grow with the problem (general_workspace_bound).
+constexpr int64_t kWideSplitBytes = int64_t(256) << 20;
+constexpr int64_t kNarrowSplitBytes = int64_t(32) << 20;
+
+int64_t split_bytes(int B, int Hkv, int n_rg, int Dv) {  // (o, m, l) of one split
+  return static_cast<int64_t>(B) * Hkv * n_rg * kGenNQ * (Dv + 2) * 4;
+}
+constexpr int kWideMinTokens = 32, kNarrowMinTokens = 128;  // of a split, where there are several
 constexpr double kNarrowTokenUs = 2.5e-5;  // per token and padded dim of one workgroup
 
 GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
@@ -823,7 +834,9 @@ GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   const double merge_us = static_cast<double>(B) * Hq * L * Dv * 8 / 4e6;  // per split
   int64_t best = 1;
   double best_cost = 0;
-  for (int64_t ns = 1; ns <= kWideMaxSplits && (ns == 1 || (T + ns - 1) / ns >= 32); ++ns) {
+  const int64_t one = split_bytes(B, Hkv, gp.n_rg, Dv);
+  for (int64_t ns = 1; ns <= kWideMaxSplits && (ns == 1 || ((T + ns - 1) / ns >= kWideMinTokens && ns * one <= kWideSplitBytes));
+       ++ns) {
     const double cost =
         static_cast<double>((blocks * ns + cus - 1) / cus) * (static_cast<double>((T + ns - 1) / ns) * token_us + 8) +
         static_cast<double>(ns) * merge_us;
@@ -851,7 +864,9 @@ GenPlan narrow_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   const double merge_us = static_cast<double>(B) * Hq * L * Dv * 8 / 4e6;  // per split
   int64_t best = 1;
   double best_cost = 0;
-  for (int64_t ns = 1; ns <= kNarrowMaxSplits && (ns == 1 || (T + ns - 1) / ns >= 128); ++ns) {
+  const int64_t one = split_bytes(B, Hkv, gp.n_rg, Dv);
+  for (int64_t ns = 1;
+       ns <= kNarrowMaxSplits && (ns == 1 || ((T + ns - 1) / ns >= kNarrowMinTokens && ns * one <= kNarrowSplitBytes)); ++ns) {
     const double cost =
         static_cast<double>((blocks * ns + cus - 1) / cus) * (static_cast<double>((T + ns - 1) / ns) * token_us + 6) +
         static_cast<double>(ns) * merge_us;
@@ -1132,16 +1147,9 @@ bool wide_call(const GenCall& c) {
   return mfma_operands(c) && mfma_fits(c, wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T));
 }
 
-int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod,
-                                bool without_wide) {
+int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || Dk <= 0 || Dv <= 0 || Hq % Hkv) return 0;
   T = std::max<int64_t>(T, 1);
-  int64_t wide = 0;
-  int ks = 0, ct = 0;
-  if (!without_wide && wide_dims(Dk, Dv, ks, ct))
-    wide = wide_layout(B, Hq, Hkv, L, Dk, Dv, narrow_plan(B, Hq, Hkv, L, Dk, Dv, T), true, true).bytes;
-  if (!without_wide && wide_rows_path(TQ_KV_PACKED, Dk, Dv, (Hq / Hkv) * L))
-    wide = std::max(wide, wide_layout(B, Hq, Hkv, L, Dk, Dv, wide_plan(B, Hq, Hkv, L, Dk, Dv, T), true, true).bytes);
   GenPlan gp = gen_plan(B, Hq, Hkv, L, T);
   const int64_t rows = static_cast<int64_t>(B) * Hq * L;
   int64_t tile_q = 0;  // the tile kernel's prepared query rows
@@ -1151,9 +1159,45 @@ int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, i
     tile_q = a256(rows * Dk * 4) + a256(rows * 4);
   }
   const int64_t groups = static_cast<int64_t>(B) * Hkv * gp.n_rg;
-  return std::max(wide, a256(rows * round32(Dk) * 4) * (prod ? 2 : 1) +
-                            a256(groups * gp.n_splits * kGenNQ * static_cast<int64_t>(Dv) * 4) +
-                            a256(groups * gp.n_splits * kGenNQ * 2 * 4) + tile_q);
+  return a256(rows * round32(Dk) * 4) * (prod ? 2 : 1) +
+         a256(groups * gp.n_splits * kGenNQ * static_cast<int64_t>(Dv) * 4) +
+         a256(groups * gp.n_splits * kGenNQ * 2 * 4) + tile_q;
+}
+
+// A bound of what any kernel of the general path needs for a problem, that grows
+// with B, L and T.  The plans do not: a plan takes fewer splits, and may need less,
+// for more rows (ceil(target / groups) splits of groups: at most target + groups).
+int64_t general_workspace_bound(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || Dk <= 0 || Dv <= 0 || Hq % Hkv) return 0;
+  T = std::max<int64_t>(T, 1);
+  const int64_t rows = static_cast<int64_t>(B) * Hq * L;
+  const int64_t n_rg = (static_cast<int64_t>(Hq / Hkv) * L + kGenNQ - 1) / kGenNQ;
+  const int64_t groups = static_cast<int64_t>(B) * Hkv * n_rg;
+  const int64_t cus = device_cu_count();
+  int64_t parts = std::min(groups * ((T + 127) / 128), groups + 2 * cus);  // gen_plan
+  int64_t tile_q = 0;
+  if (tile_rows_path(TQ_KV_PACKED, Dk, Dv, (Hq / Hkv) * L)) {  // tile_plan: of blocks of groups
+    parts = std::max(parts, std::min(groups * ((T + 255) / 256), groups + kTileRows / kGenNQ * cus));
+    tile_q = a256(rows * Dk * 4) + a256(rows * 4);
+  }
+  int64_t need = a256(rows * round32(Dk) * 4) * (prod ? 2 : 1) + a256(parts * kGenNQ * static_cast<int64_t>(Dv) * 4) +
+                 a256(parts * kGenNQ * 2 * 4) + tile_q;
+  int ks = 0, ct = 0;
+  if (wide_dims(Dk, Dv, ks, ct)) {
+    // the most partials either plan takes: splits by the tokens, or the bytes of all
+    const int64_t one = groups * kGenNQ * (Dv + 2) * 4;
+    auto most = [&](int64_t splits, int64_t least_tokens, int64_t bytes) {
+      const int64_t ns = std::min(splits, (T + least_tokens - 2) / (least_tokens - 1));
+      return std::min(ns * one, std::max(one, bytes));
+    };
+    int64_t partials = most(kNarrowMaxSplits, kNarrowMinTokens, kNarrowSplitBytes);
+    if (wide_rows_path(TQ_KV_PACKED, Dk, Dv, (Hq / Hkv) * L))
+      partials = std::max(partials, most(kWideMaxSplits, kWideMinTokens, kWideSplitBytes));
+    GenPlan none{};
+    none.n_rg = static_cast<int>(n_rg);
+    need = std::max(need, wide_layout(B, Hq, Hkv, L, Dk, Dv, none, true, true).bytes + partials + 512);
+  }
+  return need;
 }
 
 int general_attention(const GenCall& c) {
@@ -1226,7 +1270,7 @@ int general_attention(const GenCall& c) {
   const WideLayout wl =
       wide ? wide_layout(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, gp, !plain, c.mask_kind != TQ_MASK_NONE) : WideLayout{};
   const int64_t need =
-      wide ? wl.bytes : general_workspace_bytes(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T, prod, true);
+      wide ? wl.bytes : general_workspace_bytes(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T, prod);
   if (c.workspace_bytes < need)
     return fail(TQ_ERR_WORKSPACE, "attention: workspace %lld < %lld bytes", (long long)c.workspace_bytes,
                 (long long)need);
@@ -1394,7 +1438,7 @@ using namespace tq;
 extern "C" int64_t tq_attention_general_workspace_size(int B, int Hq, int Hkv, int L, int k_dim,
                                                        int v_dim, int64_t max_tokens) {
   if (max_tokens < 0) return 0;
-  return general_workspace_bytes(B, Hq, Hkv, L, k_dim, v_dim, max_tokens, true);
+  return general_workspace_bound(B, Hq, Hkv, L, k_dim, v_dim, max_tokens, true);
 }
 
 extern "C" int tq_attention_general(

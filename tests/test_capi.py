@@ -7,6 +7,7 @@ import ctypes
 import os
 import re
 
+import numpy as np
 import pytest
 
 from kaplumba_amd import _lib
@@ -97,6 +98,24 @@ def test_attention_rejects_kv_heads_beyond_the_small_rows_field():
             fake, fake, 0, fake, fake, 16, 0, None, 0, fake, fake, 1 << 30, None]
     assert lib.tq_attention(*args) == _lib.TQ_ERR_UNSUPPORTED
     assert b"kv heads" in lib.tq_last_error()
+
+
+def test_a_workspace_serves_every_smaller_problem():
+    # ops.reserve_workspace sizes it once for the largest problem: decode, verify and
+    # prefill shapes with fewer sequences, queries or tokens ask for no more
+    lib = _lib.load()
+    rng = np.random.default_rng(0)
+    log = lambda lo, hi: int(round(np.exp(rng.uniform(np.log(lo), np.log(hi)))))  # noqa: E731
+    for Hq, Hkv, D in ((16, 8, 256), (32, 8, 64), (32, 8, 128), (32, 8, 96), (8, 1, 128), (28, 4, 192), (4, 4, 512)):
+        for _ in range(300):
+            B, L, T = log(1, 64), log(1, 1024), log(1, 200000)
+            b, l, t = log(1, B), log(1, L), log(1, T)
+            for size in (lib.tq_attention_workspace_size, lib.tq_attention_prod_workspace_size):
+                assert size(b, Hq, Hkv, l, D, t) <= size(B, Hq, Hkv, L, D, T), (Hq, Hkv, D, B, L, T, b, l, t)
+            general = lib.tq_attention_general_workspace_size
+            assert general(b, Hq, Hkv, l, D, 64, t) <= general(B, Hq, Hkv, L, D, 64, T)
+            # a masked call of the same dims keeps to the size of the plain one
+            assert general(b, Hq, Hkv, l, D, D, t) <= lib.tq_attention_prod_workspace_size(B, Hq, Hkv, L, D, T)
 
 
 def test_workspace_growth_keeps_retired_buffers_bounded():
