@@ -334,14 +334,16 @@ int tq_attention_general(const void* q, int q_dtype, int B, int Hq, int Hkv, int
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference, which
  * never exposes a workspace.  The split partials and rotated queries live in
- * a static device array of TQ_NOALLOC_SCRATCH_BYTES per GPU, held until the
- * process ends; the entry point calls no hipMalloc / hipFree.  Problems whose
- * tq_attention_workspace_size() exceeds that size return TQ_ERR_WORKSPACE
- * (use tq_attention with a caller workspace).  Every call on one GPU shares
+ * a static device array of 64 MiB per GPU, held until the process ends; the
+ * entry point calls no hipMalloc / hipFree.  Every problem whose
+ * tq_attention_workspace_size() is at most TQ_NOALLOC_SCRATCH_BYTES is taken, and
+ * any larger one whose rotated queries and split partials in the tuned and
+ * vector kernels fit that size; the others return TQ_ERR_WORKSPACE (use
+ * tq_attention with a caller workspace).  Every call on one GPU shares
  * the array: calls that overlap on that GPU (other streams, other host
  * threads) race.  No initial contents are needed: a call writes every
  * scratch byte it reads.  Every other argument and the results are those of
- * tq_attention_ranged.
+ * tq_attention_ranged with a workspace of tq_attention_workspace_size() bytes.
  */
 #define TQ_NOALLOC_SCRATCH_BYTES (16ll << 20)
 int tq_attention_noalloc(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, int dim,

@@ -116,7 +116,7 @@ SIGNATURES = {
         c_void_p, c_void_p, c_int64, c_void_p]),               # out, workspace, ws bytes, stream
 }
 
-# Scratch bytes of tq_attention_noalloc (TQ_NOALLOC_SCRATCH_BYTES in the header).
+# Scratch bytes up to which tq_attention_noalloc takes every problem (TQ_NOALLOC_SCRATCH_BYTES in the header).
 TQ_NOALLOC_SCRATCH_BYTES = 16 << 20
 
 

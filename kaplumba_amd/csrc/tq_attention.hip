@@ -215,6 +215,21 @@ struct ProdKeys {
   const float* proj;
 };
 
+// The kernels that serve a call of the one-dim entry points: the general ones for
+// shapes outside the tuned kernels (other head dims; Prod keys beyond d <= 128 and 4
+// rows per kv head, or 1-bit Prod) and where the tile or wide kernel takes many
+// rows (a wide call whose types or workspace do not suit runs the tuned kernels).
+AttnPath attention_path(const GenCall& c) {
+  const bool prod = c.kv_kind == TQ_KV_PROD;
+  const int64_t rows = static_cast<int64_t>(c.Hq / c.Hkv) * c.L;
+  const bool tuned_dim = c.Dk == 64 || c.Dk == 128 || c.Dk == 256;
+  const bool prod_small = prod && c.Dk <= 128 && rows <= 4 && c.k_bits >= 2;
+  if (!tuned_dim || (prod && !prod_small)) return general_path(c);
+  if (!prod && tile_rows_path(c.kv_kind, c.Dk, c.Dk, (c.Hq / c.Hkv) * c.L)) return general_path(c);
+  if (!prod && wide_rows_path(c.kv_kind, c.Dk, c.Dk, (c.Hq / c.Hkv) * c.L) && general_path(c) == kPathWide) return kPathWide;
+  return kPathTuned;
+}
+
 int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, int dim,
                    int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_l, float scale,
                    int kv_kind, int kv_dtype, const void* k, const void* k_norms, const void* v,
@@ -226,13 +241,8 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
                    const ProdKeys* prod) {
   if (B < 0 || Hq <= 0 || Hkv <= 0 || L < 1 || Hq % Hkv)
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: bad heads/L (Hq %d, Hkv %d, L %d)", Hq, Hkv, L);
-  // Shapes outside the tuned kernels (other head dims; Prod keys beyond
-  // d <= 128 and 4 rows per kv head, or 1-bit Prod) run the general kernels.
-  const bool tuned_dim = dim == 64 || dim == 128 || dim == 256;
-  const bool prod_small = prod && dim <= 128 && static_cast<int64_t>(Hq / Hkv) * L <= 4 && k_bits >= 1;
-  const bool tile = !prod && tile_rows_path(kv_kind, dim, dim, (Hq / Hkv) * L);
-  const bool wide = !prod && wide_rows_path(kv_kind, dim, dim, (Hq / Hkv) * L);
-  if (!tuned_dim || (prod && !prod_small) || tile || wide) {
+  const bool many_rows = static_cast<int64_t>(Hq / Hkv) * L >= std::min(kTileMinRows, kWideMinRows);
+  if ((dim != 64 && dim != 128 && dim != 256) || prod || many_rows) {
     GenCall c{};
     c.q = q;
     c.q_dtype = q_dtype;
@@ -274,8 +284,7 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
     c.workspace = workspace;
     c.workspace_bytes = workspace_bytes_given;
     c.stream = stream;
-    // a wide call whose types or workspace do not suit runs the tuned kernels
-    if (!tuned_dim || (prod && !prod_small) || tile || wide_call(c)) return general_attention(c);
+    if (attention_path(c) != kPathTuned) return general_attention(c);
   }
   if (q_dtype != TQ_DTYPE_F32 && q_dtype != TQ_DTYPE_F16 && q_dtype != TQ_DTYPE_BF16)
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: q_dtype %d", q_dtype);
@@ -495,6 +504,40 @@ extern "C" int tq_attention(const void* q, int q_dtype, int B, int Hq, int Hkv, 
                              workspace_bytes_given, stream);
 }
 
+// The path of a call as an AttnPath value, for tests of the routing rules: caches and
+// queries 16-byte aligned, T tokens of capacity, workspace bytes as given; -1 where
+// that is too small for every kernel.  Host arithmetic only.
+extern "C" int tq_attention_path(int kv_kind, int q_dtype, int kv_dtype, int B, int Hq, int Hkv, int L, int k_dim,
+                                 int v_dim, int k_rot_kind, int v_rot_kind, int mask_kind, int64_t T,
+                                 int64_t workspace) {
+  if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || L <= 0 || T < 0) return -1;
+  GenCall c{};
+  c.kv_kind = kv_kind;
+  c.q_dtype = q_dtype;
+  c.kv_dtype = kv_dtype;
+  c.B = B;
+  c.Hq = Hq;
+  c.Hkv = Hkv;
+  c.L = L;
+  c.Dk = k_dim;
+  c.Dv = v_dim;
+  c.k_rot_kind = k_rot_kind;
+  c.v_rot_kind = v_rot_kind;
+  c.k_bits = 3;
+  c.mask_kind = mask_kind;
+  c.capacity = c.max_tokens = T;
+  c.workspace_bytes = workspace;
+  const bool one_dim = mask_kind == TQ_MASK_NONE && k_dim == v_dim && k_rot_kind == v_rot_kind;
+  const AttnPath path = one_dim ? attention_path(c) : general_path(c);
+  const int64_t tokens = std::max<int64_t>(T, 1);
+  int64_t need = 0;
+  if (path == kPathTuned)
+    need = workspace_bytes(plan_splits(B, Hq, Hkv, L, tokens, k_dim, kv_kind == TQ_KV_PACKED), B, Hq, Hkv, L, k_dim);
+  else if (path == kPathTile || path == kPathVector)
+    need = general_workspace_bytes(B, Hq, Hkv, L, k_dim, v_dim, tokens, kv_kind == TQ_KV_PROD);
+  return workspace < need ? -1 : path;
+}
+
 // ------------------------------------------------------------ no-alloc ----
 // Attention scratch for callers that cannot allocate (graph capture, serving
 // loops).  Each device holds its own copy of this array for the life of the
@@ -503,9 +546,8 @@ extern "C" int tq_attention(const void* q, int q_dtype, int B, int Hq, int Hkv, 
 // hipGetSymbolAddress instead.
 namespace {
 
-constexpr int64_t kScratchBytes = TQ_NOALLOC_SCRATCH_BYTES;
 constexpr int kMaxScratchDevices = 64;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kNoallocArrayBytes];
 
 std::mutex g_scratch_mutex;
 void* g_scratch_ptr[kMaxScratchDevices] = {};
@@ -545,19 +587,19 @@ extern "C" int tq_attention_noalloc(const void* q, int q_dtype, int B, int Hq, i
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention (no-alloc): bad shape (B %d, Hq %d, Hkv %d, L %d, dim %d)",
                 B, Hq, Hkv, L, dim);
   if (B == 0) return TQ_OK;
-  // the wide kernel runs where its own need fits too; no problem is refused for it
+  // by the need of the kernels before the wide and narrow ones, which keep to the array
   const int64_t need = attention_workspace_bytes(B, Hq, Hkv, L, dim, max_tokens);
-  if (need > kScratchBytes)
+  if (need > TQ_NOALLOC_SCRATCH_BYTES)
     return fail(TQ_ERR_WORKSPACE, "attention (no-alloc): the problem needs %lld bytes of scratch, "
-                "above the static %lld; use tq_attention with a caller workspace",
-                (long long)need, (long long)kScratchBytes);
+                "above the limit of %lld; use tq_attention with a caller workspace",
+                (long long)need, (long long)TQ_NOALLOC_SCRATCH_BYTES);
   void* ws = nullptr;
   const int rc = scratch_for_current_device(&ws);
   if (rc) return rc;
   return tq_attention_ranged(q, q_dtype, B, Hq, Hkv, L, dim, q_stride_b, q_stride_h, q_stride_l,
                              scale, kv_kind, kv_dtype, k, k_norms, v, v_norms, norm_dtype, k_bits,
                              v_bits, k_codebook, v_codebook, rot_kind, k_rot, v_rot, capacity,
-                             max_tokens, seq_starts, seq_lens, causal, out, ws, kScratchBytes, stream);
+                             max_tokens, seq_starts, seq_lens, causal, out, ws, kNoallocArrayBytes, stream);
 }
 
 extern "C" int tq_attention_prod(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, int dim,

@@ -119,6 +119,15 @@ bool wide_rows_path(int kv_kind, int Dk, int Dv, int rows);
 int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T,
                                 bool prod);
 
+// Scratch of tq_attention_noalloc.  It takes problems that need at most
+// TQ_NOALLOC_SCRATCH_BYTES in the kernels before the wide and narrow ones, and for
+// those the plans of the latter keep to this array: which kernel and how many
+// splits depend on the problem alone, so the results are those of
+// tq_attention_ranged with a full workspace.  (The largest such problems take 43
+// MiB with one split at d = 8, 25 at the usual dims; four splits, one workgroup
+// per CU, fit in 64.)
+constexpr int64_t kNoallocArrayBytes = int64_t(64) << 20;
+
 // Bytes with which every kernel of the general path takes this problem and every
 // smaller one (fewer sequences, query rows or tokens).
 int64_t general_workspace_bound(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T,
@@ -162,9 +171,9 @@ struct GenCall {
 
 int general_attention(const GenCall& c);
 
-// Whether general_attention would run the wide kernel for this call (shape,
-// types, alignment, workspace).
-bool wide_call(const GenCall& c);
+// The kernels that serve an attention call (shape, types, alignment, workspace).
+enum AttnPath { kPathTuned = 0, kPathTile, kPathWide, kPathNarrow, kPathVector };
+AttnPath general_path(const GenCall& c);
 int launch_wide_packed(const GenParams& p, bool f32_weights, hipStream_t st);
 int launch_wide_f16(const GenParams& p, bool f32_weights, hipStream_t st);
 int launch_wide_bf16(const GenParams& p, bool f32_weights, hipStream_t st);

@@ -821,6 +821,8 @@ int64_t split_bytes(int B, int Hkv, int n_rg, int Dv) {  // (o, m, l) of one spl
 constexpr int kWideMinTokens = 32, kNarrowMinTokens = 128;  // of a split, where there are several
 constexpr double kNarrowTokenUs = 2.5e-5;  // per token and padded dim of one workgroup
 
+int64_t scratch_splits(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, int n_rg);
+
 GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   GenPlan gp{};
   int ks = 0, ct = 0;
@@ -834,9 +836,9 @@ GenPlan wide_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   const double merge_us = static_cast<double>(B) * Hq * L * Dv * 8 / 4e6;  // per split
   int64_t best = 1;
   double best_cost = 0;
+  const int64_t most = std::min<int64_t>(kWideMaxSplits, scratch_splits(B, Hq, Hkv, L, Dk, Dv, T, gp.n_rg));
   const int64_t one = split_bytes(B, Hkv, gp.n_rg, Dv);
-  for (int64_t ns = 1; ns <= kWideMaxSplits && (ns == 1 || ((T + ns - 1) / ns >= kWideMinTokens && ns * one <= kWideSplitBytes));
-       ++ns) {
+  for (int64_t ns = 1; ns == 1 || (ns <= most && (T + ns - 1) / ns >= kWideMinTokens && ns * one <= kWideSplitBytes); ++ns) {
     const double cost =
         static_cast<double>((blocks * ns + cus - 1) / cus) * (static_cast<double>((T + ns - 1) / ns) * token_us + 8) +
         static_cast<double>(ns) * merge_us;
@@ -864,9 +866,9 @@ GenPlan narrow_plan(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T) {
   const double merge_us = static_cast<double>(B) * Hq * L * Dv * 8 / 4e6;  // per split
   int64_t best = 1;
   double best_cost = 0;
+  const int64_t most = std::min<int64_t>(kNarrowMaxSplits, scratch_splits(B, Hq, Hkv, L, Dk, Dv, T, gp.n_rg));
   const int64_t one = split_bytes(B, Hkv, gp.n_rg, Dv);
-  for (int64_t ns = 1;
-       ns <= kNarrowMaxSplits && (ns == 1 || ((T + ns - 1) / ns >= kNarrowMinTokens && ns * one <= kNarrowSplitBytes)); ++ns) {
+  for (int64_t ns = 1; ns == 1 || (ns <= most && (T + ns - 1) / ns >= kNarrowMinTokens && ns * one <= kNarrowSplitBytes); ++ns) {
     const double cost =
         static_cast<double>((blocks * ns + cus - 1) / cus) * (static_cast<double>((T + ns - 1) / ns) * token_us + 6) +
         static_cast<double>(ns) * merge_us;
@@ -898,6 +900,16 @@ WideLayout wide_layout(int B, int Hq, int Hkv, int L, int Dk, int Dv, const GenP
   w.mrange = w.qsq + (packed ? a256(rows * 4) : 0);
   w.bytes = w.mrange + (mask ? a256(rows * 8) : 0);
   return w;
+}
+
+// Splits of a wide or narrow plan that fit tq_attention_noalloc's array, where that
+// entry point takes the problem; all of them where it does not.
+int64_t scratch_splits(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, int n_rg) {
+  if (general_workspace_bytes(B, Hq, Hkv, L, Dk, Dv, T, false) > TQ_NOALLOC_SCRATCH_BYTES) return INT32_MAX;
+  GenPlan none{};
+  none.n_rg = n_rg;
+  const int64_t rest = kNoallocArrayBytes - 512 - wide_layout(B, Hq, Hkv, L, Dk, Dv, none, true, false).bytes;
+  return rest / split_bytes(B, Hkv, n_rg, Dv);
 }
 
 // Hadamard queries that wide_qprep_kernel rotates itself (its lanes hold whole padded rows)
@@ -1139,12 +1151,20 @@ bool wide_pays(const GenCall& c) {
   return work >= (masked ? (rows < 8192 ? 16 : 4) : 8);
 }
 
-bool wide_call(const GenCall& c) {
+static bool wide_call(const GenCall& c) {
   const int rows = (c.Hq / c.Hkv) * c.L;
   if (!wide_rows_path(c.kv_kind, c.Dk, c.Dv, rows) || !wide_pays(c)) return false;
   if (c.mask_kind == TQ_MASK_NONE && tile_rows_path(c.kv_kind, c.Dk, c.Dv, rows)) return false;
   const int64_t T = std::max<int64_t>(c.max_tokens, 1);
   return mfma_operands(c) && mfma_fits(c, wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T));
+}
+
+AttnPath general_path(const GenCall& c) {
+  if (c.kv_kind == TQ_KV_PACKED && c.mask_kind == TQ_MASK_NONE && tile_rows_path(c.kv_kind, c.Dk, c.Dv, (c.Hq / c.Hkv) * c.L) &&
+      static_cast<int64_t>(c.B) * c.Hq * c.L < (int64_t(1) << 30))
+    return kPathTile;
+  if (wide_call(c)) return kPathWide;
+  return narrow_call(c) ? kPathNarrow : kPathVector;
 }
 
 int64_t general_workspace_bytes(int B, int Hq, int Hkv, int L, int Dk, int Dv, int64_t T, bool prod) {
@@ -1255,11 +1275,10 @@ int general_attention(const GenCall& c) {
   if (c.max_tokens > 0 && (!c.v || (!c.k && !(prod && kb == 0))))
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: null cache pointer");
   const int64_t T = std::max<int64_t>(c.max_tokens, 1);
-  const bool tile = c.kv_kind == TQ_KV_PACKED && c.mask_kind == TQ_MASK_NONE &&
-                    tile_rows_path(c.kv_kind, c.Dk, c.Dv, (c.Hq / c.Hkv) * c.L) &&
-                    static_cast<int64_t>(c.B) * c.Hq * c.L < (int64_t(1) << 30);
-  const bool narrow = !tile && !wide_call(c) && narrow_call(c);
-  const bool wide = narrow || wide_call(c);  // either matrix-core kernel: they share layout and preparation
+  const AttnPath path = general_path(c);
+  const bool tile = path == kPathTile;
+  const bool narrow = path == kPathNarrow;
+  const bool wide = narrow || path == kPathWide;  // either matrix-core kernel: they share layout and preparation
   const GenPlan gp = narrow ? narrow_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T)
                      : wide ? wide_plan(c.B, c.Hq, c.Hkv, c.L, c.Dk, c.Dv, T)
                      : tile ? tile_plan(c.B, c.Hq, c.Hkv, c.L, T)

@@ -14,6 +14,7 @@ import pytest
 import torch
 
 from kaplumba_amd import _lib, ops
+from tests import attention_paths as paths
 from tests.test_attention_gpu import build_case, q_tensor, to_buffers
 
 pytestmark = pytest.mark.gpu
@@ -80,6 +81,20 @@ def test_noalloc_verify_dense_and_left_padding(device):
     assert torch.equal(a, b)
     q2, kv2, kc2, vc2 = _problem(device, 4, 1, 32, 8, 4, 5000, 128, 2, 1)
     a, b = _both(device, q2, kv2, kc2, vc2, causal=True)
+    assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,T,d,rot,kernel", [
+    (1, 32, 8, 250, 5200, 64, "hadamard", paths.WIDE),      # 32 blocks of rows, 8 splits
+    (1, 16, 8, 130, 4100, 256, "dense", paths.WIDE),
+    (1, 32, 8, 64, 9000, 96, "dense", paths.WIDE),
+    (8, 32, 8, 1, 6000, 96, "dense", paths.NARROW),
+    (1, 32, 8, 40, 700, 128, "hadamard", paths.TILE)])
+def test_noalloc_matches_on_the_matrix_core_kernels(device, B, Hq, Hkv, L, T, d, rot, kernel):
+    """Calls whose split partials pass the 16 MiB that decide what is taken, too."""
+    assert paths.path(B, Hq, Hkv, L, T, d, k_rot=rot) == kernel
+    q, kv, kc, vc = _problem(device, 5, B, Hq, Hkv, L, T, d, 4, 2, rot=rot)
+    a, b = _both(device, q, kv, kc, vc, causal=L > 1)
     assert torch.equal(a, b)
 
 
