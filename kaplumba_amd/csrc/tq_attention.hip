@@ -242,8 +242,9 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
   if (B < 0 || Hq <= 0 || Hkv <= 0 || L < 1 || Hq % Hkv)
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: bad heads/L (Hq %d, Hkv %d, L %d)", Hq, Hkv, L);
   const bool many_rows = static_cast<int64_t>(Hq / Hkv) * L >= std::min(kTileMinRows, kWideMinRows);
+  GenCall c{};
+  AttnPath path = kPathTuned;
   if ((dim != 64 && dim != 128 && dim != 256) || prod || many_rows) {
-    GenCall c{};
     c.q = q;
     c.q_dtype = q_dtype;
     c.B = B;
@@ -284,7 +285,9 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
     c.workspace = workspace;
     c.workspace_bytes = workspace_bytes_given;
     c.stream = stream;
-    if (attention_path(c) != kPathTuned) return general_attention(c);
+    path = attention_path(c);
+    // (a wide call of a tuned dim keeps the limits of the tuned kernels: below)
+    if (path != kPathTuned && (path != kPathWide || (dim != 64 && dim != 128 && dim != 256))) return general_attention(c);
   }
   if (q_dtype != TQ_DTYPE_F32 && q_dtype != TQ_DTYPE_F16 && q_dtype != TQ_DTYPE_BF16)
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: q_dtype %d", q_dtype);
@@ -348,6 +351,7 @@ int attention_impl(const void* q, int q_dtype, int B, int Hq, int Hkv, int L, in
                 (long long)workspace_bytes_given, (long long)need);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
     return fail(TQ_ERR_INVALID_ARGUMENT, "attention: workspace must be 256-byte aligned");
+  if (path == kPathWide) return general_attention(c);
 
   AttnParams p{};
   p.q = q;

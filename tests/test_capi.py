@@ -148,6 +148,19 @@ def _general_args(**kw):
     return list(a.values())
 
 
+def test_many_query_rows_keep_the_limits():
+    """What the tuned kernels refuse is refused at every number of query rows, also where the wide kernel serves
+    the call."""
+    lib = _lib.load()
+    fake = ctypes.c_void_p(256)
+    for L in (1, 512):
+        for dim, cap in ((64, 40_000_000), (256, 9_000_000)):  # a kv head's row of plain keys above 4 GiB
+            rc = lib.tq_attention(None, _lib.TQ_DTYPE_BF16, 1, 32, 8, L, dim, 0, 0, 0, 0.1, _lib.TQ_KV_PLAIN,
+                                  _lib.TQ_DTYPE_BF16, fake, None, fake, None, 0, 0, 0, None, None, 0, None, None,
+                                  cap, 8192, None, 1, None, None, 1 << 40, None)
+            assert rc == _lib.TQ_ERR_UNSUPPORTED and b"4 GiB" in lib.tq_last_error(), (L, dim, lib.tq_last_error())
+
+
 def test_general_attention_validates_without_the_gpu():
     lib = _lib.load()
     fake = ctypes.c_void_p(16)
