@@ -266,9 +266,7 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     (see _RETIRED_WORKSPACES); ``reserve_workspace`` sizes it once before
     graph capture.
     """
-    stream = (torch.cuda.current_stream(device).cuda_stream if device.index is None
-              else torch._C._cuda_getCurrentRawStream(device.index))
-    key = (device, stream)
+    key = (device, torch._C._cuda_getCurrentRawStream(device.index))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:
@@ -285,7 +283,9 @@ def reserve_workspace(device, B: int, Hq: int, Hkv: int, L: int, dim: int,
     caller will run (for example before capturing decode graphs for several
     batch sizes), so no later call on that stream replaces it.  Returns bytes."""
     device = torch.device(device)
-    torch.cuda.init()
+    torch.cuda.init()  # the raw stream below is asked of a context that exists
+    if device.index is None:  # tensors name their device with its index
+        device = torch.device(device.type, torch.cuda.current_device())
     nbytes = int(_lib.load().tq_attention_workspace_size(B, Hq, Hkv, L, dim, max_tokens))
     _workspace(device, nbytes)
     return nbytes
