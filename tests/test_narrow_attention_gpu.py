@@ -1,8 +1,8 @@
 """GPU parity of the narrow kernel (tq_attn_narrow.h: few query rows per kv head
 at other dims, K / V dims that differ, plain caches and array masks) vs the
 float64 oracle: every padded dim, 16-row group edges, sub-chunk and wave
-remainders, windows and masks.  Bar as in test_attention_gpu; f32 queries also
-hold the f32-class error of the kernel (weights and operands in two pieces)."""
+remainders, windows and masks.  Bar as in test_attention_gpu; f32 queries at the
+same shapes hold the f32-class error of the kernel that serves them."""
 import math
 
 import numpy as np
@@ -10,8 +10,9 @@ import pytest
 import torch
 
 from oracle import tq_oracle as O
-from kaplumba_amd import ops
+from kaplumba_amd import _lib, ops
 from kaplumba_amd.cache import create_causal_mask
+from tests import attention_paths as paths
 from tests.test_attention_gpu import assert_close, q_tensor
 from tests.test_general_attention_gpu import packed_case
 
@@ -28,7 +29,9 @@ pytestmark = pytest.mark.gpu
     (6, 2, 7, 2100, [2100, 1999], [5, 1900])])      # 21 rows: a group and a remainder; left padding
 def test_narrow_packed(device, dk, krot, dv, vrot, kb, vb, Hq, Hkv, L, T, lengths, starts):
     B = 1 if lengths is None else len(lengths)
-    packed_case(device, 70 + dk + dv + L, B, Hq, Hkv, L, T, dk, dv, kb, vb, krot, vrot, qdt="f16" if L == 7 else "bf16",
+    qdt = "f16" if L == 7 else "bf16"
+    assert paths.path(B, Hq, Hkv, L, T, dk, dv, q=qdt, k_rot=krot, v_rot=vrot) == paths.NARROW
+    packed_case(device, 70 + dk + dv + L, B, Hq, Hkv, L, T, dk, dv, kb, vb, krot, vrot, qdt=qdt,
                 lengths=lengths, starts=starts, norm="float16" if L == 4 else "float32")
 
 
@@ -36,13 +39,14 @@ def test_narrow_packed(device, dk, krot, dv, vrot, kb, vb, Hq, Hkv, L, T, length
 @pytest.mark.parametrize("L,T,W", [(1, 1500, 200), (5, 700, 33), (3, 90, 512)])
 def test_narrow_window_mask(device, d, L, T, W):
     m = create_causal_mask(L, offset=T - L, window_size=W).numpy()
+    assert paths.path(2, 8, 2, L, T, d, mask=_lib.TQ_MASK_BOOL) == paths.NARROW
     packed_case(device, 950 + d + L, 2, 8, 2, L, T, d, d, 3, 3, causal=False, mask_np=m)
 
 
 @pytest.mark.parametrize("d", [96, 128, 256])
 def test_narrow_f32_error(device, d):
-    """f32 queries and outputs: weights of two f16 pieces (2^-22), scores of three
-    products (2^-21 of |q||k| per term at most), so errors stay near f32's own."""
+    """f32 queries and outputs, which take the vector kernel's f32 arithmetic."""
+    assert paths.path(1, 8, 2, 3, 1111, d, q="f32", mask=_lib.TQ_MASK_BOOL) == paths.VECTOR
     rng = np.random.default_rng(d)
     B, Hq, Hkv, L, T = 1, 8, 2, 3, 1111
     rot = "dense" if d == 96 else "hadamard"
@@ -78,6 +82,7 @@ def test_narrow_plain(device, kvdt, dk, dv, Hq, Hkv, L, T, lengths, window):
     v = O.round_to_dtype(rng.standard_normal((B, Hkv, T, dv)).astype(np.float32), kvdt)
     q = O.round_to_dtype(rng.standard_normal((B, Hq, L, dk)).astype(np.float32), kvdt)
     m = create_causal_mask(L, offset=T - L, window_size=window).numpy() if window else None
+    assert paths.path(B, Hq, Hkv, L, T, dk, dv, plain=kvdt, q=kvdt, mask=_lib.TQ_MASK_BOOL if window else 0) == paths.NARROW
     want = O.attention_plain(q, k, v, scale=1 / math.sqrt(dk), q_dtype=kvdt, causal=m is None and L > 1,
                              lengths=lengths, mask=m)
     dt = {"f16": torch.float16, "bf16": torch.bfloat16}[kvdt]

@@ -11,7 +11,8 @@ import numpy as np
 import pytest
 import torch
 
-from kaplumba_amd import ops
+from kaplumba_amd import _lib, ops
+from tests import attention_paths as paths
 
 pytestmark = pytest.mark.gpu
 
@@ -38,13 +39,14 @@ def random_side(g, codec, Hkv, T, norms, device):
     return norms[None], words, norms.double()[..., None] * cb[idx]
 
 
-def attention64(q, scale, kc, vc, k_rows, v_rows, keep):
-    """(1, Hq, L, Dv) in float64; keep: (L, T)."""
+def attention64(q, scale, kc, vc, k_rows, v_rows, keep, bias=0.0):
+    """(1, Hq, L, Dv) in float64; keep, bias: (L, T)."""
     qs = (q * torch.tensor(scale, dtype=q.dtype)).double()
     Hkv = k_rows.shape[0]
     _, Hq, L, D = q.shape
     qr = (qs @ rotation64(kc, q.device).T).reshape(Hkv, Hq // Hkv * L, D)
-    s = (qr @ k_rows.transpose(1, 2).contiguous()).reshape(Hkv, Hq // Hkv, L, -1).masked_fill(~keep, -math.inf)
+    s = (qr @ k_rows.transpose(1, 2).contiguous()).reshape(Hkv, Hq // Hkv, L, -1)
+    s = (s + bias).masked_fill(~keep, -math.inf)
     o = torch.softmax(s, -1).reshape(Hkv, Hq // Hkv * L, -1) @ v_rows @ rotation64(vc, q.device)
     return o.reshape(1, Hq, L, -1)
 
@@ -53,6 +55,7 @@ def attention64(q, scale, kc, vc, k_rows, v_rows, keep):
 @pytest.mark.parametrize("d,rot", [(64, "hadamard"), (96, "dense"), (128, "hadamard"), (256, "hadamard")])
 @pytest.mark.parametrize("kind", ["masked", "faint", "sinking", "tiny"])
 def test_unlike_value_norms(device, Hq, Hkv, L, T, d, rot, kind):
+    assert paths.path(1, Hq, Hkv, L, T, d, q="f16", k_rot=rot, mask=_lib.TQ_MASK_BOOL) == (paths.NARROW if L == 3 else paths.WIDE)
     g = torch.Generator(device=device).manual_seed(d + L)
     kc, vc = ops.Codec(d, 4, 0, rotation=rot), ops.Codec(d, 4, 1, rotation=rot)
     kn = math.sqrt(d) * torch.exp(0.2 * torch.randn(Hkv, T, generator=g, device=device))

@@ -9,8 +9,9 @@ import pytest
 import torch
 
 from oracle import tq_oracle as O
-from kaplumba_amd import ops
+from kaplumba_amd import _lib, ops
 from kaplumba_amd.cache import create_causal_mask
+from tests import attention_paths as paths
 from tests.test_attention_gpu import assert_close, q_tensor
 from tests.test_general_attention_gpu import packed_case
 
@@ -30,8 +31,12 @@ def kv_heads(least, B, rows, T, dk, dv, tuned=False, plain=False, masked=False):
         all_rows, work = 1024, 1
     else:
         all_rows, work = (8192, 4) if masked else (1024, 8)
-    return max(least, math.ceil(all_rows / (B * rows)),
-               math.ceil(1.02 * work * 2 ** 28 / (B * rows * T * (dk + dv))))
+    n = max(least, math.ceil(all_rows / (B * rows)), math.ceil(1.02 * work * 2 ** 28 / (B * rows * T * (dk + dv))))
+    # the library's own rule, so that a moved line shows here
+    got = paths.path(B, n, n, rows, T, dk, dv, plain="f16" if plain else None, q="f16", k_rot="dense",
+                     v_rot="dense" if tuned or masked or plain else "hadamard", mask=_lib.TQ_MASK_BOOL if masked else 0)
+    assert got == paths.WIDE, (B, n, rows, T, dk, dv, got)
+    return n
 
 
 @pytest.mark.parametrize("dk,krot,dv,vrot,kb,vb", [
