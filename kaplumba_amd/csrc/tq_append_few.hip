@@ -214,7 +214,10 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
   float y[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) y[j] = __fadd_rn(__fadd_rn(acc[2][j], acc[1][j]), acc[0][j]);
-  bool tie[4] = {false, false, false, false};
+  // (a norm past f32's range has no threshold to compare with)
+  bool tie[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) tie[j] = dj[j] == INFINITY;
 #pragma unroll
   for (int m = 0; m < 15; ++m) {
     if (m >= nmid) break;  // uniform

@@ -120,3 +120,25 @@ def test_ties_are_the_vector_kernels(device, d, xdt):
         want = (y[..., None] > m).sum(-1)
         got = O.unpack_lowbit(p.cpu().numpy().astype(np.uint32)[0, 0], 4, d)
         assert np.array_equal(got, want), np.argwhere(got != want)[:4]
+
+
+@pytest.mark.parametrize("d", [8, 40, 96, 192])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("bits", [1, 3, 4])
+def test_norms_past_the_range(device, d, xdt, bits):
+    """Finite vectors whose norm is infinite: u = x / inf = 0, so every index counts the thresholds below 0."""
+    dt = {"bf16": torch.bfloat16, "f32": torch.float32}[xdt]
+    x = torch.randn(1, 1, 20, d, generator=torch.Generator().manual_seed(d)).to(dt)
+    x[0, 0, 3] *= 2e30
+    x[0, 0, 4, 1] = torch.finfo(dt).max
+    x[0, 0, 5] = torch.finfo(dt).max
+    codec = ops.Codec(d, bits, 0, rotation="dense")
+    p = torch.zeros((1, 1, 20, codec.packed_width), dtype=torch.uint32, device=device)
+    n = torch.zeros((1, 1, 20), device=device)
+    ops.append_quantize(x.to(device), codec, p, n, 0)
+    got = O.unpack_lowbit(p.cpu().numpy().astype(np.uint32)[0, 0], bits, d)
+    assert torch.isinf(n[0, 0, 3:6]).all()
+    assert (got[3:6] == (0.0 > np.array(codec.midpoints)).sum()).all()
+    rest = np.r_[0:3, 6:20]
+    assert _check(x.float().numpy()[:, :, rest], bits, d, 0, p.cpu().numpy().astype(np.uint32)[:, :, rest],
+                  n.cpu().numpy()[:, :, rest]) <= 2
