@@ -231,7 +231,10 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
 #pragma unroll
   for (int j = 0; j < 4; ++j) s_idx[(4 * g + j) * kFewIdxRow + 16 * wave + n] = static_cast<uint8_t>(idx[j]);
   if (__any(tie[0] | tie[1] | tie[2] | tie[3])) {
-    // the wave's ties as a list, then four lanes a tie, one per chain of the vector kernel
+    // the wave's ties as a list, then sixteen lanes a tie: four to each chain of the
+    // vector kernel, a quarter of its elements each, loaded and divided side by
+    // side and added in order (the chain goes from quarter to quarter, which sit
+    // one lane bit apart)
     int ties = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -241,9 +244,13 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
       ties += __builtin_popcountll(set);
     }
     wave_lds_order();
+    const int slot = (lane >> 2) & 3;
+    const int quarter = slot ^ (slot >> 1);
+    const int per = (D / 4 + 3) / 4;  // elements of a quarter, at most 2 KS
+    const int k0 = quarter * per;
 #pragma unroll 1
-    for (int t0 = 0; t0 < ties; t0 += 16) {
-      const int code = s_tie[wave][min(t0 + (lane >> 2), ties - 1)];
+    for (int t0 = 0; t0 < ties; t0 += 4) {
+      const int code = s_tie[wave][min(t0 + (lane >> 4), ties - 1)];
       const int tv = code >> 4;
       const int tn = code & 15;
       const int gv = min(static_cast<int>(blockIdx.x) * 16 + tv, n_vec - 1);
@@ -252,19 +259,27 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
                          (gv - bh * a.L) * a.sl + (lane & 3);
       const float* row = a.rot + static_cast<int64_t>(min(s0 + 16 * wave + tn, D - 1)) * D + (lane & 3);
       const float td = __shfl(den, tv, 64);
+      float u[2 * KS], r[2 * KS];
+#pragma unroll
+      for (int e = 0; e < 2 * KS; ++e) {
+        const int k = min(4 * (k0 + e), D - 4);
+        u[e] = load_elem<XDT>(a.x, tx + k);
+        r[e] = row[k];
+      }
+#pragma unroll
+      for (int e = 0; e < 2 * KS; ++e) u[e] = __fdiv_rn(u[e], td);
       float c = 0.f;
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {  // 32 elements, 8 of this chain; D is a multiple of 8
-        float u[8], r[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int k = min(32 * s + 4 * e, D - 4);
-          u[e] = load_elem<XDT>(a.x, tx + k);
-          r[e] = row[k];
+      for (int q = 0; q < 4; ++q) {
+        if (q > 0) {
+          const float from = (q & 1) ? xor_lane<4>(c) : xor_lane<8>(c);
+          c = quarter == q ? from : c;
         }
+        if (quarter == q) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (32 * s + 4 * e < D) c = __builtin_fmaf(__fdiv_rn(u[e], td), r[e], c);
+          for (int e = 0; e < 2 * KS; ++e)
+            if (e < per && 4 * (k0 + e) < D) c = __builtin_fmaf(u[e], r[e], c);
+        }
       }
       c = __fadd_rn(c, xor_lane<1>(c));
       const float ty = __fadd_rn(c, xor_lane<2>(c));
@@ -272,7 +287,7 @@ __global__ __launch_bounds__(kFewThreads) void append_few_kernel(AppendArgs ka, 
 #pragma unroll
       for (int m = 0; m < 15; ++m)
         if (m < nmid) ti += ty > mid[m] ? 1u : 0u;
-      if ((lane & 3) == 0) s_idx[tv * kFewIdxRow + 16 * wave + tn] = static_cast<uint8_t>(ti);
+      if ((lane & 3) == 0 && quarter == 3) s_idx[tv * kFewIdxRow + 16 * wave + tn] = static_cast<uint8_t>(ti);
     }
   }
   __syncthreads();
@@ -333,8 +348,9 @@ int launch_few(const AppendArgs& k, const AppendArgs& v, int sides, int dim, int
 }  // namespace
 
 // Every count of vectors: K + V, 8 heads, bf16, 3 bits, us in the vector kernel ->
-// here, ties included (one costs its workgroup 2.5 us at d = 96, 5 at 192): d = 96
-// 26 -> 4.9 for 8 vectors a side, 33 -> 13.5 for 4096; d = 192 43 -> 6.4 and 77 -> 28.
+// here, ties included (one adds 1 us to a launch, 2.5-5 with four lanes a tie):
+// d = 96 26 -> 4.9 for 8 vectors a side, 33 -> 12.0 for 4096; d = 192 43 -> 6.2 and
+// 77 -> 23.3.
 bool append_few_path(int64_t n_vec, int dim) {
   return dim % 8 == 0 && dim >= 8 && dim <= kFewMaxDim && dim != 64 && dim != 128 && dim != 256 &&
          n_vec < (int64_t(1) << 31) - 16;
