@@ -103,12 +103,13 @@ __device__ __forceinline__ void split_f16(float x, uint32_t& hi, uint32_t& lo) {
 
 // 2^(13 - e) for max |x| = f * 2^e, f in [0.5, 1): scales the largest
 // magnitude into [2^12, 2^13), far from f16 overflow and with the lo parts
-// of a hi/lo split still normal numbers.
+// of a hi/lo split still normal numbers.  At most 2^100: the scale of a row of
+// 1e-36, and its product with a codebook's, would overflow.
 __device__ __forceinline__ float f16_split_scale(float maxabs) {
   if (!(maxabs > 0.f) || !(maxabs < INFINITY)) return 1.f;
   int e;
   frexpf(maxabs, &e);
-  return ldexpf(1.f, 13 - e);
+  return ldexpf(1.f, min(13 - e, 100));
 }
 
 template <int D, int KB, int VB, int NQ>

@@ -87,3 +87,26 @@ def test_unlike_value_norms(device, Hq, Hkv, L, T, d, rot, kind):
     out = ops.attention_packed(q, k_norms, k_words, v_norms, v_words, kc, vc, 1 / math.sqrt(d), False, mask=keep)
     err = (out.double() - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max().item() <= 2.0 ** (-8 if kind == "tiny" else -11) + 2e-6, err.max().item()
+
+
+@pytest.mark.parametrize("Hq,Hkv,L,T", [(8, 2, 3, 2111), (64, 16, 160, 1111)])  # narrow, or tuned; wide or tile
+@pytest.mark.parametrize("d,rot", [(64, "hadamard"), (96, "dense"), (128, "hadamard"), (256, "hadamard")])
+@pytest.mark.parametrize("masked", [False, True])
+def test_tiny_queries(device, Hq, Hkv, L, T, d, rot, masked):
+    """Query rows of 1e-36 and 1e-30 score every key alike: their output is the mean of the values."""
+    g = torch.Generator(device=device).manual_seed(d + L)
+    kc, vc = ops.Codec(d, 4, 0, rotation=rot), ops.Codec(d, 4, 1, rotation=rot)
+    norms = torch.exp(0.3 * torch.randn(Hkv, T, generator=g, device=device))
+    k_norms, k_words, k_rows = random_side(g, kc, Hkv, T, norms, device)
+    v_norms, v_words, v_rows = random_side(g, vc, Hkv, T, norms, device)
+    q = torch.randn(1, Hq, L, d, generator=g, device=device)
+    q[0, 0] *= 1e-36
+    q[0, 1] *= 1e-30
+    q = q.to(torch.bfloat16)
+    keep = torch.arange(T, device=device)[None] <= torch.arange(T - L, T, device=device)[:, None]
+    want = attention64(q, 1 / math.sqrt(d), kc, vc, k_rows, v_rows, keep)
+    out = ops.attention_packed(q, k_norms, k_words, v_norms, v_words, kc, vc, 1 / math.sqrt(d), not masked,
+                               mask=keep if masked else None)
+    err = (out.double() - want).norm(dim=-1) / want.norm(dim=-1)
+    # bf16 outputs, and the f16 weights of the tuned dims (2^-11 each)
+    assert err.max().item() <= 2.0 ** -8 + 2.0 ** -10, err.max().item()
