@@ -160,6 +160,15 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
   const int ktok = 8 * (n >> 2) + (n & 3);
   uint32_t kreg[S::KU][S::RW], vreg[S::VU][S::RW];
   float nreg = 0.f;
+  // plain rows of more than 128 columns: values load after the scores of their own
+  // sub-chunk, where the keys' registers are free (one ahead they spill)
+  constexpr bool LATE_V = !PACKED && CT > 8;
+  auto load_v = [&](int i) {
+    const int t0 = t_begin + i * SUB;
+    // value unit u: piece u of 64 lanes (token lane / 2, half lane % 2 of block u)
+#pragma unroll
+    for (int u = 0; u < S::VU; ++u) unit_load(vbase, vstride, vb, p.vpw, p.Dv, 2 * u + (lane & 1), t0 + (lane >> 1), vreg[u]);
+  };
   auto load = [&](int i) {
     const int t0 = t_begin + i * SUB;
 #pragma unroll
@@ -170,9 +179,7 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
       const int64_t at = rowbase + min(t0 + (lane & 31), t_end - 1);
       nreg = load_norm(lane < 32 ? p.kn : p.vn, p.norm_dtype, at);
     }
-    // value unit u: piece u of 64 lanes (token lane / 2, half lane % 2 of block u)
-#pragma unroll
-    for (int u = 0; u < S::VU; ++u) unit_load(vbase, vstride, vb, p.vpw, p.Dv, 2 * u + (lane & 1), t0 + (lane >> 1), vreg[u]);
+    if constexpr (!LATE_V) load_v(i);
   };
   if (wave < nsub) load(wave);
 
@@ -322,6 +329,7 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
           C[h] = mfma_wide<SRC>(al, qh[s], C[h]);
         }
       }
+    if constexpr (LATE_V) load_v(i);
     // ---- softmax: tokens t0 + 8 g + j of this lane's row
     float y[8];
     float ym = -INFINITY;
@@ -400,7 +408,18 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
           }
         }
     }
-    // ---- O += P V, CC blocks of 16 columns at a time through the wave's tile
+    // ---- O += P V, CC blocks of 16 columns at a time through the wave's tile.
+    // Infinite values (and NaN) meet the weight itself only, as in gen_wide_kernel:
+    // a sub-chunk that holds any gives its low pieces finite values.
+    bool careful = false;
+    if constexpr (!PACKED) {
+      float z = 0.f;  // NaN from the first infinity or NaN on
+#pragma unroll
+      for (int u = 0; u < S::VU; ++u)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) z = wide_times0<SRC>(vreg[u][w], z);
+      careful = __any(z != z ? 1 : 0);
+    }
 #pragma unroll
     for (int c0 = 0; c0 < CT; c0 += S::CC) {
       wave_sync();  // the tile's last readers are behind
@@ -409,6 +428,8 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
         if (c0 + c >= CT) continue;
         u32x4_t hi, lo;
         unit_parts(vreg[c0 + c], vb, 2 * (c0 + c) + (lane & 1), vtab, vesh, hi, lo);
+        if constexpr (!PACKED)  // the slab's last token again, at weight 0
+          if (careful && t0 + (lane >> 1) >= t_end) hi = u32x4_t{0u, 0u, 0u, 0u};
         *reinterpret_cast<u32x4_t*>(vdst + c * S::VCT) = hi;
         if constexpr (PACKED) *reinterpret_cast<u32x4_t*>(vdst + (S::CC + c) * S::VCT) = lo;
       }
@@ -420,6 +441,9 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
         const uint2 h0 = read_tr(vtr[0] + c * S::VCT);
         const uint2 h1 = read_tr(vtr[1] + c * S::VCT);
         const u32x4_t bh = {h0.x, h0.y, h1.x, h1.y};
+        u32x4_t bf = bh;  // of the weights' low pieces
+        if constexpr (!PACKED)
+          if (careful) bf = wide_finite<SRC>(bh);
         if constexpr (PACKED) {
           const uint2 g0 = read_tr(vtr[0] + (S::CC + c) * S::VCT);
           const uint2 g1 = read_tr(vtr[1] + (S::CC + c) * S::VCT);
@@ -429,7 +453,7 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
           O[c0 + c] = mfma_wide<SRC>(A[1], bh, O[c0 + c]);
         } else {
 #pragma unroll
-          for (int q = 0; q < WP; ++q) O[c0 + c] = mfma_wide<SRC>(A[q], bh, O[c0 + c]);
+          for (int q = 0; q < WP; ++q) O[c0 + c] = mfma_wide<SRC>(A[q], q > 0 ? bf : bh, O[c0 + c]);
         }
       }
     }

@@ -45,6 +45,8 @@
 // that gen_mask_range_kernel found kept, its splits sharing that range evenly.
 #pragma once
 
+#include <type_traits>
+
 #include "tq_attn_general.h"
 #include "tq_attn_mfma.h"
 #include "tq_attn_slots.h"
@@ -134,6 +136,33 @@ __device__ __forceinline__ uint2 wide_mask_bytes(const uint8_t* row, int64_t st,
     w[j >> 2] |= k << (8 * (j & 3));
   }
   return make_uint2(w[0], w[1]);
+}
+
+// Two halves of a plain value operand, those that are infinite or NaN as zeros.
+template <int SRC>
+__device__ __forceinline__ uint32_t wide_finite2(uint32_t x) {
+  constexpr uint32_t ulp = SRC == kWideBf16 ? 0x00800080u : 0x04000400u;  // one exponent step
+  const uint32_t m = ((x & 0x7fff7fffu) + ulp) & 0x80008000u;             // bit 15 where all exponent bits are set
+  return x & ~(m | (m - (m >> 15)));
+}
+
+// z + 0 x of two halves: z, or NaN where a half is infinite or NaN.
+template <int SRC>
+__device__ __forceinline__ float wide_times0(uint32_t x, float z) {
+  if constexpr (SRC == kWideBf16) {
+    typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2_t, x), bf2_t{}, z, false);
+  } else {
+    typedef _Float16 f2_t __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f2_t, x), f2_t{}, z, false);
+  }
+}
+
+template <int SRC>
+__device__ __forceinline__ u32x4_t wide_finite(u32x4_t x) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = wide_finite2<SRC>(x[j]);
+  return x;
 }
 
 // An additive mask entry in log2 units; finite entries stay finite.
@@ -512,7 +541,7 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
     if constexpr (PACKED)
       if (tid < 2 * SUB) reinterpret_cast<float*>(lds + S::NRM)[tid] = nreg;
   };
-  auto put_v = [&]() {
+  auto put_v = [&](auto careful, int i) {
 #pragma unroll
     for (int u = 0; u < S::VU; ++u) {
       const int e = tid + u * kWideThreads;
@@ -520,6 +549,8 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
         const int t = e / VC8, c8 = e % VC8;
         uint4 hi, lo;
         unit_parts(vreg[u], vb, c8, vtab, vesh, hi, lo);
+        if constexpr (careful)  // the split's last token again, at weight 0
+          if (t_begin + i * SUB + t >= t_end) hi = make_uint4(0u, 0u, 0u, 0u);
         unsigned char* d = lds + S::VHI + (c8 >> 1) * S::VCT + (t >> 5) * 1024 + tile_vslot(t & 31) * 32 + (c8 & 1) * 16;
         *reinterpret_cast<uint4*>(d) = hi;
         if constexpr (PACKED) *reinterpret_cast<uint4*>(d + (S::VLO - S::VHI)) = lo;
@@ -778,13 +809,15 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
   };
 
   // O += P V of half hf of the step in the V slot
-  auto pv = [&](int hf, const u32x4_t (&A)[RT][WP]) {
+  auto pv = [&](auto careful, int hf, const u32x4_t (&A)[RT][WP]) {
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       const uint32_t off = ct * S::VCT + hf * 1024;
       const uint2 h0 = read_tr(vtr[0] + off);
       const uint2 h1 = read_tr(vtr[1] + off);
       const u32x4_t bh = {h0.x, h0.y, h1.x, h1.y};
+      u32x4_t bf = bh;  // of the weights' low pieces
+      if constexpr (careful) bf = wide_finite<SRC>(bh);
       if constexpr (PACKED) {
         const uint2 g0 = read_tr(vtr[0] + off + (S::VLO - S::VHI));
         const uint2 g1 = read_tr(vtr[1] + off + (S::VLO - S::VHI));
@@ -799,65 +832,99 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-          for (int q = 0; q < WP; ++q) O[rt][ct] = mfma_wide<SRC>(A[rt][q], bh, O[rt][ct]);
+          for (int q = 0; q < WP; ++q) O[rt][ct] = mfma_wide<SRC>(A[rt][q], q > 0 ? bf : bh, O[rt][ct]);
       }
     }
   };
 
-  // ---- K of step 0 in its slot, K of step 1 and V of step 0 loading
-  put_k();
-  if (ntiles > 1) load_k(1);
-  lds_barrier();
+  // ---- the walk over the split's tokens: K of step 0 in its slot, K of step 1 and
+  // V of step 0 loading
   const bool lead = wave < kWideNW / 2;
+  auto walk = [&](auto careful) __attribute__((always_inline)) {
+    put_k();
+    if (ntiles > 1) load_k(1);
+    lds_barrier();
 #pragma unroll 1
-  for (int i = 0; i < ntiles; ++i) {
-    const int t0 = t_begin + i * SUB;
-    const bool act = wave_live && t0 < whi && t0 + SUB > wlo;  // some row of the wave sees a token
-    u32x4_t A[H][RT][WP];
-    if (lead) {
-      put_v();
-      if (i + 1 < ntiles) load_v(i + 1);
-    }
-    if (act) {
+    for (int i = 0; i < ntiles; ++i) {
+      const int t0 = t_begin + i * SUB;
+      const bool act = wave_live && t0 < whi && t0 + SUB > wlo;  // some row of the wave sees a token
+      u32x4_t A[H][RT][WP];
+      if (lead) {
+        put_v(careful, i);
+        if (i + 1 < ntiles) load_v(i + 1);
+      }
+      if (act) {
 #pragma unroll
-      for (int hf = 0; hf < H; ++hf) {
-        uint2 mk[RT];
-        if constexpr (GEN) {
-          if (p.mask_kind == TQ_MASK_BOOL) {
+        for (int hf = 0; hf < H; ++hf) {
+          uint2 mk[RT];
+          if constexpr (GEN) {
+            if (p.mask_kind == TQ_MASK_BOOL) {
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-              mk[rt] = wide_mask_bytes(static_cast<const uint8_t*>(p.mask) + mrow[rt], p.m_st, t0 + 32 * hf + 8 * g, len);
+              for (int rt = 0; rt < RT; ++rt)
+                mk[rt] = wide_mask_bytes(static_cast<const uint8_t*>(p.mask) + mrow[rt], p.m_st, t0 + 32 * hf + 8 * g, len);
+            }
           }
+          f32x4_t C[RT][2];
+          scores(hf, C);
+          softmax(t0 + 32 * hf, hf, C, mk, A[hf]);
         }
-        f32x4_t C[RT][2];
-        scores(hf, C);
-        softmax(t0 + 32 * hf, hf, C, mk, A[hf]);
       }
-    }
-    if (!lead) {
-      put_v();
-      if (i + 1 < ntiles) load_v(i + 1);
-    }
-    lds_barrier();
-    if (lead && i + 1 < ntiles) {
-      put_k();
-      if (i + 2 < ntiles) load_k(i + 2);
-    }
-    if (act) {
+      if (!lead) {
+        put_v(careful, i);
+        if (i + 1 < ntiles) load_v(i + 1);
+      }
+      lds_barrier();
+      if (lead && i + 1 < ntiles) {
+        put_k();
+        if (i + 2 < ntiles) load_k(i + 2);
+      }
+      if (act) {
 #pragma unroll
-      for (int hf = 0; hf < H; ++hf) {
-        if (hf > 0 && pending) {
-          rescale(fac);
-          pending = false;
+        for (int hf = 0; hf < H; ++hf) {
+          if (hf > 0 && pending) {
+            rescale(fac);
+            pending = false;
+          }
+          pv(careful, hf, A[hf]);
         }
-        pv(hf, A[hf]);
       }
+      if (!lead && i + 1 < ntiles) {
+        put_k();
+        if (i + 2 < ntiles) load_k(i + 2);
+      }
+      lds_barrier();
     }
-    if (!lead && i + 1 < ntiles) {
-      put_k();
-      if (i + 2 < ntiles) load_k(i + 2);
-    }
+  };
+  walk(std::false_type{});
+  if constexpr (GEN && !PACKED) {
+    // An infinite value times the weights' low pieces, which may be negative or 0,
+    // is a NaN where its product with the weight itself (the vector kernel's) is
+    // infinite.  A block with a NaN in its result walks its tokens once more, the
+    // low pieces against finite values only; no other block pays for it.
+    bool nan = false;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) nan |= O[rt][ct][k] != O[rt][ct][k];
+    const bool any = __any(nan ? 1 : 0);
+    if (lane == 0) rng[wave].x = any ? 1 : 0;  // (the ranges have been read)
     lds_barrier();
+    int again = 0;
+#pragma unroll
+    for (int w = 0; w < kWideNW; ++w) again |= rng[w].x;
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(again) != 0, 0)) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        row[rt] = WideRow{-INFINITY, 0.f, static_cast<float>(1 << kWExp)};
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) O[rt][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+      load_k(0);
+      load_v(0);
+      walk(std::true_type{});
+    }
   }
   // ---- partials: (o, m, l) per row, o = O / (vsc sv) (packed: in the rotated value basis)
   if (!wave_live) return;
