@@ -20,7 +20,7 @@
 // coordinate lies within the bound of both kernels' rounding of a threshold
 // (tie_units), its index comes from the vector kernel's own arithmetic (IEEE
 // division, four fused chains), so the two agree bit for bit: one coordinate in
-// 3000 (d = 96, 4 bits), a branch that one wave in twelve takes.
+// 5400 at d = 96, 4 bits (2100 at d = 192), a branch that one wave in 21 (9) takes.
 #include "tq_append.h"
 
 namespace tq {

@@ -19,7 +19,8 @@
 // (8 rows a workgroup, f32 multiply-adds): d = 96, 4 bits, 8 sequences x 6000
 // tokens 112 -> 38 us, 16384 tokens 268 -> 64; one sequence x 1024 tokens 32 ->
 // 19; plain bf16 d = 96 8 x 6000 154 -> 35; a 512-key window over 8 x 6000 tokens
-// of d = 128 110 -> 22, d = 256 216 -> 41 (its registers spill).
+// of d = 128 110 -> 22, d = 256 216 -> 41.  Packed keys of more than 128
+// coordinates spill (48 bytes at KS 6, 576 at KS 8; plain KS 8 80 to 128).
 #pragma once
 
 #include "tq_attn_wide.h"

@@ -20,17 +20,20 @@
 //
 // What bounds it: matrix products, LDS reads (an operand is read once per
 // 16 RT rows) and softmax add up at two waves per SIMD.  SUB is 64 where the
-// slots fit, 32 at the widest packed heads; RT is the largest that keeps
-// queries and outputs (2 x 16 RT (KS + CT/2) registers) within half of 256.
+// slots fit, 32 at the widest packed heads.  RT is 2 up to KS = 4 and 1 beyond:
+// packed queries and outputs take 8 RT (KS + CT/2) registers, 128 of 256 at KS = 4
+// and 8.  (KS = 2 leaves room by that count, but packed kernels of RT 3 and 4 spill
+// 16 to 308 bytes there.)  The compiler's totals: 200 (KS 2, one weight piece), 224
+// (KS 8), 256 and 100 bytes of scratch (KS 4, two pieces), 214 (KS 4, plain bf16).
 //
 // Measured, append and attention of one layer, against the kernel that took
 // the call before: 512 queries x 8192 tokens under a 4096-key boolean window,
-// d = 128, 3 bits: 2815 -> 170 us (vector kernel); 2 x 500 queries x 4097
+// d = 128, 3 bits: 2815 -> 176 us (vector kernel); 2 x 500 queries x 4097
 // tokens, d = 64, K3/V4: 243 -> 129 us, and 512 queries x 4096 tokens, d = 256,
-// K4/V2, dense: 540 -> 165 us (attn_mfma_kernel: decodes per 16 or 4 rows);
-// 512 queries x 8192 plain bf16 tokens, d = 128: 345 -> 170 us
-// (attn_plain_kernel: reads K/V per 16 rows).  Partial kernels alone: 156, 119,
-// 119 and 172 us.
+// K4/V2, dense: 538 -> 152 us (attn_mfma_kernel: decodes per 16 or 4 rows);
+// 512 queries x 8192 plain bf16 tokens, d = 128: 345 -> 168 us
+// (attn_plain_kernel: reads K/V per 16 rows).  Partial kernels alone, in a trace:
+// 163, 120, 120 and 167 us.
 //
 // Weight pieces WP.  1: f16 weights, as the other packed kernels.  More where
 // the general vector kernel held weights in f32: f16 hi + lo (2; under a power
