@@ -190,33 +190,8 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
   {
     const int64_t qrow = static_cast<int64_t>(pair) * RL + rr;
     if (PACKED && p.q_rows32) {
-      const float* src = p.qrot + qrow * p.DkP + 8 * g;
-      float v[KS][8];
-      float mx = 0.f;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const bool in = 32 * s < p.DkP;
-        const float4 a = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0));
-        const float4 c = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0) + 4);
-        const bool live = in && row_ok;
-        v[s][0] = live ? a.x : 0.f, v[s][1] = live ? a.y : 0.f, v[s][2] = live ? a.z : 0.f, v[s][3] = live ? a.w : 0.f;
-        v[s][4] = live ? c.x : 0.f, v[s][5] = live ? c.y : 0.f, v[s][6] = live ? c.z : 0.f, v[s][7] = live ? c.w : 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[s][e]));
-      }
-      mx = fmaxf(mx, xor_lane<16>(mx));
-      const float2 hm = halves(mx);
-      const float sq = f16_split_scale(fmaxf(hm.x, hm.y));
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint32_t h0, l0, h1, l1;
-          split_f16(v[s][2 * e] * sq, h0, l0);
-          split_f16(v[s][2 * e + 1] * sq, h1, l1);
-          qh[s][e] = h0 | (h1 << 16);
-          if constexpr (PACKED) ql[s][e] = l0 | (l1 << 16);
-        }
+      float sq = 1.f;
+      if constexpr (PACKED) sq = wide_split_row<KS>(p.qrot + qrow * p.DkP + 8 * g, p.DkP, row_ok, qh, ql);
       qmul = sq;
     } else {
       const u32x4_t* src = reinterpret_cast<const u32x4_t*>(p.qhl) + qrow * (4 * KS * S::PARTS) + g;
@@ -238,31 +213,8 @@ __global__ __launch_bounds__(512) void gen_narrow_kernel(GenParams p, int n_grou
   float sv = 1.f;
   const int kesh = kb == 4 ? 6 : 8, vesh = vb == 4 ? 6 : 8;
   if constexpr (PACKED) {
-    float* cbl = reinterpret_cast<float*>(lds + S::TILE);
-    if (tid < (1 << kb)) cbl[tid] = p.kcb[tid];
-    if (tid < (1 << vb)) cbl[16 + tid] = p.vcb[tid];
-    lds_barrier();
-    float kmax = 0.f, vmax = 0.f;
-    for (int i = 0; i < (1 << kb); ++i) kmax = fmaxf(kmax, fabsf(cbl[i]));
-    for (int i = 0; i < (1 << vb); ++i) vmax = fmaxf(vmax, fabsf(cbl[16 + i]));
-    const float sk = f16_split_scale(kmax);
-    sv = f16_split_scale(vmax);
+    const float sk = wide_pair_tables<S::NT, S::KTAB, S::VTAB, S::TILE>(lds, p, kesh, vesh, tid, sv);
     qmul = 1.4426950408889634f / (sk * qmul);
-    for (int e = tid; e < ((1 << (2 * kb + kesh)) >> 3); e += S::NT) {
-      const int key = e >> (kesh - 3);
-      uint32_t h0, l0, h1, l1;
-      split_f16(cbl[key & ((1 << kb) - 1)] * sk, h0, l0);
-      split_f16(cbl[key >> kb] * sk, h1, l1);
-      *reinterpret_cast<uint2*>(lds + S::KTAB + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
-    }
-    for (int e = tid; e < ((1 << (2 * vb + vesh)) >> 3); e += S::NT) {
-      const int key = e >> (vesh - 3);
-      uint32_t h0, l0, h1, l1;
-      split_f16(cbl[16 + (key & ((1 << vb) - 1))] * sv, h0, l0);
-      split_f16(cbl[16 + (key >> vb)] * sv, h1, l1);
-      *reinterpret_cast<uint2*>(lds + S::VTAB + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
-    }
-    lds_barrier();
   }
   const uint32_t ktab = S::KTAB + (lane & ((1 << (kesh - 3)) - 1)) * 8;
   const uint32_t vtab = S::VTAB + (lane & ((1 << (vesh - 3)) - 1)) * 8;

@@ -247,6 +247,68 @@ __device__ __forceinline__ float wide_row_drop(WideRow& w, float wm, float top) 
   return f;
 }
 
+// A lane's coordinates 32 s + 8 g .. + 7 of a rotated query row in f32 (src: its
+// first), as hi and lo f16 parts under the row's scale, which is returned; a row
+// that is not live, and steps past DkP, are zeros.
+template <int KS>
+__device__ __forceinline__ float wide_split_row(const float* src, int DkP, bool row_live, u32x4_t (&qh)[KS], u32x4_t (&ql)[KS]) {
+  float v[KS][8];
+  float mx = 0.f;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const bool in = 32 * s < DkP;  // uniform: whole steps past the row are zero
+    const float4 a = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0));
+    const float4 c = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0) + 4);
+    const bool live = in && row_live;
+    v[s][0] = live ? a.x : 0.f, v[s][1] = live ? a.y : 0.f, v[s][2] = live ? a.z : 0.f, v[s][3] = live ? a.w : 0.f;
+    v[s][4] = live ? c.x : 0.f, v[s][5] = live ? c.y : 0.f, v[s][6] = live ? c.z : 0.f, v[s][7] = live ? c.w : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[s][e]));
+  }
+  const float sq = f16_split_scale(wide_row_max(mx));
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t h0, l0, h1, l1;
+      split_f16(v[s][2 * e] * sq, h0, l0);
+      split_f16(v[s][2 * e + 1] * sq, h1, l1);
+      qh[s][e] = h0 | (h1 << 16);
+      ql[s][e] = l0 | (l1 << 16);
+    }
+  return sq;
+}
+
+// Pair tables of both codebooks: entry (a | b << bits) = (hi c_a | hi c_b << 16,
+// lo c_a | lo c_b << 16) of the codebook scaled by a power of two (largest magnitude
+// in [2^12, 2^13)), 2^esh bytes of copies each.  Called by all NT threads; TMP: 128
+// bytes that nothing else uses.  Returns the keys' scale.
+template <int NT, int KTAB, int VTAB, int TMP>
+__device__ __forceinline__ float wide_pair_tables(unsigned char* lds, const GenParams& p, int kesh, int vesh, int tid, float& sv) {
+  float* cbl = reinterpret_cast<float*>(lds + TMP);
+  const int kb = p.kbits, vb = p.vbits;
+  if (tid < (1 << kb)) cbl[tid] = p.kcb[tid];
+  if (tid < (1 << vb)) cbl[16 + tid] = p.vcb[tid];
+  lds_barrier();
+  auto table = [&](const float* cb, int bits, int esh, int at) {
+    float mx = 0.f;
+    for (int i = 0; i < (1 << bits); ++i) mx = fmaxf(mx, fabsf(cb[i]));
+    const float sc = f16_split_scale(mx);
+    for (int e = tid; e < ((1 << (2 * bits + esh)) >> 3); e += NT) {
+      const int key = e >> (esh - 3);
+      uint32_t h0, l0, h1, l1;
+      split_f16(cb[key & ((1 << bits) - 1)] * sc, h0, l0);
+      split_f16(cb[key >> bits] * sc, h1, l1);
+      *reinterpret_cast<uint2*>(lds + at + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
+    }
+    return sc;
+  };
+  const float sk = table(cbl, kb, kesh, KTAB);
+  sv = table(cbl + 16, vb, vesh, VTAB);
+  lds_barrier();
+  return sk;
+}
+
 template <int KS, int CT, int RT, int SRC, int WP>
 __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int n_blocks) {
   using S = WideShape<KS, CT, RT, SRC, WP>;
@@ -433,33 +495,8 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
       if constexpr (PACKED) rows32 = p.q_rows32 != 0;
       if (rows32) {
         if constexpr (PACKED) {
-          const float* src = p.qrot + (pair_row0 + rr) * p.DkP + 8 * g;
-          float v[KS][8];
-          float mx = 0.f;
-#pragma unroll
-          for (int s = 0; s < KS; ++s) {
-            const bool in = 32 * s < p.DkP;  // uniform: whole steps past the row are zero
-            const float4 a = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0));
-            const float4 c = *reinterpret_cast<const float4*>(src + (in ? 32 * s : 0) + 4);
-            const bool live = in && row_ok[rt];
-            v[s][0] = live ? a.x : 0.f, v[s][1] = live ? a.y : 0.f, v[s][2] = live ? a.z : 0.f, v[s][3] = live ? a.w : 0.f;
-            v[s][4] = live ? c.x : 0.f, v[s][5] = live ? c.y : 0.f, v[s][6] = live ? c.z : 0.f, v[s][7] = live ? c.w : 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[s][e]));
-          }
-          mx = fmaxf(mx, xor_lane<16>(mx));
-          const float2 hm = halves(mx);
-          const float sq = f16_split_scale(fmaxf(hm.x, hm.y));
-#pragma unroll
-          for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              uint32_t h0, l0, h1, l1;
-              split_f16(v[s][2 * e] * sq, h0, l0);
-              split_f16(v[s][2 * e + 1] * sq, h1, l1);
-              qh[rt][s][e] = h0 | (h1 << 16);
-              ql[rt][s][e] = l0 | (l1 << 16);
-            }
+          const float sq =
+              wide_split_row<KS>(p.qrot + (pair_row0 + rr) * p.DkP + 8 * g, p.DkP, row_ok[rt], qh[rt], ql[rt]);
           qmul[rt] = sq;
         }
       } else {
@@ -479,37 +516,13 @@ __global__ __launch_bounds__(kWideThreads) void gen_wide_kernel(GenParams p, int
     }
   }
 
-  // ---- pair tables: entry (a | b << bits) = (hi c_a | hi c_b << 16, lo c_a | lo c_b << 16)
-  // of the codebooks scaled by a power of two (largest magnitude in [2^12, 2^13))
+  // ---- pair tables
   float sv = 1.f;
   const int kesh = kb == 4 ? 6 : 8, vesh = vb == 4 ? 6 : 8;  // log2 of an entry's bytes over its copies
   if constexpr (PACKED) {
-    float* cbl = reinterpret_cast<float*>(lds + S::KHI);
-    if (tid < (1 << kb)) cbl[tid] = p.kcb[tid];
-    if (tid < (1 << vb)) cbl[16 + tid] = p.vcb[tid];
-    __syncthreads();
-    float kmax = 0.f, vmax = 0.f;
-    for (int i = 0; i < (1 << kb); ++i) kmax = fmaxf(kmax, fabsf(cbl[i]));
-    for (int i = 0; i < (1 << vb); ++i) vmax = fmaxf(vmax, fabsf(cbl[16 + i]));
-    const float sk = f16_split_scale(kmax);
-    sv = f16_split_scale(vmax);
+    const float sk = wide_pair_tables<kWideThreads, S::KTAB, S::VTAB, S::KHI>(lds, p, kesh, vesh, tid, sv);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) qmul[rt] = 1.4426950408889634f / (sk * qmul[rt]);
-    for (int e = tid; e < ((1 << (2 * kb + kesh)) >> 3); e += kWideThreads) {
-      const int key = e >> (kesh - 3);
-      uint32_t h0, l0, h1, l1;
-      split_f16(cbl[key & ((1 << kb) - 1)] * sk, h0, l0);
-      split_f16(cbl[key >> kb] * sk, h1, l1);
-      *reinterpret_cast<uint2*>(lds + S::KTAB + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
-    }
-    for (int e = tid; e < ((1 << (2 * vb + vesh)) >> 3); e += kWideThreads) {
-      const int key = e >> (vesh - 3);
-      uint32_t h0, l0, h1, l1;
-      split_f16(cbl[16 + (key & ((1 << vb) - 1))] * sv, h0, l0);
-      split_f16(cbl[16 + (key >> vb)] * sv, h1, l1);
-      *reinterpret_cast<uint2*>(lds + S::VTAB + e * 8) = make_uint2(h0 | (h1 << 16), l0 | (l1 << 16));
-    }
-    __syncthreads();
   }
   const uint32_t ktab = S::KTAB + (lane & ((1 << (kesh - 3)) - 1)) * 8;
   const uint32_t vtab = S::VTAB + (lane & ((1 << (vesh - 3)) - 1)) * 8;
