@@ -103,14 +103,17 @@ __device__ __forceinline__ void split_f16(float x, uint32_t& hi, uint32_t& lo) {
 
 // 2^(13 - e) for max |x| = f * 2^e, f in [0.5, 1): scales the largest
 // magnitude into [2^12, 2^13), far from f16 overflow and with the lo parts
-// of a hi/lo split still normal numbers.  At most 2^100: the scale of a row of
-// 1e-36, and its product with a codebook's, would overflow.
+// of a hi/lo split still normal numbers.
 __device__ __forceinline__ float f16_split_scale(float maxabs) {
   if (!(maxabs > 0.f) || !(maxabs < INFINITY)) return 1.f;
   int e;
   frexpf(maxabs, &e);
-  return ldexpf(1.f, min(13 - e, 100));
+  return ldexpf(1.f, 13 - e);
 }
+
+// The same of a query row, at most 2^99: the scale of a row of 1e-36, and its
+// product with a codebook's, would overflow.
+__device__ __forceinline__ float f16_query_scale(float maxabs) { return f16_split_scale(fmaxf(maxabs, 0x1p-87f)); }
 
 template <int D, int KB, int VB, int NQ>
 struct MfmaShape {
@@ -538,7 +541,7 @@ __global__ __launch_bounds__((MfmaShape<D, KB, VB, NQ>::NT), 1) void attn_mfma_k
   float qmax = 0.f;
 #pragma unroll
   for (int r = 0; r < NQ; ++r) qmax = fmaxf(qmax, s_qs[r]);
-  const float sq = f16_split_scale(qmax);
+  const float sq = f16_query_scale(qmax);
   // With 4-row groups the hi and lo pieces share one operand: A rows 0..3
   // hold the rows' hi parts, rows 4..7 their lo parts (rows 8..15 zero), so
   // one MFMA per k step gives both products and a lane exchange adds them

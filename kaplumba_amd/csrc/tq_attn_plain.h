@@ -231,7 +231,7 @@ __global__ __launch_bounds__(D >= 256 ? 256 : 512, 1) void attn_plain_kernel(Att
   float qmax = 0.f;
 #pragma unroll
   for (int r = 0; r < NQ; ++r) qmax = fmaxf(qmax, s_qs[r]);
-  const float sq = f16_split_scale(qmax);
+  const float sq = f16_query_scale(qmax);
   u32x4_t qh[KS], ql[KS];
   {
     const float qsl = n < NQ ? sq : 0.f;  // rows n >= NQ: zeros, no branches

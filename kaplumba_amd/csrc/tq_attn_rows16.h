@@ -393,7 +393,7 @@ __global__ __launch_bounds__(512, 1) void attn_rows16_kernel(AttnParams p) {
   float qm = 0.f;
 #pragma unroll
   for (int r = 0; r < NQ; ++r) qm = fmaxf(qm, reinterpret_cast<const float*>(lds + S::QMAX_OFF)[r]);
-  const float sq = f16_split_scale(qm);
+  const float sq = f16_query_scale(qm);
   for (int idx = tid; idx < NQ * D; idx += NT) {
     const int r = idx / D;
     const int c = idx % D;

@@ -414,8 +414,8 @@ __global__ __launch_bounds__(512, 1) void attn_small_kernel(AttnParams p) {
   // query pieces in B-operand order: staging [p][r][h][i] holds
   // q_p,r[h D/2 + 8 i + e], e = 0..7, as f16 (one hi/lo scale for all rows)
   const float* qmaxs = reinterpret_cast<const float*>(lds + S::QMAX_OFF);
-  const float sq = f16_split_scale(fmaxf(fmaxf(qmaxs[0], qmaxs[1]), fmaxf(qmaxs[2], qmaxs[3])));
-  const float sqp = PROD ? f16_split_scale(fmaxf(fmaxf(qmaxs[4], qmaxs[5]), fmaxf(qmaxs[6], qmaxs[7]))) : 1.f;
+  const float sq = f16_query_scale(fmaxf(fmaxf(qmaxs[0], qmaxs[1]), fmaxf(qmaxs[2], qmaxs[3])));
+  const float sqp = PROD ? f16_query_scale(fmaxf(fmaxf(qmaxs[4], qmaxs[5]), fmaxf(qmaxs[6], qmaxs[7]))) : 1.f;
   for (int idx = tid; idx < S::NQS * NQ * D; idx += NT) {
     const int set = idx / (NQ * D);
     const int r = (idx / D) % NQ;

@@ -415,7 +415,7 @@ __global__ __launch_bounds__((StageShape<D, KB, VB>::NT), 1) void attn_stage_ker
     float m = 0.f;
 #pragma unroll
     for (int e = 0; e < QE; ++e) m = fmaxf(m, fabsf(y[e]));
-    const float sq_row = f16_split_scale(wave_max(m));
+    const float sq_row = f16_query_scale(wave_max(m));
     if (lane == 0) reinterpret_cast<float*>(lds + S::QSC_OFF)[wave] = sq_row;
     STAGE_STAMP(4);
     uint32_t* st = reinterpret_cast<uint32_t*>(lds + S::QST_OFF);

@@ -724,7 +724,7 @@ __global__ __launch_bounds__(kTileQpThreads) void gen_tile_qprep_kernel(GenParam
     const float2 hv = halves(mx);
     mx = fmaxf(hv.x, hv.y);  // the row's largest magnitude
   }
-  const float sq = f16_split_scale(mx);
+  const float sq = f16_query_scale(mx);
   if (!ok) return;
   u32x4_t* dst = reinterpret_cast<u32x4_t*>(p.qhl) + static_cast<int64_t>(row) * 32 + 2 * g8;
 #pragma unroll

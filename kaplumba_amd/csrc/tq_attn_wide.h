@@ -265,7 +265,7 @@ __device__ __forceinline__ float wide_split_row(const float* src, int DkP, bool 
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[s][e]));
   }
-  const float sq = f16_split_scale(wide_row_max(mx));
+  const float sq = f16_query_scale(wide_row_max(mx));
 #pragma unroll
   for (int s = 0; s < KS; ++s)
 #pragma unroll

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kWideQpThreads) void wide_qprep_kernel(GenParams p,
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[u][e]));
     }
     mx = row16_max(mx);
-    const float sq = f16_split_scale(mx);
+    const float sq = f16_query_scale(mx);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int w = j + 16 * u;

@@ -89,7 +89,7 @@ def test_unlike_value_norms(device, Hq, Hkv, L, T, d, rot, kind):
     assert err.max().item() <= 2.0 ** (-8 if kind == "tiny" else -11) + 2e-6, err.max().item()
 
 
-@pytest.mark.parametrize("Hq,Hkv,L,T", [(8, 2, 3, 2111), (64, 16, 160, 1111)])  # narrow, or tuned; wide or tile
+@pytest.mark.parametrize("Hq,Hkv,L,T", [(8, 2, 1, 2111), (8, 2, 3, 2111), (64, 16, 160, 1111)])  # narrow or tuned; wide or tile
 @pytest.mark.parametrize("d,rot", [(64, "hadamard"), (96, "dense"), (128, "hadamard"), (256, "hadamard")])
 @pytest.mark.parametrize("masked", [False, True])
 def test_tiny_queries(device, Hq, Hkv, L, T, d, rot, masked):
@@ -100,8 +100,9 @@ def test_tiny_queries(device, Hq, Hkv, L, T, d, rot, masked):
     k_norms, k_words, k_rows = random_side(g, kc, Hkv, T, norms, device)
     v_norms, v_words, v_rows = random_side(g, vc, Hkv, T, norms, device)
     q = torch.randn(1, Hq, L, d, generator=g, device=device)
-    q[0, 0] *= 1e-36
-    q[0, 1] *= 1e-30
+    q[0, : Hq // Hkv] *= 1e-36  # a whole kv head's rows: some kernels scale them together
+    q[0, Hq // Hkv] *= 1e-36
+    q[0, Hq // Hkv + 1] *= 1e-30
     q = q.to(torch.bfloat16)
     keep = torch.arange(T, device=device)[None] <= torch.arange(T - L, T, device=device)[:, None]
     want = attention64(q, 1 / math.sqrt(d), kc, vc, k_rows, v_rows, keep)
